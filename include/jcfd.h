@@ -146,8 +146,10 @@ int jcfd_fvm_plan_set_cg_persistent(jcfd_fvm_plan* plan, int32_t enabled);
 /* Tile shapes and FFT radix schedule of the three step kernels.  No
  * counterpart in the reference (XLA picks its own kernels); set by the
  * project's autotuner (jax_cfd_amd.autotune), which times the menu on the
- * device.  Tile shapes never change results; radix 4 instead of 8 changes
- * the FFT rounding (results stay within fp32 round-off of each other). */
+ * device.  Until they are set, every launch picks them from its own size
+ * (get_tiles reports the whole batch's).  Tile shapes never change results;
+ * radix 4 instead of 8 changes the FFT rounding (results stay within fp32
+ * round-off of each other). */
 typedef struct {
   int32_t rows_forward; /* rows per workgroup of the stencil kernel: 1, 2, 4, 8; 16, 32
                            march over the rows with a ring of staged rows (n 256, 512) */

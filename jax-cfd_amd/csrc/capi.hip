@@ -301,6 +301,7 @@ struct jcfd_fvm_plan {
   CgBuffers cg{};
   float* rhs = nullptr;
   int* status_host = nullptr;  // pinned, 4 ints
+  bool tiles_set = false;  // set_tiles pinned the shapes; otherwise each launch's size picks them
   bool cg_persistent = false;  // one cooperative launch per CG solve (opt-in: slower, see the header)
   int cg_maxiter = 0;
   int cg_last_iterations = 0;
@@ -341,6 +342,7 @@ struct jcfd_ns2d_plan {
   float2* pbuf = nullptr;
   float2* ws = nullptr;  // the state in the step kernels' internal layout
   int64_t bytes = 0;
+  bool tiles_set = false;  // as in jcfd_fvm_plan
   GraphCache graphs;
 };
 
@@ -536,7 +538,9 @@ int fvm_rk_step(const jcfd_fvm_plan* p, const FvmBuffers& b, hipStream_t s) {
 // One step: the fast-diagonal step kernels (or the Runge-Kutta stages), then
 // (implicit diffusion plans) the diffusion solve in place on the output.
 int fvm_full_step(jcfd_fvm_plan* p, const FvmBuffers& b, hipStream_t s) {
-  int rc = p->rk_terms != nullptr ? fvm_rk_step(p, b, s) : fvm_launch_step(p->params, b, s);
+  FvmParams q = p->params;
+  if (!p->tiles_set) (void)fvm_default_tiles(&q, nb(b));  // a slot list may be shorter than the batch
+  int rc = p->rk_terms != nullptr ? fvm_rk_step(p, b, s) : fvm_launch_step(q, b, s);
   if (rc == JCFD_OK) rc = fvm_diffuse_output(p, b, s);
   return rc;
 }
@@ -652,9 +656,9 @@ int jcfd_fvm_plan_create(const jcfd_fvm_config* config, jcfd_fvm_plan** plan) {
   q.has_forcing = c.has_forcing ? 1 : 0;
   q.lin = static_cast<float>(c.linear_coefficient);
   q.convect = c.convect;
-  (void)fvm_default_tiles(&q);
 
   p->batch = c.batch > 1 ? c.batch : 1;
+  (void)fvm_default_tiles(&q, p->batch);
   p->graphs.enabled = p->batch > 1;
   const size_t nn = static_cast<size_t>(n) * n * p->batch;
   int rc = JCFD_OK;
@@ -794,6 +798,7 @@ int jcfd_fvm_plan_set_tiles(jcfd_fvm_plan* p, const jcfd_fvm_tiles* tiles) {
   p->params.w_cols = t[1];
   p->params.rb_proj = t[2];
   p->params.radix = tiles->radix;
+  p->tiles_set = true;
   p->graphs.release();  // captured launches carry the old shapes
   return JCFD_OK;
 }
@@ -1934,6 +1939,7 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
   for (int k = 0; k < p->n_stages; ++k) {
     stages[k] = p->stages[k];
     stages[k].slots = slots;
+    if (!p->tiles_set) (void)ns_default_tiles(&stages[k], p->n, count);
   }
   const int ns = p->n_stages;
   NsBuffers b{};
@@ -2076,7 +2082,7 @@ int jcfd_ns2d_plan_create(const jcfd_ns2d_config* config, jcfd_ns2d_plan** plan)
     q.mu = static_cast<float>(0.5 * c.dt * (alpha[k + 1] - alpha[k]));
     q.read_h = k > 0 ? 1 : 0;
     q.slots = nullptr;
-    (void)ns_default_tiles(&q, n);
+    (void)ns_default_tiles(&q, n, c.batch);
   }
   *plan = p;
   return JCFD_OK;
@@ -2105,6 +2111,7 @@ int jcfd_ns2d_plan_set_tiles(jcfd_ns2d_plan* p, const jcfd_ns2d_tiles* tiles) {
     q.rb_rows = tiles->rows;
     q.radix = tiles->radix;
   }
+  p->tiles_set = true;
   p->graphs.release();  // captured launches carry the old shapes
   return JCFD_OK;
 }

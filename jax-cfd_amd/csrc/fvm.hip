@@ -831,14 +831,45 @@ __global__ void fvm_divergence_kernel(FvmParams p, const float* __restrict__ u,
   out[e] = ddx + ddy;
 }
 
-// Per-size tile shapes: RB rows per row block, W columns per column tile.
-template <int N> struct Tiles;
-template <> struct Tiles<32> { static constexpr int RB = 4, W = 8; };
-template <> struct Tiles<64> { static constexpr int RB = 4, W = 8; };
-template <> struct Tiles<128> { static constexpr int RB = 4, W = 8; };
-template <> struct Tiles<256> { static constexpr int RB = 4, W = 8; };
-template <> struct Tiles<512> { static constexpr int RB = 2, W = 8; };
-template <> struct Tiles<1024> { static constexpr int RB = 1, W = 4; };
+// Rows per workgroup of row kernels that fill the chip.
+template <int N> struct Tiles { static constexpr int RB = 4; };
+template <> struct Tiles<512> { static constexpr int RB = 2; };
+template <> struct Tiles<1024> { static constexpr int RB = 1; };
+
+// Tile shapes of a launch of `count` instances of size N, for plans whose
+// shapes were not set.  A launch that leaves CUs idle wants many small tiles,
+// one that fills the chip wants fewer, larger ones (less halo recomputation,
+// wider column accesses); the lines lie where the two measured the same, with
+// R = rows and C = packed spectrum columns over all instances.  us per launch,
+// small shape / fixed default (RB 4, 4, 4, 2, 1 for 64..1024; W 8, 8, 8, 8, 4)
+// / largest-useful shape:
+//   rows-forward   1 x 256^2  5.5 / 9.6 (RB 1 / 4);   128 x 256^2 116 / 90 / 68 (RB 1 / 4 / 16)
+//                  1 x 512^2  9.5 / 11.0 (RB 1 / 2);   64 x 512^2 277 / 228 / 155 (RB 1 / 2 / 16)
+//                  8 x 256^2  11.6 / 10.9 / 11.9 (RB 1 / 2 / 4)
+//   Poisson cols   1 x 256^2  4.2 / 9.3 (W 1 / 8);     128 x 256^2 45.8 / 23.2 / 22.6 (W 1 / 8 / 4)
+//                  1 x 1024^2 11.2 / 18.9 (W 1 / 4);   16 x 1024^2 75 / 59 (W 1 / 4)
+//   rows-project   1 x 256^2  3.0 / 3.8 (RB 1 / 4);    128 x 256^2 36 / 26 (RB 1 / 4)
+template <int N>
+void auto_tiles(FvmParams* p, int count) {
+  const long long R = static_cast<long long>(N) * count, C = R / 2;
+  if (N == 1024) p->rb_fwd = 1;
+  else if ((N == 512 && R >= 8192) || (N == 256 && R >= 12288)) p->rb_fwd = 16;  // marching form
+  else if (N <= 128 && R >= 16384) p->rb_fwd = 8;
+  else p->rb_fwd = R < 1024 ? 1 : (R < 4096 ? 2 : 4);
+  int w = 1;
+  const int cap = N <= 64 ? 8 : (N == 128 ? 16 : 4);
+  while (2 * w <= cap && C / (2 * w) >= (N <= 64 ? 256 : (w < 4 ? 512 : 1024))) w *= 2;
+  p->w_cols = w;
+  p->rb_proj = R < 1024 ? 1 : ((N >= 512 || R < 2048) ? 2 : 4);
+}
+
+// Rows per workgroup of the row kernels that have no tunable shape (explicit
+// terms, projection, Runge-Kutta combination, filters): one row while that
+// leaves CUs idle, else Tiles<N>::RB.
+template <int N>
+bool one_row(int count) {
+  return Tiles<N>::RB > 1 && static_cast<long long>(N) * count < 1024;
+}
 
 // ---- tunable step kernels ---------------------------------------------------
 // The three step kernels are built for a menu of tile shapes and both radix
@@ -957,29 +988,68 @@ bool tile_on_menu(int which, int tile) {
   return which == 0 ? row(tile) : (which == 1 ? col(tile) : proj(tile));
 }
 
+// A row kernel of MODE with Tiles<N>::RB rows per workgroup, or one row for a
+// launch of few rows; radix-8 schedule.
+template <int N, int MODE>
+void launch_rows_forward(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
+  constexpr int RB = Tiles<N>::RB;
+  if (one_row<N>(nb(b)))
+    hipLaunchKernelGGL((fvm_rows_forward<N, 1, MODE>), dim3(N, nb(b)), dim3(kThreads), 0, s, p, b);
+  else
+    hipLaunchKernelGGL((fvm_rows_forward<N, RB, MODE>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+}
+
+template <int N, int MODE>
+void launch_rows_project(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
+  constexpr int RB = Tiles<N>::RB;
+  if (one_row<N>(nb(b)))
+    hipLaunchKernelGGL((fvm_rows_project<N, 1, MODE>), dim3(N, nb(b)), dim3(kThreads), 0, s, p, b);
+  else
+    hipLaunchKernelGGL((fvm_rows_project<N, RB, MODE>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+}
+
+// The Poisson column kernel at the tile width the launch's size asks for,
+// radix-8 schedule.
+template <int N, int W>
+bool launch_cols_w(int w, const FvmBuffers& b, float scale, hipStream_t s) {
+  if constexpr (W <= 16 && cols_ok<N, W>()) {
+    if (w == W) {
+      hipLaunchKernelGGL((fvm_poisson_cols<N, W>), dim3(N / 2 / W, nb(b)), dim3(kThreads), 0, s, b, scale);
+      return true;
+    }
+    return launch_cols_w<N, 2 * W>(w, b, scale, s);
+  }
+  return false;
+}
+template <int N>
+int launch_cols(const FvmBuffers& b, float scale, hipStream_t s) {
+  FvmParams t{};
+  auto_tiles<N>(&t, nb(b));
+  if (!launch_cols_w<N, 1>(t.w_cols, b, scale, s))
+    return fail(JCFD_ERR_UNSUPPORTED, "Poisson column tile not built for n = " + std::to_string(N));
+  return JCFD_OK;
+}
+
 template <int N>
 int launch_explicit(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-  constexpr int RB = Tiles<N>::RB;
-  hipLaunchKernelGGL((fvm_rows_forward<N, RB, 2>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+  launch_rows_forward<N, 2>(p, b, s);
   return check_hip(hipGetLastError(), "fvm explicit-terms launch");
 }
 
 template <int N>
 int launch_projection(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-  constexpr int RB = Tiles<N>::RB, W = Tiles<N>::W;
-  hipLaunchKernelGGL((fvm_rows_forward<N, RB, 1>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
-  hipLaunchKernelGGL((fvm_poisson_cols<N, W>), dim3(N / 2 / W, nb(b)), dim3(kThreads), 0, s, b, 1.0f);
-  hipLaunchKernelGGL((fvm_rows_project<N, RB, 0>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+  launch_rows_forward<N, 1>(p, b, s);
+  if (const int rc = launch_cols<N>(b, 1.0f, s)) return rc;
+  launch_rows_project<N, 0>(p, b, s);
   return check_hip(hipGetLastError(), "fvm projection launch");
 }
 
 template <int N>
 int launch_filter(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-  constexpr int RB = Tiles<N>::RB, W = Tiles<N>::W;
   const float scale = 1.0f / (static_cast<float>(N) * static_cast<float>(N));
-  hipLaunchKernelGGL((fvm_rows_forward<N, RB, 3>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
-  hipLaunchKernelGGL((fvm_poisson_cols<N, W>), dim3(N / 2 / W, nb(b)), dim3(kThreads), 0, s, b, scale);
-  hipLaunchKernelGGL((fvm_rows_project<N, RB, 1>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+  launch_rows_forward<N, 3>(p, b, s);
+  if (const int rc = launch_cols<N>(b, scale, s)) return rc;
+  launch_rows_project<N, 1>(p, b, s);
   return check_hip(hipGetLastError(), "spectral filter launch");
 }
 
@@ -987,7 +1057,6 @@ int launch_filter(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
 // rfft2(u)) with m = D / n^2 the implicit-diffusion multiplier.
 template <int N>
 int launch_diffuse(const FvmParams& p, const FvmBuffers& b, const float* mult, hipStream_t s) {
-  constexpr int RB = Tiles<N>::RB, W = Tiles<N>::W;
   for (int c = 0; c < 2; ++c) {
     FvmBuffers f = b;
     float* field = c == 0 ? b.u_out : b.v_out;
@@ -995,26 +1064,24 @@ int launch_diffuse(const FvmParams& p, const FvmBuffers& b, const float* mult, h
     f.u_out = field;
     f.lam = mult;
     f.lam_mode = 1;  // the plan's multiplier table, column by column
-    hipLaunchKernelGGL((fvm_rows_forward<N, RB, 3>), dim3(N / RB, nb(f)), dim3(kThreads), 0, s, p, f);
-    hipLaunchKernelGGL((fvm_poisson_cols<N, W>), dim3(N / 2 / W, nb(f)), dim3(kThreads), 0, s, f, 1.0f);
-    hipLaunchKernelGGL((fvm_rows_project<N, RB, 3>), dim3(N / RB, nb(f)), dim3(kThreads), 0, s, p, f);
+    launch_rows_forward<N, 3>(p, f, s);
+    if (const int rc = launch_cols<N>(f, 1.0f, s)) return rc;
+    launch_rows_project<N, 3>(p, f, s);
   }
   return check_hip(hipGetLastError(), "implicit diffusion launch");
 }
 
 template <int N>
 int launch_rk_explicit(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-  constexpr int RB = Tiles<N>::RB;
-  hipLaunchKernelGGL((fvm_rows_forward<N, RB, 2>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+  launch_rows_forward<N, 2>(p, b, s);
   return check_hip(hipGetLastError(), "rk explicit-terms launch");
 }
 
 template <int N>
 int launch_rk_project(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-  constexpr int RB = Tiles<N>::RB, W = Tiles<N>::W;
-  hipLaunchKernelGGL((fvm_rows_forward<N, RB, 5>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
-  hipLaunchKernelGGL((fvm_poisson_cols<N, W>), dim3(N / 2 / W, nb(b)), dim3(kThreads), 0, s, b, 1.0f);
-  hipLaunchKernelGGL((fvm_rows_project<N, RB, 0>), dim3(N / RB, nb(b)), dim3(kThreads), 0, s, p, b);
+  launch_rows_forward<N, 5>(p, b, s);
+  if (const int rc = launch_cols<N>(b, 1.0f, s)) return rc;
+  launch_rows_project<N, 0>(p, b, s);
   return check_hip(hipGetLastError(), "rk projection launch");
 }
 
@@ -1039,15 +1106,13 @@ template <int N> struct ExplicitOp {
 };
 template <int N> struct ForwardRhsOp {
   static int run(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-    constexpr int RB = Tiles<N>::RB;
-    hipLaunchKernelGGL((fvm_rows_forward<N, RB, 4>), dim3(N / RB), dim3(kThreads), 0, s, p, b);
+    launch_rows_forward<N, 4>(p, b, s);
     return check_hip(hipGetLastError(), "fvm forward (CG rhs)");
   }
 };
 template <int N> struct ProjectQOp {
   static int run(const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
-    constexpr int RB = Tiles<N>::RB;
-    hipLaunchKernelGGL((fvm_rows_project<N, RB, 2>), dim3(N / RB), dim3(kThreads), 0, s, p, b);
+    launch_rows_project<N, 2>(p, b, s);
     return check_hip(hipGetLastError(), "fvm project (CG q)");
   }
 };
@@ -1190,10 +1255,8 @@ bool fvm_size_supported(int n) {
 bool fvm_group_size_supported(int n) { return fvm_size_supported(n) && n <= kFvmGroupMaxN; }
 
 template <int N> struct DefaultTilesOp {
-  static int run(FvmParams* p) {
-    p->rb_fwd = Tiles<N>::RB;
-    p->w_cols = Tiles<N>::W;
-    p->rb_proj = Tiles<N>::RB;
+  static int run(FvmParams* p, int count) {
+    auto_tiles<N>(p, count);
     p->radix = 8;
     return JCFD_OK;
   }
@@ -1205,7 +1268,7 @@ template <int N> struct TileMenuOp {
   }
 };
 
-int fvm_default_tiles(FvmParams* p) { return dispatch_n<DefaultTilesOp>(p->n, p); }
+int fvm_default_tiles(FvmParams* p, int count) { return dispatch_n<DefaultTilesOp>(p->n, p, count); }
 
 bool fvm_tile_supported(int n, int which, int tile) {
   bool ok = false;

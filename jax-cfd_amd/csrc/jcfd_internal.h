@@ -200,8 +200,8 @@ int fvm_launch_semilagrangian(int n, const float* c, const float* u, const float
 int fvm_launch_filter(const FvmParams& p, const float* x, const float* multiplier, float* out,
                       float2* spec, const float2* tw, hipStream_t s);
 bool fvm_size_supported(int n);
-// Default tile shapes and radix of size p->n into p.
-int fvm_default_tiles(FvmParams* p);
+// Tile shapes and radix of a launch of `count` instances of size p->n into p.
+int fvm_default_tiles(FvmParams* p, int count);
 // Whether kernel class `which` (0 rows-forward, 1 Poisson columns,
 // 2 rows-project) is built with tile `tile` for size n.
 bool fvm_tile_supported(int n, int which, int tile);
@@ -325,8 +325,8 @@ bool ns_group_size_supported(int n);
 int ns_group_tiles(int n, int list);
 int ns_group_launch(int cls, int max_n, const NsGroupQueue& q, int stage, int grid, hipStream_t s);
 bool ns_size_supported(int n);
-// Default tile shapes and radix for size n into q.
-int ns_default_tiles(NsParams* q, int n);
+// Tile shapes and radix of a launch of `count` instances of size n into q.
+int ns_default_tiles(NsParams* q, int n, int count);
 // Whether step kernel class `which` (0 cols-inverse, 1 rows, 2/3 cols-forward)
 // is built with tile `tile` (columns per tile; rows per workgroup for 1).
 bool ns_tile_supported(int n, int which, int tile);

@@ -967,25 +967,28 @@ int ns_one_impl(int which, const NsParams* stages, int nstages, const NsBuffers&
   }
 }
 
-template <int N> struct NsDefaultOp {
-  static void run(NsParams* q) {
-    q->w_cols = NsTiles<N>::W;
-    q->rb_rows = NsTiles<N>::RB;
-    q->radix = 8;
-  }
-};
 }  // namespace
 
-int ns_default_tiles(NsParams* q, int n) {
-  switch (n) {
-    case 32: NsDefaultOp<32>::run(q); return JCFD_OK;
-    case 64: NsDefaultOp<64>::run(q); return JCFD_OK;
-    case 128: NsDefaultOp<128>::run(q); return JCFD_OK;
-    case 256: NsDefaultOp<256>::run(q); return JCFD_OK;
-    case 512: NsDefaultOp<512>::run(q); return JCFD_OK;
-    case 1024: NsDefaultOp<1024>::run(q); return JCFD_OK;
-    default: return fail(JCFD_ERR_UNSUPPORTED, "spectral grid size not built");
-  }
+// Tile shapes of plans whose shapes were not set.  The column kernels want
+// one column per workgroup until the launch fills the chip many times over
+// (a column of 1024 or 512 words is work enough for 256 threads; shorter
+// columns share a workgroup sooner), and never the wide tiles whose
+// registers and LDS leave few workgroups per CU.  us per step spent in the
+// column kernels, W = 1 / 2 / 4 / 8: 1 x 256^2 32 / 42 / 83 / 173, 64 x 256^2
+// 215 / 183 / 220 / 327, 1 x 512^2 46 / 84 / 176 / 336, 64 x 512^2
+// 779 / 690 / 965 / 1537, 16 x 64^2 29 / 29 / 30 / 43, 256 x 64^2
+// 121 / 80 / 67 / 66; in the row kernel, RB = 1 / 2 / 4: 1 x 256^2
+// 21 / 22 / 26, 64 x 256^2 218 / 165 / 154, 64 x 512^2 645 / 530 / 532.
+int ns_default_tiles(NsParams* q, int n, int count) {
+  if (!ns_size_supported(n)) return fail(JCFD_ERR_UNSUPPORTED, "spectral grid size not built");
+  const long long rows = static_cast<long long>(n) * count, cols = rows / 2;
+  q->w_cols = n >= 512 ? (cols < 8192 ? 1 : 2)
+              : n == 256 ? (cols < 2048 ? 1 : 2)
+                         : (cols < (n == 32 ? 1024 : 512) ? 1 : cols < (n == 128 ? 4096 : 1024) ? (n == 32 ? 1 : 2)
+                                                                : cols < 8192 || n == 128 ? 4 : 8);
+  q->rb_rows = n >= 512 ? 2 : (rows < 512 ? 1 : (rows < 2048 ? 2 : 4));
+  q->radix = 8;
+  return JCFD_OK;
 }
 
 bool ns_tile_supported(int n, int which, int tile) {

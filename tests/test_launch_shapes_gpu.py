@@ -1,0 +1,83 @@
+"""Launch shapes picked from a launch's size, on both sides of every line of
+the rules: each must step bit-identically to the same plan with one-row,
+one-column tiles set by hand (tile shapes never change results), for whole
+batches and for short slot lists of a large batch."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev():
+  return torch.device('cuda', 0)
+
+
+def _fvm(n, batch, **kw):
+  import dataclasses
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.base import _fvm
+  spec = dataclasses.replace(serving.FvmFamily(n, _dev()).spec, **kw)
+  gen = torch.Generator(device=_dev()).manual_seed(n + batch)
+  u = torch.randn((batch, n, n), device=_dev(), generator=gen)
+  v = torch.randn((batch, n, n), device=_dev(), generator=gen)
+  return _fvm.FvmPlan(spec, _dev(), batch=batch), u, v
+
+
+# rows or columns over all instances at the rules' lines, and one below
+@pytest.mark.parametrize("n,batch", [(32, 7), (32, 32), (32, 512), (64, 7), (64, 8), (64, 15), (64, 64),
+                                     (64, 256), (128, 7), (128, 8), (128, 31), (128, 128),
+                                     (256, 2), (256, 3), (256, 4), (256, 16), (256, 47), (256, 48),
+                                     (512, 2), (512, 8), (512, 15), (512, 16), (1024, 1), (1024, 3)])
+def test_fvm_rule_steps_as_one_row_tiles(n, batch):
+  plan, u, v = _fvm(n, batch)
+  if batch == 1:
+    u, v = u[0], v[0]
+  got = plan.step(u, v, 2)
+  plan.set_tiles(1, 1, 1, 8)
+  want = plan.step(u, v, 2)
+  print(f"n={n} batch={batch}", flush=True)
+  assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n,batch", [(32, 64), (128, 40), (256, 48), (512, 16)])
+def test_fvm_short_slot_lists(n, batch):
+  plan, u, v = _fvm(n, batch)
+  want = plan.step(u, v, 2)
+  slots = torch.tensor([batch - 1, 0, 2], dtype=torch.int32, device=_dev())
+  u1, v1 = u.clone(), v.clone()
+  plan.step_slots(u1, v1, slots, 2)
+  idx = slots.long()
+  assert torch.equal(u1[idx], want[0][idx]) and torch.equal(v1[idx], want[1][idx])
+  assert torch.equal(u1[1], u[1])
+
+
+# row kernels without a tunable shape: one row per workgroup for few rows
+@pytest.mark.parametrize("kw", [dict(diffusion=1), dict(rk_stages=2, rk_a=(1.0,), rk_b=(0.5, 0.5))])
+@pytest.mark.parametrize("n,batch", [(32, 33), (128, 9), (256, 4), (512, 2)])
+def test_fvm_untuned_kernels_match_lone_instances(n, batch, kw):
+  plan, u, v = _fvm(n, batch, **kw)
+  one, _, _ = _fvm(n, 1, **kw)
+  got = plan.step(u, v, 2)
+  for k in (0, batch - 1):
+    want = one.step(u[k].contiguous(), v[k].contiguous(), 2)
+    assert torch.equal(got[0][k], want[0]) and torch.equal(got[1][k], want[1])
+
+
+@pytest.mark.parametrize("n,batch", [(32, 63), (32, 64), (64, 16), (64, 32), (64, 256), (128, 7),
+                                     (128, 8), (128, 64), (256, 15), (256, 16), (512, 1),
+                                     (512, 31), (512, 32), (1024, 2), (1024, 16)])
+def test_spectral_rule_steps_as_one_column_tiles(n, batch):
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  plan = _ns2d.Ns2dPlan(serving.SpectralFamily(n, _dev()).spec, batch, _dev())
+  gen = torch.Generator(device=_dev()).manual_seed(n + batch)
+  w = plan.rfft2(torch.randn((batch, n, n), device=_dev(), generator=gen))
+  got = plan.step(w, 2)
+  plan.set_tiles(1, 1, 8)
+  assert torch.equal(got, plan.step(w, 2))
+  if batch > 3:
+    slots = torch.tensor([batch - 1, 1], dtype=torch.int32, device=_dev())
+    other = _ns2d.Ns2dPlan(plan.spec, batch, _dev())
+    w1 = w.clone()
+    other.step_slots(w1, slots, 2)
+    assert torch.equal(w1[slots.long()], got[slots.long()])
