@@ -599,13 +599,22 @@ def _served(dev, requests, kernel_reps, group=(), runs=3, warmup_passes=1):
 def _ns2d_kernel_key(kname, n, batch, tiles):
   """_kernel_key of a spectral plan's step kernel for its tiles."""
   w, rb, radix = tiles["cols"], tiles["rows"], tiles["radix"]
-  cols_grid = batch * (n // 2) // w * 256
-  name = {"ns_cols_inverse": f"ns_cols_inverse<{n}, {w}, 4, {radix}>",
-          "ns_rows": f"ns_rows<{n}, {rb}, {radix}>",
-          "ns_cols_update_inverse": f"ns_cols_forward<{n}, {w}, 2, {radix}>",
-          "ns_cols_update": f"ns_cols_forward<{n}, {w}, 1, {radix}>"}[kname]
-  grid = batch * n // rb * 256 if kname == "ns_rows" else cols_grid
-  return f"{name} grid={grid}"
+  if kname == "ns_rows":
+    rs = 1024 // n  # rows per wavefront
+    name = f"ns_rows_seq<{n}, {radix}>" if rb == 4 * rs else f"ns_rows<{n}, {min(rb, rs)}, {radix}>"
+    threads = 256 if rb == 4 * rs else 256 * max(1, rb // rs)
+    return f"{name} grid={batch * (n // rb) * threads}"
+  if w <= {32: 16, 64: 8, 128: 4, 256: 2}.get(n, 1):  # the staged kernels
+    name = {"ns_cols_inverse": f"ns_cols_inverse_staged<{n}, {w}, {radix}>",
+            "ns_cols_update_inverse": f"ns_cols_forward_staged<{n}, {w}, 2, {radix}>",
+            "ns_cols_update": f"ns_cols_forward_staged<{n}, {w}, 1, {radix}>"}[kname]
+    threads = 256
+  else:
+    name = {"ns_cols_inverse": f"ns_cols_inverse<{n}, 4, {radix}>",
+            "ns_cols_update_inverse": f"ns_cols_forward<{n}, 2, {radix}>",
+            "ns_cols_update": f"ns_cols_forward<{n}, 1, {radix}>"}[kname]
+    threads = 64 * -(-w // max(1, 512 // n))
+  return f"{name} grid={batch * (n // 2 // w) * threads}"
 
 
 def _fvm_plan_kernel_key(kname, n, batch, tiles):

@@ -408,7 +408,7 @@ int jcfd_ns2d_plan_set_graphs(jcfd_ns2d_plan* plan, int32_t enabled);
  * change results; radix 4 changes the FFT rounding. */
 typedef struct {
   int32_t cols;  /* packed spectrum columns per workgroup of the column kernels: 1..16 */
-  int32_t rows;  /* rows per workgroup of the row (nonlinear product) kernel: 1, 2, 4 */
+  int32_t rows;  /* rows per workgroup of the row (nonlinear product) kernel: 1, 2, 4, 8, 16 */
   int32_t radix; /* largest FFT radix: 8 or 4 */
 } jcfd_ns2d_tiles;
 int jcfd_ns2d_plan_get_tiles(const jcfd_ns2d_plan* plan, jcfd_ns2d_tiles* tiles);

@@ -1935,26 +1935,44 @@ namespace {
 // enabled) and moved back.
 int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slots, int count,
            int64_t nsteps, hipStream_t s) {
-  NsParams stages[JCFD_MAX_RK_STAGES];
-  for (int k = 0; k < p->n_stages; ++k) {
-    stages[k] = p->stages[k];
-    stages[k].slots = slots;
-    if (!p->tiles_set) (void)ns_default_tiles(&stages[k], p->n, count);
-  }
+  const size_t n = static_cast<size_t>(p->n);
+  const size_t ext = n * (n / 2 + 1), half = n * (n / 2);
   const int ns = p->n_stages;
-  NsBuffers b{};
-  b.u_in = p->ws;
-  b.u_out = p->ws;
-  b.h = p->h;
-  b.g = p->g;
-  b.pbuf = p->pbuf;
-  int rc;
-  if ((rc = ns_launch_state_convert(p->n, true, w_in, p->ws, slots, count, s))) return rc;
-  if ((rc = ns_launch_step(p->n, stages, ns, b, count, s))) return rc;
-  if ((rc = run_steps(p->graphs, b.u_out, nullptr, slots, count, nsteps - 1, s,
-                      [&](hipStream_t gs) { return ns_launch_step(p->n, stages, ns, b, count, gs); })))
-    return rc;
-  return ns_launch_state_convert(p->n, false, p->ws, w_out, slots, count, s);
+  // A step streams 28 bytes per cell through its kernels.  Batches whose
+  // share exceeds the 256 MB last-level cache run in parts that fit, each
+  // part all its steps: the spectra one kernel writes are then still cached
+  // when the next reads them (512^2: 17.1 us per instance and step at 32
+  // instances, 18.5 at 16, 19.1 at 64).
+  constexpr size_t kPartCells = size_t(8) << 20;
+  const int most = static_cast<int>(std::max<size_t>(1, kPartCells / (n * n)));
+  const int parts = (count + most - 1) / most;
+  for (int k = 0; k < parts; ++k) {
+    const int first = static_cast<int>(static_cast<int64_t>(count) * k / parts);
+    const int m = static_cast<int>(static_cast<int64_t>(count) * (k + 1) / parts) - first;
+    // instances are reached through the slot list, or by offset
+    const int* sl = slots ? slots + first : nullptr;
+    const size_t o = slots ? 0 : static_cast<size_t>(first);
+    NsParams stages[JCFD_MAX_RK_STAGES];
+    for (int i = 0; i < ns; ++i) {
+      stages[i] = p->stages[i];
+      stages[i].slots = sl;
+      if (!p->tiles_set) (void)ns_default_tiles(&stages[i], p->n, m);
+    }
+    NsBuffers b{};
+    b.u_in = p->ws + o * ext;
+    b.u_out = p->ws + o * ext;
+    b.h = p->h + o * ext;
+    b.g = p->g + o * 4 * half;
+    b.pbuf = p->pbuf + o * half;
+    int rc;
+    if ((rc = ns_launch_state_convert(p->n, true, w_in + o * ext, p->ws + o * ext, sl, m, s))) return rc;
+    if ((rc = ns_launch_step(p->n, stages, ns, b, m, s))) return rc;
+    if ((rc = run_steps(p->graphs, b.u_out, nullptr, sl, m, nsteps - 1, s,
+                        [&](hipStream_t gs) { return ns_launch_step(p->n, stages, ns, b, m, gs); })))
+      return rc;
+    if ((rc = ns_launch_state_convert(p->n, false, p->ws + o * ext, w_out + o * ext, sl, m, s))) return rc;
+  }
+  return JCFD_OK;
 }
 }  // namespace
 
@@ -2064,6 +2082,8 @@ int jcfd_ns2d_plan_create(const jcfd_ns2d_config* config, jcfd_ns2d_plan** plan)
     NsParams& q = p->stages[k];
     q.kx = p->kx;
     q.ky = p->ky;
+    q.dnx = dnx;
+    q.rcp_dnx = 1.0f / dnx;
     q.tw = p->tw;
     q.force_idx = p->force_idx;
     q.force_val = p->force_val;

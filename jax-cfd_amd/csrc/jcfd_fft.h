@@ -247,6 +247,108 @@ __device__ __forceinline__ void lds_fft_waves(float2* buf, const float2* tw, int
   __syncthreads();
 }
 
+// ---- transforms held in registers ------------------------------------------
+// A transform of length N by L = N / E lanes of one wavefront, lane j holding
+// elements j + e L, e = 0 .. E-1.  Butterfly g = j + b L of a radix-R pass
+// then reads elements g + r N / R of its own lane, and the last pass writes
+// elements of its own lane too: data enters and leaves in registers, in
+// natural order, and LDS carries only the reorderings between passes (two
+// for N = 512, radix 8), where the staged transforms above write and read
+// LDS around every pass.  The exchange buffer belongs to the wavefront, so no
+// workgroup barrier is needed anywhere.  T transforms share a wavefront
+// (their elements interleaved in LDS); one spare word per 8 makes the
+// strided writes of the first pass free of bank conflicts, and every
+// address is one base per pass plus a constant.  Same passes, twiddles and
+// operation order as lds_fft: the results are bit-identical.
+constexpr int fft_radix(int rem, int maxr) { return (maxr >= 8 && rem % 8 == 0) ? 8 : (rem % 4 == 0 ? 4 : 2); }
+constexpr int fft_pad(int i) { return i + i / 8; }
+
+// Twiddles per lane of the passes before the one with NS = upto.
+constexpr int reg_tw_count(int n, int e, int maxr, int upto) {
+  int c = 0;
+  for (int ns = 1; ns < upto;) {
+    const int r = fft_radix(n / ns, maxr);
+    if (ns > 1) c += ((n / e) % ns == 0 ? 1 : e / r) * (r - 1);
+    ns *= r;
+  }
+  return c;
+}
+
+// A lane's twiddles of every pass, loaded once and kept in registers over any
+// number of transforms (inverse ones conjugate them on use).
+template <int N, int E, int MAXR>
+struct RegTwiddles {
+  static constexpr int L = N / E;
+  static constexpr int COUNT = reg_tw_count(N, E, MAXR, N);
+  float2 w[COUNT];
+  // entry k of the length-N table is tab[k * STRIDE]
+  template <int STRIDE, int NS = 1>
+  __device__ __forceinline__ void load(const float2* __restrict__ tab, int j) {
+    if constexpr (NS < N) {
+      constexpr int R = fft_radix(N / NS, MAXR), OFF = reg_tw_count(N, E, MAXR, NS);
+      constexpr int TWS = N / (NS * R), B = L % NS == 0 ? 1 : E / R;
+      static_assert(L % NS == 0 || NS * R == N, "only the last pass has more twiddle indices than lanes");
+      if constexpr (NS > 1) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+          const int k = L % NS == 0 ? j % NS : j + b * L;
+#pragma unroll
+          for (int r = 1; r < R; ++r) w[OFF + b * (R - 1) + r - 1] = tab[r * k * TWS * STRIDE];
+        }
+      }
+      load<STRIDE, NS * R>(tab, j);
+    }
+  }
+};
+
+// LDS words (float2) of T transforms' exchange buffer.
+template <int N, int T>
+constexpr int kRegFftWords = fft_pad(N) * T;
+
+// v: this lane's elements; x: the wavefront's buffer plus the transform's
+// index t (element i of transform t at x[fft_pad(i) * T]).
+template <int N, int E, int T, bool INV, int MAXR, int NS = 1>
+__device__ __forceinline__ void reg_fft(float2 (&v)[E], const RegTwiddles<N, E, MAXR>& tw, float2* x, int j) {
+  if constexpr (NS < N) {
+    constexpr int L = N / E, R = fft_radix(N / NS, MAXR), B = E / R;
+    constexpr int OFF = reg_tw_count(N, E, MAXR, NS);
+    static_assert(E % R == 0, "whole butterflies per lane");
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      float2 a[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) a[r] = v[b + r * B];
+      if constexpr (NS > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          float2 w = tw.w[OFF + (L % NS == 0 ? 0 : b) * (R - 1) + r - 1];
+          if (INV) w.y = -w.y;
+          a[r] = cmul(a[r], w);
+        }
+      }
+      dft_radix<R, INV>(a);
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[b + r * B] = a[r];
+    }
+    if constexpr (NS * R < N) {
+      // butterfly g = j + b L writes r at (g / NS) NS R + g % NS + r NS
+      static_assert(L % NS == 0 && (B == 1 || (L * R) % 8 == 0), "constant offsets between butterflies");
+      const int base = (j / NS) * NS * R + j % NS;
+      float2* wr = x + fft_pad(base) * T;
+      wave_lds_sync();  // earlier reads of the buffer come first
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int r = 0; r < R; ++r) wr[fft_pad(b * L * R + r * NS) * T] = v[b + r * B];
+      wave_lds_sync();
+      const float2* rd = x + fft_pad(j) * T;
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = rd[fft_pad(e * L) * T];
+      reg_fft<N, E, T, INV, MAXR, NS * R>(v, tw, x, j);
+    }
+  }
+}
+
 // A length-N twiddle table (entries k * STRIDE of the source table) staged
 // through registers: load() issues all of a thread's global loads, store()
 // writes them to LDS.  Splitting the two lets a kernel keep the loads in
@@ -311,20 +413,20 @@ struct F2Triple {
 
 
 // After an in-place length-n/2 forward transform of z (row in LDS), the
-// packed half-spectrum word k of the real row: needs Z[k] and Z[n/2 - k].
+// packed half-spectrum word k of the real row, from a = Z[k] and zmk =
+// Z[n/2 - k] (unused for k = 0).
 // twn = exp(-2 pi i k / n) for this k.
-__device__ __forceinline__ float2 r2c_combine(const float2* Z, int k, int half, float2 twn) {
-  if (k == 0) {
-    float2 z0 = Z[0];
-    return make_float2(z0.x + z0.y, z0.x - z0.y);
-  }
-  const float2 a = Z[k];
-  const float2 b = cconj(Z[half - k]);
+__device__ __forceinline__ float2 r2c_pair(float2 a, float2 zmk, int k, float2 twn) {
+  if (k == 0) return make_float2(a.x + a.y, a.x - a.y);
+  const float2 b = cconj(zmk);
   // Ze = (a + b)/2, Zo = (a - b)/(2i); X = Ze + W^k Zo
   const float2 ze = make_float2(0.5f * (a.x + b.x), 0.5f * (a.y + b.y));
   const float2 d = csub(a, b);
   const float2 zo = make_float2(0.5f * d.y, -0.5f * d.x);
   return cadd(ze, cmul(twn, zo));
+}
+__device__ __forceinline__ float2 r2c_combine(const float2* Z, int k, int half, float2 twn) {
+  return r2c_pair(Z[k], Z[(half - k) & (half - 1)], k, twn);
 }
 
 // Inverse combine: from packed half-spectrum words P[k], P[n/2 - k] build

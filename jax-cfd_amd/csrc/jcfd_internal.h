@@ -268,6 +268,7 @@ int li_launch_interpolate(int n, const float* coef, const float* x, int key, flo
 struct NsParams {
   const float* kx;        // fftfreq(n, dx), n values
   const float* ky;        // rfftfreq(n, dy), n/2+1 values
+  float dnx, rcp_dnx;     // fp32(dx n) and RN(1 / dnx): kx[i] = index / dnx
   const float2* tw;       // twiddles exp(-2 pi i k / n)
   const int* force_idx;   // (p, c) pairs of the forcing-curl entries
   const float2* force_val;

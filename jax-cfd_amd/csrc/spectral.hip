@@ -44,16 +44,13 @@ constexpr int kThreads = 256;
 
 // Internal layout of packed half spectra (n rows x n/2 words: the four
 // derivative spectra G and the product spectrum P): column tiles of kTw<N>
-// words, each tile one contiguous block of n rows x kTw words.  A column
-// kernel's tile is then a contiguous block, and a row kernel's rows cover
-// whole cache lines in every tile (4 rows x 4 words = 128 bytes), where the
-// row-major layout left 32-byte pieces of 2 KB rows to both.  From 512 on
-// the column kernels run two-column tiles: tiles of 2 words make each of
-// their rows a whole 16-byte piece of one tile (with 4-word tiles two
-// workgroups wrote the halves of every 32-byte piece; the update-and-inverse
-// kernel at 64 x 512^2 ran 149 instead of 133 us).
+// words, each tile one contiguous block of n rows x kTw words.  kTw is the
+// number of columns a column kernel's wavefront holds side by side, up to 4:
+// its loads and stores are then whole contiguous runs (at 64 x 512^2 the
+// update-and-inverse kernel took 123 / 146 / 185 us with tiles of 1 / 2 / 4
+// words), while the row kernel's pieces are its rows x kTw words.
 template <int N>
-constexpr int kTw = N >= 512 ? 2 : 4;
+constexpr int kTw = N == 512 ? 1 : N == 1024 || N == 256 ? 2 : 4;
 template <int N>
 __device__ __forceinline__ int tix(int p, int c) {
   return ((c / kTw<N>) * N + p) * kTw<N> + (c % kTw<N>);
@@ -87,239 +84,202 @@ __device__ __forceinline__ NsMult ns_mult(const NsParams& q, float kx, float ky,
 // i a * z
 __device__ __forceinline__ float2 mul_i(float a, float2 z) { return make_float2(-a * z.y, a * z.x); }
 
-// Spectrum m in {0: d_x w, 1: d_y w, 2: v_x, 3: v_y, 4: w itself} at (p, c).
-__device__ __forceinline__ float2 ns_spectrum(int m, const NsMult& k, float2 w) {
-  switch (m) {
-    case 0: return mul_i(k.ax, w);
-    case 1: return mul_i(k.ay, w);
-    case 2: return mul_i(k.ay, make_float2(k.psi * w.x, k.psi * w.y));
-    case 3: return mul_i(-k.ax, make_float2(k.psi * w.x, k.psi * w.y));
-    default: return w;
+// ---- column kernels ----------------------------------------------------------
+// A column transform is held in the registers of one wavefront's lanes
+// (reg_fft): N / E lanes per column, T columns side by side, neighbouring
+// lanes on neighbouring columns.  E = 8 words per lane (16 for N = 1024), so a
+// wavefront's tile is 512 (1024) words.  Everything a lane needs between the
+// forward transform, the update and the inverse transforms of the four
+// spectra sits at the same rows p = j + e L, so the tile never leaves its
+// registers: LDS carries two exchanges per 512-point transform, and no
+// workgroup barrier exists; the wavefronts of a workgroup are independent.
+// What bounds them is the stream of u, h, P and G: 16 x 512^2
+// update-and-inverse 30 us (5.0 TB/s) where the staged kernel takes 39,
+// 64 x 256^2 30 (35), 8 x 1024^2 68 (97).  Steps: 64 x 256^2 336 -> 277 us,
+// 256 x 128^2 364 -> 256, 32 x 512^2 599 -> 548, 8 x 1024^2 759 -> 645
+// (staged kernels at their best shapes -> these).
+template <int N>
+struct ColShape {
+  static constexpr int E = N == 1024 ? 16 : 8;
+  static constexpr int L = N / E;  // lanes per column
+  static constexpr int T = 64 / L;  // columns per wavefront
+};
+template <int N>
+constexpr int col_waves(int w) {  // wavefronts of a workgroup of w columns
+  return (w + ColShape<N>::T - 1) / ColShape<N>::T;
+}
+// LDS of a workgroup of `waves` wavefronts: their exchange buffers, then
+// vorticity columns 0 and N/2 of tile 0.
+template <int N>
+constexpr int col_lds(int waves) {
+  return (waves * kRegFftWords<N, ColShape<N>::T> + 2 * N) * static_cast<int>(sizeof(float2));
+}
+template <int N>
+struct ColLds {
+  float2 *x, *w0, *wn;
+  __device__ __forceinline__ ColLds(char* smem, int waves, int wave) {
+    float2* f = reinterpret_cast<float2*>(smem);
+    x = f + wave * kRegFftWords<N, ColShape<N>::T>;
+    w0 = f + waves * kRegFftWords<N, ColShape<N>::T>;
+    wn = w0 + N;
   }
+};
+
+// One lane's place in its wavefront's tile of columns from c0, of which the
+// workgroup owns the first w.
+template <int N>
+struct ColLane {
+  static constexpr int E = ColShape<N>::E, L = ColShape<N>::L, T = ColShape<N>::T;
+  int j;     // rows j + e L
+  int c;     // column
+  int t;     // its index in the wavefront
+  bool own;  // whether the column is this workgroup's (false: a surplus lane, which works on column c0 and stores nothing)
+  __device__ __forceinline__ ColLane(int c0, int w, int lane) : j(lane / T), c(c0), t(lane % T), own(lane % T < w) {
+    if (own) c = c0 + t;
+  }
+};
+
+// kx at row p = j + e L (e a compile-time number once unrolled): the table
+// entry fp32(index) / fp32(dx n), by over_step's correctly rounded quotient,
+// so neither loads nor registers are spent on the table.
+template <int N>
+__device__ __forceinline__ float lane_kx(const NsParams& q, float jf, int e) {
+  constexpr int E = ColShape<N>::E, L = ColShape<N>::L;
+  return over_step(jf + static_cast<float>(e < E / 2 ? e * L : e * L - N), q.dnx, q.rcp_dnx);
 }
 
-// Spectra built and inverse-transformed per round of the inverse column
-// work: a round's spectra sit side by side as NSP * W columns of one LDS
-// tile, so one set of FFT passes (and barriers) serves all of them.  NSP is
-// the largest of 4, 2, 1 whose round fits kNsRoundWords complex words.
-constexpr int kNsMaxSpectraPerRound = 4;
-constexpr int kNsRoundWords = 2048;
-template <int N, int W>
-struct NsRound {
-  static constexpr int value = (kNsMaxSpectraPerRound >= 4 && 4 * N * W <= kNsRoundWords) ? 4
-                               : (kNsMaxSpectraPerRound >= 2 && 2 * N * W <= kNsRoundWords) ? 2
-                                                                                            : 1;
-};
-
-template <int N, int W>
-struct ColShared {
-  float2 buf[N * W * NsRound<N, W>::value];  // work tile [p][c] (inverse rounds: [p][spectrum][c])
-  float2 w0[N];       // tile 0: vorticity column 0
-  float2 wn[N];       // tile 0: vorticity column N/2
-  float2 tw[N];
-  float kx[N];        // fftfreq
-  float ky[N / 2 + 1];  // rfftfreq
-};
-
-// Elements of a column tile are owned by threads as e = tid + k * kThreads;
-// each thread keeps its vorticity values in registers across the four spectra
-// (only tile 0's DC/Nyquist columns, which pair rows p and -p, also go through
-// LDS).
-template <int N, int W>
-struct WTile {
-  static constexpr int PER = (N * W + kThreads - 1) / kThreads;
-  float2 w[PER];
-};
-
-// Build spectrum m of the tile into sm.buf (scaled by 1/n^2), symmetrising and
-// packing the DC/Nyquist pair into local column 0 of tile 0.  psi[k] is
-// -1/laplacian at this thread's element k (columns other than 0; one
-// division per element for all four spectra); 2 pi kx, 2 pi ky come from
-// the LDS wavenumber tables.
-template <int N, int W, int NSP = 1>
-__device__ __forceinline__ void build_spectrum(ColShared<N, W>& sm, const WTile<N, W>& wt,
-                                               const float (&psi)[WTile<N, W>::PER],
-                                               const NsParams& q, int m, int slot, int c0, int tid) {
-  constexpr int H = N / 2;
-#pragma unroll
-  for (int k = 0; k < WTile<N, W>::PER; ++k) {
-    const int e = tid + k * kThreads;
-    if (e >= N * W) break;
-    const int p = e / W, c = e % W, cg = c0 + c;
-    float2 out;
-    if (cg != 0) {
-      NsMult mk;
-      mk.ax = q.two_pi * sm.kx[p];
-      mk.ay = q.two_pi * sm.ky[cg];
-      mk.psi = psi[k];
-      out = ns_spectrum(m, mk, wt.w[k]);
-    } else {
-      const int pm = (N - p) & (N - 1);
-      const float2 a0 = ns_spectrum(m, ns_mult(q, sm.kx[p], sm.ky[0], p == 0), sm.w0[p]);
-      const float2 b0 = ns_spectrum(m, ns_mult(q, sm.kx[pm], sm.ky[0], pm == 0), sm.w0[pm]);
-      const float2 ah = ns_spectrum(m, ns_mult(q, sm.kx[p], sm.ky[H], false), sm.wn[p]);
-      const float2 bh = ns_spectrum(m, ns_mult(q, sm.kx[pm], sm.ky[H], false), sm.wn[pm]);
-      const float2 s0 = make_float2(0.5f * (a0.x + b0.x), 0.5f * (a0.y - b0.y));
-      const float2 sh = make_float2(0.5f * (ah.x + bh.x), 0.5f * (ah.y - bh.y));
-      out = make_float2(s0.x - sh.y, s0.y + sh.x);  // s0 + i sh
-    }
-    sm.buf[p * (NSP * W) + slot * W + c] = make_float2(out.x * q.inv_nn, out.y * q.inv_nn);
-  }
+// x, as a value the compiler has to take as new: what is computed from it is
+// recomputed where it is used instead of being kept in registers from an
+// earlier use (a loop's invariants and the values shared by its halves cost
+// the column kernels the fourth wavefront per SIMD).
+__device__ __forceinline__ float recompute(float x) {
+  asm volatile("" : "+v"(x));
+  return x;
 }
 
 // Inverse column transforms of the tile -> G[0..NSPEC): the four derivative
-// spectra (NSPEC = 4) or the field itself (NSPEC = 1).  sm.w0 / sm.wn must be
-// visible (barrier) before the call.
-template <int N, int W, int NSPEC = 4, int R = 8>
-__device__ __forceinline__ void cols_inverse_body(ColShared<N, W>& sm, const WTile<N, W>& wt,
-                                                  const NsParams& q, float2* __restrict__ g,
-                                                  int c0, int tid) {
-  constexpr int H = N / 2;
-  constexpr int PER = WTile<N, W>::PER;
+// spectra (NSPEC = 4: d_x w, d_y w, v_x, v_y) or the field itself (NSPEC = 1),
+// scaled by 1/n^2.  w becomes psi w, psi = -1/laplacian, for the last two, so
+// no second array is held.  Column 0 is the symmetrised pair of the DC and
+// Nyquist columns, s0 + i sh with s(p) = (a(p) + conj a(-p)) / 2, from the two
+// columns in LDS (w0, wn): kx(-p) = -kx(p) (but at 0 and N/2), psi(-p) = psi(p).
+template <int N, int NSPEC, int R, typename TW>
+__device__ __forceinline__ void cols_inverse_body(float2 (&w)[ColShape<N>::E], const TW& tw, const ColLane<N>& ln,
+                                                  const ColLds<N>& lds, const NsParams& q,
+                                                  float2* __restrict__ g) {
+  using S = ColShape<N>;
+  constexpr int E = S::E, L = S::L, H = N / 2;
   const size_t gstride = static_cast<size_t>(N) * H;
-  float psi[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int e = tid + k * kThreads;
-    const int p = (e < N * W ? e : N * W - 1) / W, cg = c0 + e % W;
-    psi[k] = (NSPEC == 4 && cg != 0) ? ns_mult(q, sm.kx[p], sm.ky[cg], false).psi : 0.f;
-  }
-  constexpr int NSP = NSPEC < NsRound<N, W>::value ? NSPEC : NsRound<N, W>::value;
-  static_assert(NSPEC % NSP == 0, "whole rounds");
+  const float ky = q.ky[ln.c], kyh = q.ky[H];
+  const float ay = q.two_pi * ky, ayh = q.two_pi * kyh;
 #pragma unroll 1
-  for (int m0 = 0; m0 < NSPEC; m0 += NSP) {
+  for (int m = 0; m < NSPEC; ++m) {
+    const float jf = recompute(static_cast<float>(ln.j));
+    if (m == 2) {
 #pragma unroll
-    for (int j = 0; j < NSP; ++j)
-      build_spectrum<N, W, NSP>(sm, wt, psi, q, NSPEC == 1 ? 4 : m0 + j, j, c0, tid);
-    __syncthreads();
-    lds_fft<N, NSP * W, kThreads, NSP * W, 1, true, true, R>(sm.buf, sm.tw, tid);
-#pragma unroll
-    for (int j = 0; j < NSP; ++j) {
-      float2* gm = g + (m0 + j) * gstride;
-      float2 o[PER];
-#pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int e = tid + k * kThreads;
-        if ((N * W) % kThreads == 0 || e < N * W) o[k] = sm.buf[(e / W) * (NSP * W) + j * W + e % W];
+      for (int e = 0; e < E; ++e) {
+        const float psi = ns_mult(q, lane_kx<N>(q, jf, e), ky, ln.c == 0 && ln.j + e * L == 0).psi;
+        w[e] = make_float2(psi * w[e].x, psi * w[e].y);
       }
+      if (ln.c == 0 && ln.own) {  // the two columns in LDS likewise
+        wave_lds_sync();
 #pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int e = tid + k * kThreads;
-        if ((N * W) % kThreads == 0 || e < N * W) gm[tix<N>(e / W, c0 + e % W)] = o[k];
+        for (int e = 0; e < E; ++e) {
+          __builtin_amdgcn_sched_barrier(0);
+          const int p = ln.j + e * L;
+          const float psih = ns_mult(q, lane_kx<N>(q, jf, e), kyh, false).psi;
+          lds.w0[p] = w[e];
+          lds.wn[p] = make_float2(psih * lds.wn[p].x, psih * lds.wn[p].y);
+        }
+        wave_lds_sync();
       }
     }
-    __syncthreads();
-  }
-}
-
-// The state tile (internal layout when TILED, else the external rfft2
-// layout) into registers; tile 0 also stages columns 0 and N/2 in LDS.
-template <int N, int W, bool TILED>
-__device__ __forceinline__ void load_w_tile(ColShared<N, W>& sm, WTile<N, W>& wt, const NsParams& q,
-                                            const float2* __restrict__ w, int c0, int tid) {
-  constexpr int H1 = N / 2 + 1;
-  auto at = [&](int p, int c) { return TILED ? six<N>(p, c) : p * H1 + c; };
+    // the spectrum's multiplier is i times kx or ky; v_y's is -i kx
+    const bool along_y = m == 1 || m == 2;
+    const float sign = m == 3 ? -1.0f : 1.0f;
+    float2 v[E];
 #pragma unroll
-  for (int k = 0; k < WTile<N, W>::PER; ++k) {
-    const int e = tid + k * kThreads;
-    if (e >= N * W) break;
-    const int p = e / W, c = e % W;
-    wt.w[k] = w[at(p, c0 + c)];
-  }
-  if (c0 == 0) {
-    constexpr int PN = (N + kThreads - 1) / kThreads;
-    float2 a[PN], b[PN];
+    for (int e = 0; e < E; ++e) {
+      const float k = along_y ? ay : q.two_pi * lane_kx<N>(q, jf, e);
+      v[e] = NSPEC == 1 ? w[e] : mul_i(sign * k, w[e]);
+    }
+    if (ln.c == 0 && ln.own) {
 #pragma unroll
-    for (int k = 0; k < PN; ++k) {
-      const int p = tid + k * kThreads;
-      if (N % kThreads == 0 || p < N) {
-        a[k] = w[at(p, 0)];
-        b[k] = w[at(p, N / 2)];
+      for (int e = 0; e < E; ++e) {
+        __builtin_amdgcn_sched_barrier(0);  // one element's temporaries at a time
+        const int p = ln.j + e * L, pm = (N - p) & (N - 1);
+        const float2 z0 = lds.w0[pm], zp = lds.wn[p], zm = lds.wn[pm];
+        const float kx1 = lane_kx<N>(q, jf, e);
+        const float kp = sign * (q.two_pi * kx1), km = pm == p ? kp : -kp;
+        const float2 a0 = v[e];
+        const float2 b0 = NSPEC == 1 ? z0 : mul_i(along_y ? ay : km, z0);
+        const float2 ah = NSPEC == 1 ? zp : mul_i(along_y ? ayh : kp, zp);
+        const float2 bh = NSPEC == 1 ? zm : mul_i(along_y ? ayh : km, zm);
+        const float2 s0 = make_float2(0.5f * (a0.x + b0.x), 0.5f * (a0.y - b0.y));
+        const float2 sh = make_float2(0.5f * (ah.x + bh.x), 0.5f * (ah.y - bh.y));
+        v[e] = make_float2(s0.x - sh.y, s0.y + sh.x);  // s0 + i sh
       }
     }
 #pragma unroll
-    for (int k = 0; k < PN; ++k) {
-      const int p = tid + k * kThreads;
-      if (N % kThreads == 0 || p < N) {
-        sm.w0[p] = a[k];
-        sm.wn[p] = b[k];
-      }
+    for (int e = 0; e < E; ++e) v[e] = make_float2(v[e].x * q.inv_nn, v[e].y * q.inv_nn);
+    reg_fft<N, E, S::T, true, R>(v, tw, lds.x + ln.t, ln.j);
+    if (ln.own) {
+      float2* gm = g + m * gstride + tix<N>(ln.j, ln.c);
+#pragma unroll
+      for (int e = 0; e < E; ++e) gm[e * (L * kTw<N>)] = v[e];
     }
   }
 }
 
-// Wavenumber tables staged through registers (load() issues the global
-// loads, store() writes LDS), like TwiddleStage.
+// Minimum waves per SIMD asked of the column kernels: 128 registers hold an E =
+// 8 tile with its old (u, h) and twiddles, 256 an E = 16 one.
 template <int N>
-struct WavenumberStage {
-  static constexpr int PX = (N + kThreads - 1) / kThreads;
-  static constexpr int PY = (N / 2 + 1 + kThreads - 1) / kThreads;
-  float x[PX], y[PY];
-  __device__ __forceinline__ void load(const NsParams& q, int tid) {
-#pragma unroll
-    for (int k = 0; k < PX; ++k) {
-      const int i = tid + k * kThreads;
-      x[k] = q.kx[N % kThreads == 0 || i < N ? i : N - 1];
-    }
-#pragma unroll
-    for (int k = 0; k < PY; ++k) {
-      const int i = tid + k * kThreads;
-      y[k] = q.ky[i <= N / 2 ? i : N / 2];
-    }
-  }
-  __device__ __forceinline__ void store(float* kx, float* ky, int tid) const {
-#pragma unroll
-    for (int k = 0; k < PX; ++k) {
-      const int i = tid + k * kThreads;
-      if (N % kThreads == 0 || i < N) kx[i] = x[k];
-    }
-#pragma unroll
-    for (int k = 0; k < PY; ++k) {
-      const int i = tid + k * kThreads;
-      if (i <= N / 2) ky[i] = y[k];
-    }
-  }
+struct NsColOcc {
+  static constexpr int value = N == 1024 ? 2 : 4;
 };
 
-
-// Minimum waves per SIMD asked of the column kernels: 5 for the 512-point
-// tiles of one or two columns, the most their LDS (inverse rounds of two or
-// four spectra) allows; other shapes keep the compiler's choice (wider
-// tiles would spill).
-template <int N, int W>
-struct NsColWaves {
-  static constexpr int value = (N == 512 && W <= 2) ? 5 : 1;
-};
-
-// One column tile: the state's W columns from c0 -> the inverse transforms of
-// the four spectra (NSPEC = 4) or of the field (NSPEC = 1); w and g already
-// point at the instance.
-template <int N, int W, int NSPEC, int R = 8>
-__device__ __forceinline__ void cols_inverse_tile(ColShared<N, W>& sm, const NsParams& q,
+// One wavefront's columns from c0: the state -> the inverse transforms of the
+// four spectra (NSPEC = 4) or of the field (NSPEC = 1); w and g already point
+// at the instance.
+template <int N, int NSPEC, int R>
+__device__ __forceinline__ void cols_inverse_tile(const ColLds<N>& lds, const NsParams& q,
                                                   const float2* __restrict__ w, float2* __restrict__ g,
-                                                  int c0, int tid) {
-  WTile<N, W> wt;
-  TwiddleStage<N, 1, kThreads> tw;
-  WavenumberStage<N> wn;
-  tw.load(q.tw, tid);
-  wn.load(q, tid);
+                                                  int c0, int width, int lane) {
+  using S = ColShape<N>;
+  constexpr int E = S::E, L = S::L, H = N / 2;
+  const ColLane<N> ln(c0, width, lane);
   // the step (NSPEC = 4) reads the internal state, irfft2 (NSPEC = 1) the
   // caller's array
-  load_w_tile<N, W, NSPEC == 4>(sm, wt, q, w, c0, tid);
-  tw.store(sm.tw, tid);
-  wn.store(sm.kx, sm.ky, tid);
-  __syncthreads();
-  cols_inverse_body<N, W, NSPEC, R>(sm, wt, q, g, c0, tid);
+  auto at = [&](int p, int c) { return NSPEC == 4 ? six<N>(p, c) : p * (H + 1) + c; };
+  float2 wt[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) wt[e] = w[at(ln.j + e * L, ln.c)];
+  RegTwiddles<N, E, R> tw;
+  tw.template load<1>(q.tw, ln.j);
+  if (c0 == 0) {
+    if (ln.c == 0 && ln.own) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        lds.w0[ln.j + e * L] = wt[e];
+        lds.wn[ln.j + e * L] = w[at(ln.j + e * L, H)];
+      }
+    }
+    wave_lds_sync();
+  }
+  cols_inverse_body<N, NSPEC, R>(wt, tw, ln, lds, q, g);
 }
 
-template <int N, int W, int NSPEC, int R = 8>
-__global__ __launch_bounds__(kThreads, (NsColWaves<N, W>::value)) void ns_cols_inverse(NsParams q, const float2* __restrict__ w,
-                                                            float2* __restrict__ g) {
-  __shared__ ColShared<N, W> sm;
-  const int c0 = xcd_tile(blockIdx.x, gridDim.x) * W;
+template <int N, int NSPEC, int R>
+__global__ __launch_bounds__(1024 / ColShape<N>::E * 8, (NsColOcc<N>::value)) void ns_cols_inverse(
+    NsParams q, const float2* __restrict__ w, float2* __restrict__ g, int width) {
+  extern __shared__ float4 ns_smem[];
+  const int wave = threadIdx.x / 64;
+  const ColLds<N> lds(reinterpret_cast<char*>(ns_smem), blockDim.x / 64, wave);
+  const int c0 = xcd_tile(blockIdx.x, gridDim.x) * width + wave * ColShape<N>::T;
   const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
-  cols_inverse_tile<N, W, NSPEC, R>(sm, q, w + inst * static_cast<size_t>(N) * (N / 2 + 1),
-                                    g + inst * NSPEC * static_cast<size_t>(N) * (N / 2), c0, threadIdx.x);
+  cols_inverse_tile<N, NSPEC, R>(lds, q, w + inst * static_cast<size_t>(N) * (N / 2 + 1),
+                                        g + inst * NSPEC * static_cast<size_t>(N) * (N / 2), c0, width,
+                                        threadIdx.x % 64);
 }
 
 // Packed real row transforms of a batch of real (N, N) fields.
@@ -379,113 +339,217 @@ __global__ __launch_bounds__(kThreads) void rows_c2r(NsParams q, const float2* _
   for (int e = tid; e < RB * N; e += kThreads) x[static_cast<size_t>(i0) * N + e] = zf[e];
 }
 
-template <int N, int RB>
-struct RowsShared {
-  float2 rows[4 * RB * (N / 2)];  // transform t = m * RB + r
-  float2 twn[N];
-  float2 twh[N / 2];
+// ---- row kernel -----------------------------------------------------------
+// A wavefront transforms RS rows of one spectrum in registers (512 words, E =
+// 8 per lane); the four wavefronts of a group take the four spectra of the
+// same rows, wavefront 0 then forms the product and transforms it forward
+// (64 x 256^2: 31 us with every pass staged in LDS, 22 us so).
+// RB rows per workgroup: RB / RS groups, or one group with surplus lanes.
+template <int N>
+struct RowShape {
+  static constexpr int H = N / 2, E = 8;
+  static constexpr int L = H / E;      // lanes per row
+  static constexpr int RS = 64 / L;    // rows per wavefront
 };
-
-// One row block: rows i0 .. i0+RB-1 of the four spectra G -> the product
-// spectrum rows of P; g and pout already point at the instance.
-template <int N, int RB, int R = 8>
-__device__ __forceinline__ void rows_tile(RowsShared<N, RB>& sm, const NsParams& q,
-                                          const float2* __restrict__ g, float2* __restrict__ pout,
-                                          int i0, int tid) {
-  constexpr int H = N / 2;
-  const size_t gstride = static_cast<size_t>(N) * H;
-  float2* rows = sm.rows;
-  // the product spectrum overwrites the first transform's rows (gx, element
-  // by element: each element is read and written by its owner only)
-  float2* prod = sm.rows;
-  float2* twn = sm.twn;
-  float2* twh = sm.twh;
-  // Load the four spectra's rows in chunks (all loads of a chunk issued
-  // together); the twiddle tables go to LDS while the first chunk is in
-  // flight.  Words are taken in mirror pairs (kk, H - kk), kk < H/2: both
-  // outputs of a pair need both words, so each word is read once.  Element
-  // e walks the first half of the tiled layout in memory order: word w of
-  // the tile, then row r (the RB rows of a tile are contiguous), then the
-  // tile, then the spectrum m; word H/2 (its own mirror) goes alone.
-  constexpr int HH = H / 2;
-  constexpr int TW = kTw<N>;
-  static_assert(HH % TW == 0, "whole tiles in each half row");
-  constexpr int TOT = 4 * RB * HH;
-  constexpr int PER = (TOT + kThreads - 1) / kThreads;
-  constexpr int C = PER < 8 ? PER : 8;
-  static_assert(4 * RB <= kThreads, "one thread per middle word");
-  TwiddleStage<N, 1, kThreads> ta;
-  TwiddleStage<H, 2, kThreads> tb;
-  ta.load(q.tw, tid);
-  tb.load(q.tw, tid);
-  float2 mid = make_float2(0.f, 0.f);
-  if (tid < 4 * RB) mid = g[(tid / RB) * gstride + tix<N>(i0 + tid % RB, HH)];
-#pragma unroll 1
-  for (int k0 = 0; k0 < PER; k0 += C) {
-    float2 a[C], b[C];
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-      const int e = tid + (k0 + k) * kThreads;
-      if (e < TOT) {
-        const int r = (e / TW) % RB, kk = ((e / (TW * RB)) % (HH / TW)) * TW + e % TW;
-        const float2* gm = g + (e / (RB * HH)) * gstride;
-        a[k] = gm[tix<N>(i0 + r, kk)];
-        b[k] = gm[tix<N>(i0 + r, (H - kk) & (H - 1))];
-      }
-    }
-    if (k0 == 0) {
-      ta.store(twn, tid);
-      tb.store(twh, tid);
-      __syncthreads();
-      if (tid < 4 * RB) rows[tid * H + HH] = c2r_combine(mid, mid, HH, twn[HH]);
-    }
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-      const int e = tid + (k0 + k) * kThreads;
-      if (e < TOT) {
-        const int r = (e / TW) % RB, kk = ((e / (TW * RB)) % (HH / TW)) * TW + e % TW;
-        float2* row = rows + ((e / (RB * HH)) * RB + r) * H;
-        row[kk] = c2r_combine(a[k], b[k], kk, twn[kk]);
-        if (kk != 0) row[H - kk] = c2r_combine(b[k], a[k], H - kk, twn[H - kk]);
-      }
-    }
-  }
-  __syncthreads();
-  lds_fft_waves<H, 4 * RB, kThreads, 1, H, true, R>(rows, twh, tid);
-  // advection = -(grad_x * vx + grad_y * vy)  (spectral/equations.py:170)
-  const float* gx = reinterpret_cast<const float*>(rows);
-  const float* gy = gx + RB * N;
-  const float* vx = gy + RB * N;
-  const float* vy = vx + RB * N;
-  float* pr = reinterpret_cast<float*>(prod);
-  staged<RB * N, 8, kThreads>(
-      tid, [&](int e) { return -(gx[e] * vx[e] + gy[e] * vy[e]); },
-      [&](int e, float v) { pr[e] = v; });
-  __syncthreads();
-  // The product's RB forward transforms: with radix-8 passes a transform
-  // has H / 8 butterflies, half a wavefront's lanes or fewer for n <= 512;
-  // radix-4 passes (H / 4 butterflies) issue fewer instructions per
-  // wavefront there.  A function of n and the plan's radix only, so every
-  // row tile shape still gives the same bits.
-  constexpr int RF = (R == 8 && N <= 512) ? 4 : R;
-  lds_fft_waves<H, RB, kThreads, 1, H, false, RF>(prod, twh, tid);
-  // element e in the tiled layout's memory order, as for the loads
-  auto row_of = [](int e) { return (e / TW) % RB; };
-  auto word_of = [](int e) { return (e / (TW * RB)) * TW + e % TW; };
-  staged<RB * H, 8, kThreads>(
-      tid, [&](int e) { return r2c_combine(prod + row_of(e) * H, word_of(e), H, twn[word_of(e)]); },
-      [&](int e, float2 v) { pout[tix<N>(i0 + row_of(e), word_of(e))] = v; });
+template <int N>
+constexpr int row_groups(int rb) {
+  return rb > RowShape<N>::RS ? rb / RowShape<N>::RS : 1;
+}
+template <int N>
+constexpr int kRowBuffer = kRegFftWords<N / 2, RowShape<N>::RS>;  // words per wavefront
+template <int N>
+constexpr int row_lds(int rb) {
+  return row_groups<N>(rb) * 4 * kRowBuffer<N> * static_cast<int>(sizeof(float2));
 }
 
+// NR rows per group from i0: spectrum m = wave % 4 of G -> the product
+// spectrum rows of P; g and pout already point at the instance.
+template <int N, int NR, int R>
+__device__ __forceinline__ void rows_tile(float2* smem, const NsParams& q, const float2* __restrict__ g,
+                                          float2* __restrict__ pout, int i0, int tid) {
+  using S = RowShape<N>;
+  constexpr int H = S::H, E = S::E, L = S::L, RS = S::RS, HH = H / 2, TW = kTw<N>;
+  static_assert(NR <= RS, "rows per wavefront");
+  const int wave = tid / 64, lane = tid % 64, m = wave % 4;
+  i0 += (wave / 4) * NR;
+  float2* xb = smem + wave * kRowBuffer<N>;
+  const float2* gm = g + m * static_cast<size_t>(N) * H;
+  // Loads in the tiled layout's memory order (word of the tile, row, tile),
+  // in mirror pairs (kk, H - kk), kk < H/2: both outputs of a pair need both
+  // words, so each word is read once; word H/2 (its own mirror) goes alone.
+  // Element k of row r goes to LDS word fft_pad(k) RS + r, where the
+  // transform's lanes pick it up.
+  constexpr int TOT = NR * HH, PER = (TOT + 63) / 64;
+  auto row_of = [](int e) { return (e / TW) % NR; };
+  auto word_of = [](int e) { return (e / (TW * NR)) * TW + e % TW; };
+  float2 a[PER], b[PER], ta[PER], tb[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e0 = lane + 64 * k, e = TOT % 64 == 0 || e0 < TOT ? e0 : TOT - 1;
+    const int r = row_of(e), kk = word_of(e);
+    a[k] = gm[tix<N>(i0 + r, kk)];
+    b[k] = gm[tix<N>(i0 + r, (H - kk) & (H - 1))];
+    ta[k] = q.tw[kk];
+    tb[k] = q.tw[(H - kk) & (N - 1)];
+  }
+  float2 mid = make_float2(0.f, 0.f);
+  const float2 tmid = q.tw[HH];
+  if (lane < NR) mid = gm[tix<N>(i0 + lane, HH)];
+  const int j = lane / RS, t = lane % RS;
+  RegTwiddles<H, E, R> tw;
+  tw.template load<2>(q.tw, j);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = lane + 64 * k;
+    if (TOT % 64 == 0 || e < TOT) {
+      const int r = row_of(e), kk = word_of(e);
+      xb[fft_pad(kk) * RS + r] = c2r_combine(a[k], b[k], kk, ta[k]);
+      if (kk != 0) xb[fft_pad(H - kk) * RS + r] = c2r_combine(b[k], a[k], H - kk, tb[k]);
+    }
+  }
+  if (lane < NR) xb[fft_pad(HH) * RS + lane] = c2r_combine(mid, mid, HH, tmid);
+  wave_lds_sync();
+  float2 v[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = xb[fft_pad(j) * RS + fft_pad(e * L) * RS + t];
+  reg_fft<H, E, RS, true, R>(v, tw, xb + t, j);
+  // advection = -(grad_x * vx + grad_y * vy)  (spectral/equations.py:170):
+  // each wavefront leaves its field in its own buffer, wavefront 0 of the
+  // group reads the other three
+  if (m != 0) {
+    wave_lds_sync();
+#pragma unroll
+    for (int e = 0; e < E; ++e) xb[lane + 64 * e] = v[e];
+  }
+  __syncthreads();
+  if (m != 0) return;
+  const float2* gy = xb + kRowBuffer<N>;
+  const float2* vx = gy + kRowBuffer<N>;
+  const float2* vy = vx + kRowBuffer<N>;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const float2 y = gy[lane + 64 * e], cx = vx[lane + 64 * e], cy = vy[lane + 64 * e];
+    v[e] = make_float2(-(v[e].x * cx.x + y.x * cy.x), -(v[e].y * cx.y + y.y * cy.y));
+  }
+  reg_fft<H, E, RS, false, R>(v, tw, xb + t, j);
+  wave_lds_sync();
+#pragma unroll
+  for (int e = 0; e < E; ++e) xb[fft_pad(j) * RS + fft_pad(e * L) * RS + t] = v[e];
+  wave_lds_sync();
+  constexpr int OUT = NR * H, POUT = (OUT + 63) / 64;
+#pragma unroll
+  for (int k = 0; k < POUT; ++k) {
+    const int e = lane + 64 * k;
+    if (OUT % 64 == 0 || e < OUT) {
+      const int r = row_of(e), kk = word_of(e);
+      pout[tix<N>(i0 + r, kk)] = r2c_pair(xb[fft_pad(kk) * RS + r], xb[fft_pad((H - kk) & (H - 1)) * RS + r], kk, q.tw[kk]);
+    }
+  }
+}
 
-template <int N, int RB, int R = 8>
-__global__ __launch_bounds__(kThreads) void ns_rows(NsParams q, const float2* __restrict__ g,
-                                                    float2* __restrict__ pout) {
-  __shared__ RowsShared<N, RB> sm;
+template <int N, int NR, int R>
+__global__ __launch_bounds__(1024) void ns_rows(NsParams q, const float2* __restrict__ g,
+                                                float2* __restrict__ pout) {
+  extern __shared__ float4 ns_smem[];
   const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
   const size_t gstride = static_cast<size_t>(N) * (N / 2);
-  rows_tile<N, RB, R>(sm, q, g + inst * 4 * gstride, pout + inst * gstride,
-                      xcd_tile(blockIdx.x, gridDim.x) * RB, threadIdx.x);
+  rows_tile<N, NR, R>(reinterpret_cast<float2*>(ns_smem), q, g + inst * 4 * gstride, pout + inst * gstride,
+                      xcd_tile(blockIdx.x, gridDim.x) * (blockDim.x / 256) * NR, threadIdx.x);
+}
+
+// The row kernel of launches that fill the chip: four wavefronts take 4 RS
+// rows, each wavefront its RS rows of the four spectra one after the other
+// (the next spectrum's words on their way meanwhile), so every wavefront
+// works to the end and the workgroup's global pieces are 4 RS rows x kTw
+// words long.  The words come in through one of two staging buffers; a
+// wavefront's part of a buffer then serves as its exchange buffer.
+template <int N, int R>
+__device__ __forceinline__ void rows_seq_tile(float2* smem, const NsParams& q, const float2* __restrict__ g,
+                                              float2* __restrict__ pout, int i0, int tid) {
+  using S = RowShape<N>;
+  constexpr int H = S::H, E = S::E, L = S::L, RS = S::RS, RB = 4 * RS, HH = H / 2, TW = kTw<N>;
+  constexpr int PER = RB * HH / 256, OUT = RB * H / 256, BUF = 4 * kRowBuffer<N>;
+  static_assert(RB * HH % 256 == 0 && HH % TW == 0, "whole chunks");
+  const int wave = tid / 64, lane = tid % 64;
+  auto row_of = [](int e) { return (e / TW) % RB; };
+  auto word_of = [](int e) { return (e / (TW * RB)) * TW + e % TW; };
+  // word k of row r of the block
+  auto slot = [](int r, int k) { return (r / RS) * kRowBuffer<N> + fft_pad(k) * RS + r % RS; };
+  const size_t gstride = static_cast<size_t>(N) * H;
+  float2 a[PER], b[PER], mid = make_float2(0.f, 0.f);
+  auto load = [&](int m) {
+    const float2* gm = g + m * gstride;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + 256 * k, r = row_of(e), kk = word_of(e);
+      a[k] = gm[tix<N>(i0 + r, kk)];
+      b[k] = gm[tix<N>(i0 + r, (H - kk) & (H - 1))];
+    }
+    if (tid < RB) mid = gm[tix<N>(i0 + tid, HH)];
+  };
+  load(0);
+  const float2 tmid = q.tw[HH];
+  const int j = lane / RS, t = lane % RS;
+  RegTwiddles<H, E, R> tw;
+  tw.template load<2>(q.tw, j);
+  // advection = -(grad_x * vx + grad_y * vy)  (spectral/equations.py:170)
+  float2 v[E], prod[E];
+#pragma unroll
+  for (int step = 0; step < 4; ++step) {
+    constexpr int order[4] = {0, 2, 1, 3};  // grad_x, vx, grad_y, vy
+    float2* buf = smem + (step & 1) * BUF;
+    const float2* tab = q.tw;  // the combine's twiddles are read again for each spectrum: registers are scarcer
+    asm volatile("" : "+s"(tab));
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + 256 * k, r = row_of(e), kk = word_of(e);
+      buf[slot(r, kk)] = c2r_combine(a[k], b[k], kk, as_global(tab)[kk]);
+      if (kk != 0) buf[slot(r, H - kk)] = c2r_combine(b[k], a[k], H - kk, as_global(tab)[H - kk]);
+    }
+    if (tid < RB) buf[slot(tid, HH)] = c2r_combine(mid, mid, HH, tmid);
+    if (step < 3) load(order[step < 3 ? step + 1 : 3]);
+    // also orders the rewriting of a buffer after every wavefront's last
+    // exchange in it, two steps before
+    __syncthreads();
+    float2* xb = buf + wave * kRowBuffer<N> + t;
+    float2 f[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) f[e] = xb[(fft_pad(j) + fft_pad(e * L)) * RS];
+    reg_fft<H, E, RS, true, R>(f, tw, xb, j);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (step == 0) prod[e] = f[e];
+      else if (step == 1) prod[e] = make_float2(prod[e].x * f[e].x, prod[e].y * f[e].y);
+      else if (step == 2) v[e] = f[e];
+      else v[e] = make_float2(-(prod[e].x + v[e].x * f[e].x), -(prod[e].y + v[e].y * f[e].y));
+    }
+  }
+  float2* xw = smem + BUF + wave * kRowBuffer<N> + t;
+  reg_fft<H, E, RS, false, R>(v, tw, xw, j);
+  wave_lds_sync();
+#pragma unroll
+  for (int e = 0; e < E; ++e) xw[(fft_pad(j) + fft_pad(e * L)) * RS] = v[e];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < OUT; ++k) {
+    const int e = tid + 256 * k, r = row_of(e), kk = word_of(e);
+    const float2* z = smem + BUF;
+    pout[tix<N>(i0 + r, kk)] = r2c_pair(z[slot(r, kk)], z[slot(r, (H - kk) & (H - 1))], kk, q.tw[kk]);
+  }
+}
+template <int N>
+constexpr int row_seq_lds() {
+  return 2 * 4 * kRowBuffer<N> * static_cast<int>(sizeof(float2));
+}
+
+template <int N, int R>
+__global__ __launch_bounds__(256, 4) void ns_rows_seq(NsParams q, const float2* __restrict__ g,
+                                                      float2* __restrict__ pout) {
+  extern __shared__ float4 ns_smem[];
+  const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
+  const size_t gstride = static_cast<size_t>(N) * (N / 2);
+  rows_seq_tile<N, R>(reinterpret_cast<float2*>(ns_smem), q, g + inst * 4 * gstride, pout + inst * gstride,
+                      xcd_tile(blockIdx.x, gridDim.x) * 4 * RowShape<N>::RS, threadIdx.x);
 }
 
 // External rfft2 layout <-> internal state layout of one instance per
@@ -516,8 +580,6 @@ __global__ __launch_bounds__(kThreads) void ns_state_convert(const float2* __res
     dst[base + static_cast<size_t>(p) * H1 + c] = src[base + t];
 }
 
-constexpr int kForceRegs = 4;  // forcing-curl entries kept in registers
-
 // 2/3 rule mask (spectral/utils.py:128-134).
 __device__ __forceinline__ float ns_filter(const NsParams& q, int p, int c) {
   if (!q.smooth) return 1.0f;
@@ -525,20 +587,416 @@ __device__ __forceinline__ float ns_filter(const NsParams& q, int p, int c) {
   return (row && c < q.filt_cols) ? 1.0f : 0.0f;
 }
 
-// MODE 0: write F (explicit terms) to u_out in the external layout.
-// MODE 1: RK/CN update of (u, h) (internal state layout).
-// MODE 2: update, then the next stage's inverse column work on the new tile.
-// One column tile of the forward column pass: P's W columns from c0 ->
-// explicit terms (MODE 0), the RK/CN update (MODE 1), or the update followed
-// by the next stage's inverse work (MODE 2); all pointers already point at
-// the instance.
-template <int N, int W, int MODE, int R = 8>
-__device__ __forceinline__ void cols_forward_tile(ColShared<N, W>& sm, const NsParams& q,
+// One wavefront's columns from c0 of the forward column pass: P's columns ->
+// explicit terms F in the external layout (MODE 0), the RK/CN update of
+// (u, h) in the internal state layout (MODE 1), or the update followed by the
+// next stage's inverse work on the new columns (MODE 2); all pointers already
+// point at the instance.
+template <int N, int MODE, int R>
+__device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const NsParams& q,
+                                                  const float2* __restrict__ pin, const float2* u_in,
+                                                  float2* u_out, float2* h, float2* __restrict__ g,
+                                                  int c0, int width, int lane) {
+  using S = ColShape<N>;
+  constexpr int E = S::E, L = S::L, T = S::T, H = N / 2, H1 = H + 1;
+  constexpr int ES = L * kTw<N>;  // words between a lane's elements, in P, G, u and h
+  const ColLane<N> ln(c0, width, lane);
+  const int at0 = tix<N>(ln.j, ln.c);  // the lane's element 0 (u and h: six = tix for c < N/2)
+  // Every global load up front, in the order of use: P and the twiddles,
+  // then the state (each element is read and written by its owner only, so
+  // reading u and h before the transform is safe also when u_in == u_out).
+  float2 v[E];
+  const float2* pl = pin + at0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = pl[e * ES];
+  RegTwiddles<N, E, R> tw;
+  tw.template load<1>(q.tw, ln.j);
+  [[maybe_unused]] float2 uo[MODE == 0 ? 1 : E], ho[MODE == 0 ? 1 : E];
+  [[maybe_unused]] float ky = 0.f;
+  if constexpr (MODE != 0) {
+    const float2* ul = u_in + at0;
+    const float2* hl = h + at0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      uo[e] = ul[e * ES];
+      ho[e] = q.read_h ? hl[e * ES] : make_float2(0.f, 0.f);
+    }
+    ky = q.ky[ln.c];
+    if (ln.c == 0 && ln.own) {  // (u, h) of the Nyquist column, parked in LDS
+      const float2* uh = u_in + six<N>(ln.j, H);
+      const float2* hh = h + six<N>(ln.j, H);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        lds.wn[ln.j + e * L] = uh[e * L];
+        if (q.read_h) lds.w0[ln.j + e * L] = hh[e * L];
+      }
+    }
+  }
+  float2* x = lds.x;
+  reg_fft<N, E, T, false, R>(v, tw, x + ln.t, ln.j);
+
+  // h = F + beta h;  u = (u + g h + mu L u) / (1 - mu L), with the old
+  // (u, h) at wavenumber (kx, ky) given; returns u and leaves h in fv.
+  auto update = [&](float kxp, float kyc, float2& fv, float2 u0, float2 h0) -> float2 {
+    if (q.read_h) fv = make_float2(fv.x + q.beta * h0.x, fv.y + q.beta * h0.y);
+    const float lap = q.neg_four_pi_sq * (kxp * kxp + kyc * kyc);
+    const float Lc = q.nu * lap - q.drag;
+    const float2 lu = make_float2(Lc * u0.x, Lc * u0.y);
+    const float2 xx = make_float2((u0.x + q.g * fv.x) + q.mu * lu.x, (u0.y + q.g * fv.y) + q.mu * lu.y);
+    const float inv = 1.0f / (1.0f - q.mu * Lc);
+    return make_float2(inv * xx.x, inv * xx.y);
+  };
+  [[maybe_unused]] const float jf = recompute(static_cast<float>(ln.j));
+
+  if (c0 == 0) {
+    // column 0 of tile 0 carries the DC (A) and Nyquist (B) columns:
+    // A = (Y(p) + conj Y(-p))/2, B = (Y(p) - conj Y(-p))/(2i)
+    float2* xt = x + ln.t;
+    wave_lds_sync();
+#pragma unroll
+    for (int e = 0; e < E; ++e) xt[fft_pad(ln.j + e * L) * T] = v[e];
+    wave_lds_sync();
+    if (ln.c == 0 && ln.own) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const float2 ym = cconj(xt[fft_pad((N - ln.j - e * L) & (N - 1)) * T]);
+        v[e] = make_float2(0.5f * (v[e].x + ym.x), 0.5f * (v[e].y + ym.y));
+      }
+      bool forced = false;  // entries in the Nyquist column
+      for (int t = 0; t < q.n_force; ++t) forced |= q.force_idx[2 * t + 1] == H;
+      // F at (p, H), from the transform left in the exchange buffer
+      auto nyquist = [&](int p) -> float2 {
+        const float2 d = csub(xt[fft_pad(p) * T], cconj(xt[fft_pad((N - p) & (N - 1)) * T]));
+        const float m = ns_filter(q, p, H);
+        float2 f = make_float2((0.5f * d.y) * m, (-0.5f * d.x) * m);
+        if (forced)
+          for (int t = 0; t < q.n_force; ++t)
+            if (q.force_idx[2 * t] == p && q.force_idx[2 * t + 1] == H) f = cadd(f, q.force_val[t]);
+        return f;
+      };
+      if constexpr (MODE == 0) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) u_out[(ln.j + e * L) * H1 + H] = nyquist(ln.j + e * L);
+      } else {
+        const float kyh = q.ky[H];
+        float2* hn = h + six<N>(ln.j, H);
+        float2* un = u_out + six<N>(ln.j, H);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+          const int p = ln.j + e * L;
+          const float2 h0 = q.read_h ? lds.w0[p] : make_float2(0.f, 0.f);
+          float2 f = nyquist(p);
+          const float2 w = update(lane_kx<N>(q, jf, e), kyh, f, lds.wn[p], h0);
+          hn[e * L] = f;
+          un[e * L] = w;
+          if constexpr (MODE == 2) lds.wn[p] = w;
+        }
+      }
+    }
+  }
+  // F: the filter, then the sparse, time-constant forcing curl entries (the
+  // list is the same for every lane; row p belongs to lane p % L, element p / L)
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const float m = ns_filter(q, ln.j + e * L, ln.c);
+    v[e] = make_float2(v[e].x * m, v[e].y * m);
+  }
+  for (int t = 0; t < q.n_force; ++t) {
+    const int fp = q.force_idx[2 * t], fc = q.force_idx[2 * t + 1], se = fp / L;
+    if (fc == ln.c && fp % L == ln.j) {
+      const float2 f = q.force_val[t];
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (e == se) v[e] = cadd(v[e], f);
+    }
+  }
+  if constexpr (MODE == 0) {
+    if (ln.own) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) u_out[(ln.j + e * L) * H1 + ln.c] = v[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two elements' updates in registers at a time
+      uo[e] = update(lane_kx<N>(q, jf, e), ky, v[e], uo[e], ho[e]);
+    }
+    if (ln.own) {
+      float2* hs = h + at0;
+      float2* us = u_out + at0;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        hs[e * ES] = v[e];
+        us[e * ES] = uo[e];
+      }
+    }
+  }
+  if constexpr (MODE == 2) {
+    if (c0 == 0) {
+      if (ln.c == 0 && ln.own) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) lds.w0[ln.j + e * L] = uo[e];
+      }
+      wave_lds_sync();
+    }
+    cols_inverse_body<N, 4, R>(uo, tw, ln, lds, q, g);
+  }
+}
+
+template <int N, int MODE, int R>
+__global__ __launch_bounds__(1024 / ColShape<N>::E * 8, (NsColOcc<N>::value)) void ns_cols_forward(
+    NsParams q, const float2* __restrict__ pin, const float2* u_in, float2* u_out, float2* h,
+    float2* __restrict__ g, int width) {
+  extern __shared__ float4 ns_smem[];
+  const int wave = threadIdx.x / 64;
+  const ColLds<N> lds(reinterpret_cast<char*>(ns_smem), blockDim.x / 64, wave);
+  const int c0 = xcd_tile(blockIdx.x, gridDim.x) * width + wave * ColShape<N>::T;
+  const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
+  const size_t ext = static_cast<size_t>(N) * (N / 2 + 1);
+  cols_forward_tile<N, MODE, R>(lds, q, pin + inst * static_cast<size_t>(N) * (N / 2),
+                                u_in ? u_in + inst * ext : nullptr, u_out + inst * ext,
+                                h ? h + inst * ext : nullptr,
+                                g ? g + inst * 4 * static_cast<size_t>(N) * (N / 2) : nullptr, c0, width,
+                                threadIdx.x % 64);
+}
+
+// ---- staged column kernels: launches too small to fill the chip -----------
+// A workgroup of 256 threads per tile of W columns, the tile in LDS around
+// every pass: a lone 512-word column keeps four wavefronts busy, where a
+// register transform is one wavefront's serial work (1 x 256^2
+// update-and-inverse 6.1 us against 12.7; at 64 x 256^2, where wavefronts
+// abound, 35 against 30, at 16 x 512^2 39 against 30).
+constexpr int kForceRegs = 4;  // forcing-curl entries kept in registers
+// Widest tile the staged kernels serve; wider ones are for large launches.
+template <int N>
+constexpr int kStagedMaxW = N == 32 ? 16 : N == 64 ? 8 : N == 128 ? 4 : N == 256 ? 2 : 1;
+
+// Spectrum m in {0: d_x w, 1: d_y w, 2: v_x, 3: v_y} at (p, c).
+__device__ __forceinline__ float2 ns_spectrum(int m, const NsMult& k, float2 w) {
+  switch (m) {
+    case 0: return mul_i(k.ax, w);
+    case 1: return mul_i(k.ay, w);
+    case 2: return mul_i(k.ay, make_float2(k.psi * w.x, k.psi * w.y));
+    default: return mul_i(-k.ax, make_float2(k.psi * w.x, k.psi * w.y));
+  }
+}
+
+// Spectra built and inverse-transformed per round of the inverse column
+// work: a round's spectra sit side by side as NSP * W columns of one LDS
+// tile, so one set of FFT passes (and barriers) serves all of them.  NSP is
+// the largest of 4, 2, 1 whose round fits kNsRoundWords complex words.
+constexpr int kNsMaxSpectraPerRound = 4;
+constexpr int kNsRoundWords = 2048;
+template <int N, int W>
+struct NsRound {
+  static constexpr int value = (kNsMaxSpectraPerRound >= 4 && 4 * N * W <= kNsRoundWords) ? 4
+                               : (kNsMaxSpectraPerRound >= 2 && 2 * N * W <= kNsRoundWords) ? 2
+                                                                                            : 1;
+};
+
+template <int N, int W>
+struct StagedCols {
+  float2 buf[N * W * NsRound<N, W>::value];  // work tile [p][c] (inverse rounds: [p][spectrum][c])
+  float2 w0[N];       // tile 0: vorticity column 0
+  float2 wn[N];       // tile 0: vorticity column N/2
+  float2 tw[N];
+  float kx[N];        // fftfreq
+  float ky[N / 2 + 1];  // rfftfreq
+};
+
+// Elements of a column tile are owned by threads as e = tid + k * kThreads;
+// each thread keeps its vorticity values in registers across the four spectra
+// (only tile 0's DC/Nyquist columns, which pair rows p and -p, also go through
+// LDS).
+template <int N, int W>
+struct WTile {
+  static constexpr int PER = (N * W + kThreads - 1) / kThreads;
+  float2 w[PER];
+};
+
+// Build spectrum m of the tile into sm.buf (scaled by 1/n^2), symmetrising and
+// packing the DC/Nyquist pair into local column 0 of tile 0.  psi[k] is
+// -1/laplacian at this thread's element k (columns other than 0; one
+// division per element for all four spectra); 2 pi kx, 2 pi ky come from
+// the LDS wavenumber tables.
+template <int N, int W, int NSP = 1>
+__device__ __forceinline__ void staged_spectrum(StagedCols<N, W>& sm, const WTile<N, W>& wt,
+                                               const float (&psi)[WTile<N, W>::PER],
+                                               const NsParams& q, int m, int slot, int c0, int tid) {
+  constexpr int H = N / 2;
+#pragma unroll
+  for (int k = 0; k < WTile<N, W>::PER; ++k) {
+    const int e = tid + k * kThreads;
+    if (e >= N * W) break;
+    const int p = e / W, c = e % W, cg = c0 + c;
+    float2 out;
+    if (cg != 0) {
+      NsMult mk;
+      mk.ax = q.two_pi * sm.kx[p];
+      mk.ay = q.two_pi * sm.ky[cg];
+      mk.psi = psi[k];
+      out = ns_spectrum(m, mk, wt.w[k]);
+    } else {
+      const int pm = (N - p) & (N - 1);
+      const float2 a0 = ns_spectrum(m, ns_mult(q, sm.kx[p], sm.ky[0], p == 0), sm.w0[p]);
+      const float2 b0 = ns_spectrum(m, ns_mult(q, sm.kx[pm], sm.ky[0], pm == 0), sm.w0[pm]);
+      const float2 ah = ns_spectrum(m, ns_mult(q, sm.kx[p], sm.ky[H], false), sm.wn[p]);
+      const float2 bh = ns_spectrum(m, ns_mult(q, sm.kx[pm], sm.ky[H], false), sm.wn[pm]);
+      const float2 s0 = make_float2(0.5f * (a0.x + b0.x), 0.5f * (a0.y - b0.y));
+      const float2 sh = make_float2(0.5f * (ah.x + bh.x), 0.5f * (ah.y - bh.y));
+      out = make_float2(s0.x - sh.y, s0.y + sh.x);  // s0 + i sh
+    }
+    sm.buf[p * (NSP * W) + slot * W + c] = make_float2(out.x * q.inv_nn, out.y * q.inv_nn);
+  }
+}
+
+// Inverse column transforms of the tile -> G[0..4).  sm.w0 / sm.wn must be
+// visible (barrier) before the call.
+template <int N, int W, int R>
+__device__ __forceinline__ void staged_inverse_body(StagedCols<N, W>& sm, const WTile<N, W>& wt,
+                                                  const NsParams& q, float2* __restrict__ g,
+                                                  int c0, int tid) {
+  constexpr int H = N / 2;
+  constexpr int PER = WTile<N, W>::PER;
+  const size_t gstride = static_cast<size_t>(N) * H;
+  float psi[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = tid + k * kThreads;
+    const int p = (e < N * W ? e : N * W - 1) / W, cg = c0 + e % W;
+    psi[k] = cg != 0 ? ns_mult(q, sm.kx[p], sm.ky[cg], false).psi : 0.f;
+  }
+  constexpr int NSP = NsRound<N, W>::value;
+#pragma unroll 1
+  for (int m0 = 0; m0 < 4; m0 += NSP) {
+#pragma unroll
+    for (int j = 0; j < NSP; ++j)
+      staged_spectrum<N, W, NSP>(sm, wt, psi, q, m0 + j, j, c0, tid);
+    __syncthreads();
+    lds_fft<N, NSP * W, kThreads, NSP * W, 1, true, true, R>(sm.buf, sm.tw, tid);
+#pragma unroll
+    for (int j = 0; j < NSP; ++j) {
+      float2* gm = g + (m0 + j) * gstride;
+      float2 o[PER];
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int e = tid + k * kThreads;
+        if ((N * W) % kThreads == 0 || e < N * W) o[k] = sm.buf[(e / W) * (NSP * W) + j * W + e % W];
+      }
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int e = tid + k * kThreads;
+        if ((N * W) % kThreads == 0 || e < N * W) gm[tix<N>(e / W, c0 + e % W)] = o[k];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The state tile into registers; tile 0 also stages columns 0 and N/2 in LDS.
+template <int N, int W>
+__device__ __forceinline__ void staged_load(StagedCols<N, W>& sm, WTile<N, W>& wt, const NsParams& q,
+                                            const float2* __restrict__ w, int c0, int tid) {
+#pragma unroll
+  for (int k = 0; k < WTile<N, W>::PER; ++k) {
+    const int e = tid + k * kThreads;
+    if (e >= N * W) break;
+    const int p = e / W, c = e % W;
+    wt.w[k] = w[six<N>(p, c0 + c)];
+  }
+  if (c0 == 0) {
+    constexpr int PN = (N + kThreads - 1) / kThreads;
+    float2 a[PN], b[PN];
+#pragma unroll
+    for (int k = 0; k < PN; ++k) {
+      const int p = tid + k * kThreads;
+      if (N % kThreads == 0 || p < N) {
+        a[k] = w[six<N>(p, 0)];
+        b[k] = w[six<N>(p, N / 2)];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < PN; ++k) {
+      const int p = tid + k * kThreads;
+      if (N % kThreads == 0 || p < N) {
+        sm.w0[p] = a[k];
+        sm.wn[p] = b[k];
+      }
+    }
+  }
+}
+
+// Wavenumber tables staged through registers (load() issues the global
+// loads, store() writes LDS), like TwiddleStage.
+template <int N>
+struct WavenumberStage {
+  static constexpr int PX = (N + kThreads - 1) / kThreads;
+  static constexpr int PY = (N / 2 + 1 + kThreads - 1) / kThreads;
+  float x[PX], y[PY];
+  __device__ __forceinline__ void load(const NsParams& q, int tid) {
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      const int i = tid + k * kThreads;
+      x[k] = q.kx[N % kThreads == 0 || i < N ? i : N - 1];
+    }
+#pragma unroll
+    for (int k = 0; k < PY; ++k) {
+      const int i = tid + k * kThreads;
+      y[k] = q.ky[i <= N / 2 ? i : N / 2];
+    }
+  }
+  __device__ __forceinline__ void store(float* kx, float* ky, int tid) const {
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      const int i = tid + k * kThreads;
+      if (N % kThreads == 0 || i < N) kx[i] = x[k];
+    }
+#pragma unroll
+    for (int k = 0; k < PY; ++k) {
+      const int i = tid + k * kThreads;
+      if (i <= N / 2) ky[i] = y[k];
+    }
+  }
+};
+
+
+// Minimum waves per SIMD asked of the column kernels: 5 for the 512-point
+// tiles of one or two columns, the most their LDS (inverse rounds of two or
+// four spectra) allows; other shapes keep the compiler's choice (wider
+// tiles would spill).
+template <int N, int W>
+struct StagedWaves {
+  static constexpr int value = (N == 512 && W <= 2) ? 5 : 1;
+};
+
+template <int N, int W, int R>
+__global__ __launch_bounds__(kThreads, (StagedWaves<N, W>::value)) void ns_cols_inverse_staged(
+    NsParams q, const float2* __restrict__ w, float2* __restrict__ g) {
+  __shared__ StagedCols<N, W> sm;
+  const int tid = threadIdx.x;
+  const int c0 = xcd_tile(blockIdx.x, gridDim.x) * W;
+  const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
+  WTile<N, W> wt;
+  TwiddleStage<N, 1, kThreads> tw;
+  WavenumberStage<N> wn;
+  tw.load(q.tw, tid);
+  wn.load(q, tid);
+  staged_load<N, W>(sm, wt, q, w + inst * static_cast<size_t>(N) * (N / 2 + 1), c0, tid);
+  tw.store(sm.tw, tid);
+  wn.store(sm.kx, sm.ky, tid);
+  __syncthreads();
+  staged_inverse_body<N, W, R>(sm, wt, q, g + inst * 4 * static_cast<size_t>(N) * (N / 2), c0, tid);
+}
+
+// As cols_forward_tile: the update (MODE 1), or the update and the next
+// stage's inverse work on the same tile (MODE 2).
+template <int N, int W, int MODE, int R>
+__device__ __forceinline__ void staged_forward_tile(StagedCols<N, W>& sm, const NsParams& q,
                                                   const float2* __restrict__ pin, const float2* u_in,
                                                   float2* u_out, float2* h, float2* __restrict__ g,
                                                   int c0, int tid) {
   constexpr int H = N / 2;
-  constexpr int H1 = H + 1;
   constexpr int PER = (N * W + kThreads - 1) / kThreads;
 
   // Every global load of the kernel's first half is issued up front: the
@@ -549,29 +1007,27 @@ __device__ __forceinline__ void cols_forward_tile(ColShared<N, W>& sm, const NsP
   // before it, so the tables (needed first) go first and (u, h) (needed
   // after the transform) last.
   TwiddleStage<N, 1, kThreads> tws;
-  [[maybe_unused]] WavenumberStage<N> wns;
+  WavenumberStage<N> wns;
   tws.load(q.tw, tid);
-  if constexpr (MODE != 0) wns.load(q, tid);
+  wns.load(q, tid);
   float2 pv[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int e = tid + k * kThreads;
     if ((N * W) % kThreads == 0 || e < N * W) pv[k] = pin[tix<N>(e / W, c0 + e % W)];
   }
-  [[maybe_unused]] float2 u_pre[MODE == 0 ? 1 : PER], h_pre[MODE == 0 ? 1 : PER];
-  if constexpr (MODE != 0) {
+  float2 u_pre[PER], h_pre[PER];
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int e = tid + k * kThreads;
-      if ((N * W) % kThreads == 0 || e < N * W) {
-        const int idx = six<N>(e / W, c0 + e % W);
-        u_pre[k] = u_in[idx];
-        h_pre[k] = q.read_h ? h[idx] : make_float2(0.f, 0.f);
-      }
+  for (int k = 0; k < PER; ++k) {
+    const int e = tid + k * kThreads;
+    if ((N * W) % kThreads == 0 || e < N * W) {
+      const int idx = six<N>(e / W, c0 + e % W);
+      u_pre[k] = u_in[idx];
+      h_pre[k] = q.read_h ? h[idx] : make_float2(0.f, 0.f);
     }
   }
   tws.store(sm.tw, tid);
-  if constexpr (MODE != 0) wns.store(sm.kx, sm.ky, tid);
+  wns.store(sm.kx, sm.ky, tid);
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int e = tid + k * kThreads;
@@ -618,7 +1074,7 @@ __device__ __forceinline__ void cols_forward_tile(ColShared<N, W>& sm, const NsP
   }
 
   // Per element: F at (p, cg) (filter, then the sparse, time-constant forcing
-  // curl entries), then the update (or F itself for MODE 0); tile 0 also
+  // curl entries), then the update; tile 0 also
   // handles column N/2.  One pass, so no array of F values stays live.
   [[maybe_unused]] WTile<N, W> wt;
 #pragma unroll
@@ -653,43 +1109,39 @@ __device__ __forceinline__ void cols_forward_tile(ColShared<N, W>& sm, const NsP
           if (cg == 0 && fp == p && fc == H) fh = cadd(fh, q.force_val[t]);
         }
       }
-      if constexpr (MODE == 0) {
-        u_out[p * H1 + cg] = f;
-        if (cg == 0) u_out[p * H1 + H] = fh;
-      } else {
-        const float2 un = update_with(p, cg, f, u_pre[k], h_pre[k]);
-        if constexpr (MODE == 2) {
-          wt.w[k] = un;
-          if (cg == 0) {
-            sm.w0[p] = un;
-            sm.wn[p] = update_nyquist(p, fh);
-          }
-        } else {
-          if (cg == 0) update_nyquist(p, fh);
+      const float2 un = update_with(p, cg, f, u_pre[k], h_pre[k]);
+      if constexpr (MODE == 2) {
+        wt.w[k] = un;
+        if (cg == 0) {
+          sm.w0[p] = un;
+          sm.wn[p] = update_nyquist(p, fh);
         }
+      } else {
+        if (cg == 0) update_nyquist(p, fh);
       }
     }
   }
   if constexpr (MODE == 2) {
     __syncthreads();  // sm.buf read by all; sm.w0 / sm.wn written
-    cols_inverse_body<N, W, 4, R>(sm, wt, q, g, c0, tid);
+    staged_inverse_body<N, W, R>(sm, wt, q, g, c0, tid);
   }
 }
 
 
-template <int N, int W, int MODE, int R = 8>
-__global__ __launch_bounds__(kThreads, (NsColWaves<N, W>::value)) void ns_cols_forward(NsParams q, const float2* __restrict__ pin,
+template <int N, int W, int MODE, int R>
+__global__ __launch_bounds__(kThreads, (StagedWaves<N, W>::value)) void ns_cols_forward_staged(NsParams q, const float2* __restrict__ pin,
                                                             const float2* u_in, float2* u_out,
                                                             float2* h, float2* __restrict__ g) {
-  __shared__ ColShared<N, W> sm;
+  __shared__ StagedCols<N, W> sm;
   const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
   const size_t ext = static_cast<size_t>(N) * (N / 2 + 1);
-  cols_forward_tile<N, W, MODE, R>(sm, q, pin + inst * static_cast<size_t>(N) * (N / 2),
+  staged_forward_tile<N, W, MODE, R>(sm, q, pin + inst * static_cast<size_t>(N) * (N / 2),
                                    u_in ? u_in + inst * ext : nullptr, u_out + inst * ext,
                                    h ? h + inst * ext : nullptr,
                                    g ? g + inst * 4 * static_cast<size_t>(N) * (N / 2) : nullptr,
                                    xcd_tile(blockIdx.x, gridDim.x) * W, threadIdx.x);
 }
+
 
 // ---- mixed-size group step ---------------------------------------------------
 // Every item is 1024 complex words of work whatever its grid size (column
@@ -699,32 +1151,44 @@ __global__ __launch_bounds__(kThreads, (NsColWaves<N, W>::value)) void ns_cols_f
 template <int N>
 struct NsGroupShape {
   static constexpr int W = (1024 / N < N / 2) ? 1024 / N : N / 2;
-  static constexpr int RB = (1024 / N < N / 4) ? 1024 / N : N / 4;
+  static constexpr bool kSeq = N >= 256;  // rows by rows_seq_tile
+  static constexpr int RB = kSeq ? 4 * RowShape<N>::RS : ((1024 / N < N / 4) ? 1024 / N : N / 4);
 };
+
+// Threads of a group launch: two wavefronts of columns, or the four of a row
+// block.
+constexpr int ns_group_threads(int cls) { return cls == 1 ? 256 : 128; }
 
 template <int N, int CLS>
 __device__ __forceinline__ void ns_group_tile(const NsGroupDesc& d, int tile, int tid, char* smem) {
   using S = NsGroupShape<N>;
   if constexpr (CLS == 1) {
-    rows_tile<N, S::RB, 8>(*reinterpret_cast<RowsShared<N, S::RB>*>(smem), d.q, d.g, d.pbuf,
-                           tile * S::RB, tid);
-  } else {
-    auto& sm = *reinterpret_cast<ColShared<N, S::W>*>(smem);
-    if constexpr (CLS == 0)
-      cols_inverse_tile<N, S::W, 4, 8>(sm, d.q, d.ws, d.g, tile * S::W, tid);
+    if constexpr (S::kSeq)
+      rows_seq_tile<N, 8>(reinterpret_cast<float2*>(smem), d.q, d.g, d.pbuf, tile * S::RB, tid);
     else
-      cols_forward_tile<N, S::W, CLS == 2 ? 2 : 1, 8>(sm, d.q, d.pbuf, d.ws, d.ws, d.h, d.g,
-                                                       tile * S::W, tid);
+      rows_tile<N, S::RB, 8>(reinterpret_cast<float2*>(smem), d.q, d.g, d.pbuf, tile * S::RB, tid);
+  } else {
+    const int wave = tid / 64;
+    constexpr int waves = col_waves<N>(S::W);
+    if (wave >= waves) return;
+    const ColLds<N> lds(smem, waves, wave);
+    const int c0 = tile * S::W + wave * ColShape<N>::T;
+    if constexpr (CLS == 0)
+      cols_inverse_tile<N, 4, 8>(lds, d.q, d.ws, d.g, c0, S::W, tid % 64);
+    else
+      cols_forward_tile<N, CLS == 2 ? 2 : 1, 8>(lds, d.q, d.pbuf, d.ws, d.ws, d.h, d.g, c0, S::W, tid % 64);
   }
 }
 
 // One workgroup per item (the host launches exactly the list's item count):
 // the hardware's workgroup dispatch keeps the CUs full, as for the per-size
-// kernels, with no loop state held in registers.
-template <int CLS>
-__global__ __launch_bounds__(kThreads) void ns_group_phase(const NsGroupDesc* __restrict__ descs,
-                                                           const NsGroupItem* __restrict__ items,
-                                                           const int* __restrict__ n_items, int stage) {
+// kernels, with no loop state held in registers.  Groups with 1024^2
+// instances have a build of their own (BIG): its 16 words per lane would
+// cost every other size registers.
+template <int CLS, bool BIG>
+__global__ __launch_bounds__(ns_group_threads(CLS), BIG ? 2 : 4) void ns_group_phase(
+    const NsGroupDesc* __restrict__ descs, const NsGroupItem* __restrict__ items,
+    const int* __restrict__ n_items, int stage) {
   extern __shared__ float4 ns_group_smem[];
   char* smem = reinterpret_cast<char*>(ns_group_smem);
   const int it = blockIdx.x;
@@ -748,7 +1212,9 @@ __global__ __launch_bounds__(kThreads) void ns_group_phase(const NsGroupDesc* __
     case 128: ns_group_tile<128, CLS>(d, w.tile, t, smem); break;
     case 256: ns_group_tile<256, CLS>(d, w.tile, t, smem); break;
     case 512: ns_group_tile<512, CLS>(d, w.tile, t, smem); break;
-    case 1024: ns_group_tile<1024, CLS>(d, w.tile, t, smem); break;
+    case 1024:
+      if constexpr (BIG) ns_group_tile<1024, CLS>(d, w.tile, t, smem);
+      break;
     default: break;  // rejected on the host
   }
 }
@@ -756,8 +1222,7 @@ __global__ __launch_bounds__(kThreads) void ns_group_phase(const NsGroupDesc* __
 template <int N>
 constexpr int ns_group_lds_n(int cls) {
   using S = NsGroupShape<N>;
-  return cls == 1 ? static_cast<int>(sizeof(RowsShared<N, S::RB>))
-                  : static_cast<int>(sizeof(ColShared<N, S::W>));
+  return cls == 1 ? (S::kSeq ? row_seq_lds<N>() : row_lds<N>(S::RB)) : col_lds<N>(col_waves<N>(S::W));
 }
 
 // dynamic LDS stays within the 64 KiB a launch gets without raising the
@@ -787,37 +1252,60 @@ template <> struct NsTiles<256> { static constexpr int W = 8, RB = 2; };
 template <> struct NsTiles<512> { static constexpr int W = 8, RB = 1; };
 template <> struct NsTiles<1024> { static constexpr int W = 4, RB = 1; };
 
+template <int N, int NSPEC, int R>
+void launch_cols_inverse(int w, const NsParams& q, const float2* in, float2* g, int batch, hipStream_t s) {
+  const int waves = col_waves<N>(w);
+  hipLaunchKernelGGL((ns_cols_inverse<N, NSPEC, R>), dim3(N / 2 / w, batch), dim3(64 * waves), col_lds<N>(waves), s,
+                     q, in, g, w);
+}
+template <int N, int MODE, int R>
+void launch_cols_forward(int w, const NsParams& q, const float2* pbuf, const float2* u_in, float2* u_out, float2* h,
+                         float2* g, int batch, hipStream_t s) {
+  const int waves = col_waves<N>(w);
+  hipLaunchKernelGGL((ns_cols_forward<N, MODE, R>), dim3(N / 2 / w, batch), dim3(64 * waves), col_lds<N>(waves), s, q,
+                     pbuf, u_in, u_out, h, g, w);
+}
+template <int N, int RB, int R>
+void launch_rows(const NsParams& q, const float2* g, float2* pbuf, int batch, hipStream_t s) {
+  constexpr int RS = RowShape<N>::RS, NR = RB < RS ? RB : RS;
+  if constexpr (RB == 4 * RS)
+    hipLaunchKernelGGL((ns_rows_seq<N, R>), dim3(N / RB, batch), dim3(256), row_seq_lds<N>(), s, q, g, pbuf);
+  else
+    hipLaunchKernelGGL((ns_rows<N, NR, R>), dim3(N / RB, batch), dim3(256 * row_groups<N>(RB)), row_lds<N>(RB), s, q,
+                       g, pbuf);
+}
+
 template <int N>
 struct NsOps {
   static constexpr int W = NsTiles<N>::W, RB = NsTiles<N>::RB;
   static int cols_inverse(const NsParams& q, const float2* w, float2* g, int batch, hipStream_t s) {
-    hipLaunchKernelGGL((ns_cols_inverse<N, W, 4>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, q, w, g);
+    launch_cols_inverse<N, 4, 8>(W, q, w, g, batch, s);
     return check_hip(hipGetLastError(), "ns_cols_inverse");
   }
+  // The external layout's rows are read and written column by column here,
+  // so many columns share a workgroup (and its cache lines).
   static int rfft2(const NsParams& q, const float* x, float2* out, float2* pbuf, int batch,
                    hipStream_t s) {
     NsParams plain = q;
     plain.smooth = 0;
     plain.n_force = 0;
     hipLaunchKernelGGL((rows_r2c<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, q, x, pbuf);
-    hipLaunchKernelGGL((ns_cols_forward<N, W, 0>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, plain,
-                       pbuf, nullptr, out, nullptr, nullptr);
+    launch_cols_forward<N, 0, 8>(W, plain, pbuf, nullptr, out, nullptr, nullptr, batch, s);
     return check_hip(hipGetLastError(), "rfft2");
   }
   static int irfft2(const NsParams& q, const float2* in, float* x, float2* pbuf, int batch,
                     hipStream_t s) {
-    hipLaunchKernelGGL((ns_cols_inverse<N, W, 1>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, q, in, pbuf);
+    launch_cols_inverse<N, 1, 8>(W, q, in, pbuf, batch, s);
     hipLaunchKernelGGL((rows_c2r<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, q, pbuf, x);
     return check_hip(hipGetLastError(), "irfft2");
   }
   static int rows(const NsParams& q, const float2* g, float2* pbuf, int batch, hipStream_t s) {
-    hipLaunchKernelGGL((ns_rows<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, q, g, pbuf);
+    launch_rows<N, (N >= 512 ? RB : 4), 8>(q, g, pbuf, batch, s);
     return check_hip(hipGetLastError(), "ns_rows");
   }
   // Forward column transforms of P -> explicit terms F (no update).
   static int explicit_cols(const NsParams& q, const float2* pbuf, float2* out, int batch, hipStream_t s) {
-    hipLaunchKernelGGL((ns_cols_forward<N, W, 0>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, q, pbuf,
-                       nullptr, out, nullptr, nullptr);
+    launch_cols_forward<N, 0, 8>(W, q, pbuf, nullptr, out, nullptr, nullptr, batch, s);
     return check_hip(hipGetLastError(), "ns_cols_forward");
   }
 };
@@ -829,13 +1317,13 @@ struct NsOps {
 // regroup the same per-column / per-row arithmetic and never change results.
 constexpr int kNsLdsMax = 96 * 1024;
 
-template <int N, int W>
-constexpr bool ns_cols_ok() {
-  return W <= N / 2 && N * W <= 16 * kThreads && sizeof(ColShared<N, W>) <= kNsLdsMax;
+template <int N>
+constexpr bool ns_cols_ok(int w) {
+  return w <= N / 2 && N * w <= 16 * kThreads && col_lds<N>(col_waves<N>(w)) <= kNsLdsMax;
 }
-template <int N, int RB>
-constexpr bool ns_rows_ok() {
-  return RB <= N / 4 && (4 * RB * (N / 2) + N + N / 2) * 8 <= kNsLdsMax;
+template <int N>
+constexpr bool ns_rows_ok(int rb) {
+  return rb <= N / 4 && row_groups<N>(rb) <= 4 && row_lds<N>(rb) <= kNsLdsMax;
 }
 
 // which: 0 cols-inverse, 1 rows, 2 cols-forward + update + next inverse,
@@ -844,23 +1332,30 @@ template <int N, int T, int R>
 int ns_variant(int which, const NsParams& q, const float2* a, const float2* u_in, float2* u_out,
                float2* h, float2* g, int batch, hipStream_t s) {
   if (which == 1) {
-    if constexpr (ns_rows_ok<N, T>()) {
-      hipLaunchKernelGGL((ns_rows<N, T, R>), dim3(N / T, batch), dim3(kThreads), 0, s, q, a, g);
+    if constexpr (ns_rows_ok<N>(T)) {
+      launch_rows<N, T, R>(q, a, g, batch, s);
       return JCFD_OK;
     }
     return JCFD_ERR_UNSUPPORTED;
   }
-  if constexpr (ns_cols_ok<N, T>()) {
+  if (!ns_cols_ok<N>(T)) return JCFD_ERR_UNSUPPORTED;
+  if constexpr (T <= kStagedMaxW<N>) {
     const dim3 grid(N / 2 / T, batch);
     if (which == 0)
-      hipLaunchKernelGGL((ns_cols_inverse<N, T, 4, R>), grid, dim3(kThreads), 0, s, q, a, g);
+      hipLaunchKernelGGL((ns_cols_inverse_staged<N, T, R>), grid, dim3(kThreads), 0, s, q, a, g);
     else if (which == 2)
-      hipLaunchKernelGGL((ns_cols_forward<N, T, 2, R>), grid, dim3(kThreads), 0, s, q, a, u_in, u_out, h, g);
+      hipLaunchKernelGGL((ns_cols_forward_staged<N, T, 2, R>), grid, dim3(kThreads), 0, s, q, a, u_in, u_out, h, g);
     else
-      hipLaunchKernelGGL((ns_cols_forward<N, T, 1, R>), grid, dim3(kThreads), 0, s, q, a, u_in, u_out, h, g);
+      hipLaunchKernelGGL((ns_cols_forward_staged<N, T, 1, R>), grid, dim3(kThreads), 0, s, q, a, u_in, u_out, h, g);
     return JCFD_OK;
   }
-  return JCFD_ERR_UNSUPPORTED;
+  if (which == 0)
+    launch_cols_inverse<N, 4, R>(T, q, a, g, batch, s);
+  else if (which == 2)
+    launch_cols_forward<N, 2, R>(T, q, a, u_in, u_out, h, g, batch, s);
+  else
+    launch_cols_forward<N, 1, R>(T, q, a, u_in, u_out, h, g, batch, s);
+  return JCFD_OK;
 }
 
 template <int N, int R>
@@ -870,8 +1365,8 @@ int ns_tile(int which, int tile, const NsParams& q, const float2* a, const float
     case 1: return ns_variant<N, 1, R>(which, q, a, u_in, u_out, h, g, batch, s);
     case 2: return ns_variant<N, 2, R>(which, q, a, u_in, u_out, h, g, batch, s);
     case 4: return ns_variant<N, 4, R>(which, q, a, u_in, u_out, h, g, batch, s);
-    case 8: return which == 1 ? JCFD_ERR_UNSUPPORTED : ns_variant<N, 8, R>(which, q, a, u_in, u_out, h, g, batch, s);
-    case 16: return which == 1 ? JCFD_ERR_UNSUPPORTED : ns_variant<N, 16, R>(which, q, a, u_in, u_out, h, g, batch, s);
+    case 8: return ns_variant<N, 8, R>(which, q, a, u_in, u_out, h, g, batch, s);
+    case 16: return ns_variant<N, 16, R>(which, q, a, u_in, u_out, h, g, batch, s);
     default: return JCFD_ERR_UNSUPPORTED;
   }
 }
@@ -903,11 +1398,11 @@ int ns_step_impl(const NsParams* stages, int nstages, const NsBuffers& b, int ba
 template <int N>
 bool ns_tile_on_menu(int which, int tile) {
   switch (tile) {
-    case 1: return which == 1 ? ns_rows_ok<N, 1>() : ns_cols_ok<N, 1>();
-    case 2: return which == 1 ? ns_rows_ok<N, 2>() : ns_cols_ok<N, 2>();
-    case 4: return which == 1 ? ns_rows_ok<N, 4>() : ns_cols_ok<N, 4>();
-    case 8: return which != 1 && ns_cols_ok<N, 8>();
-    case 16: return which != 1 && ns_cols_ok<N, 16>();
+    case 1: return which == 1 ? ns_rows_ok<N>(1) : ns_cols_ok<N>(1);
+    case 2: return which == 1 ? ns_rows_ok<N>(2) : ns_cols_ok<N>(2);
+    case 4: return which == 1 ? ns_rows_ok<N>(4) : ns_cols_ok<N>(4);
+    case 8: return which == 1 ? ns_rows_ok<N>(8) : ns_cols_ok<N>(8);
+    case 16: return which == 1 ? ns_rows_ok<N>(16) : ns_cols_ok<N>(16);
     default: return false;
   }
 }
@@ -937,17 +1432,26 @@ int ns_group_tiles(int n, int list) {
   }
 }
 
+namespace {
+template <bool BIG>
+int ns_group_dispatch(int cls, int max_n, const NsGroupQueue& q, int stage, int grid, hipStream_t s) {
+  const size_t lds = static_cast<size_t>(ns_group_lds(cls, max_n));
+  const dim3 g(grid), t(ns_group_threads(cls));
+  switch (cls) {
+    case 0: hipLaunchKernelGGL((ns_group_phase<0, BIG>), g, t, lds, s, q.descs, q.items[0], q.n_items, stage); break;
+    case 1: hipLaunchKernelGGL((ns_group_phase<1, BIG>), g, t, lds, s, q.descs, q.items[1], q.n_items + 1, stage); break;
+    case 2: hipLaunchKernelGGL((ns_group_phase<2, BIG>), g, t, lds, s, q.descs, q.items[0], q.n_items, stage); break;
+    default: hipLaunchKernelGGL((ns_group_phase<3, BIG>), g, t, lds, s, q.descs, q.items[0], q.n_items, stage);
+  }
+  return check_hip(hipGetLastError(), "spectral group launch");
+}
+}  // namespace
+
 int ns_group_launch(int cls, int max_n, const NsGroupQueue& q, int stage, int grid, hipStream_t s) {
   if (!ns_group_size_supported(max_n))
     return fail(JCFD_ERR_UNSUPPORTED, "spectral group grid size not supported: " + std::to_string(max_n));
-  const size_t lds = static_cast<size_t>(ns_group_lds(cls, max_n));
-  switch (cls) {
-    case 0: hipLaunchKernelGGL(ns_group_phase<0>, dim3(grid), dim3(kThreads), lds, s, q.descs, q.items[0], q.n_items, stage); break;
-    case 1: hipLaunchKernelGGL(ns_group_phase<1>, dim3(grid), dim3(kThreads), lds, s, q.descs, q.items[1], q.n_items + 1, stage); break;
-    case 2: hipLaunchKernelGGL(ns_group_phase<2>, dim3(grid), dim3(kThreads), lds, s, q.descs, q.items[0], q.n_items, stage); break;
-    default: hipLaunchKernelGGL(ns_group_phase<3>, dim3(grid), dim3(kThreads), lds, s, q.descs, q.items[0], q.n_items, stage);
-  }
-  return check_hip(hipGetLastError(), "spectral group launch");
+  return max_n > 512 ? ns_group_dispatch<true>(cls, max_n, q, stage, grid, s)
+                     : ns_group_dispatch<false>(cls, max_n, q, stage, grid, s);
 }
 
 bool ns_size_supported(int n) {
@@ -969,24 +1473,44 @@ int ns_one_impl(int which, const NsParams* stages, int nstages, const NsBuffers&
 
 }  // namespace
 
-// Tile shapes of plans whose shapes were not set.  The column kernels want
-// one column per workgroup until the launch fills the chip many times over
-// (a column of 1024 or 512 words is work enough for 256 threads; shorter
-// columns share a workgroup sooner), and never the wide tiles whose
-// registers and LDS leave few workgroups per CU.  us per step spent in the
-// column kernels, W = 1 / 2 / 4 / 8: 1 x 256^2 32 / 42 / 83 / 173, 64 x 256^2
-// 215 / 183 / 220 / 327, 1 x 512^2 46 / 84 / 176 / 336, 64 x 512^2
-// 779 / 690 / 965 / 1537, 16 x 64^2 29 / 29 / 30 / 43, 256 x 64^2
-// 121 / 80 / 67 / 66; in the row kernel, RB = 1 / 2 / 4: 1 x 256^2
-// 21 / 22 / 26, 64 x 256^2 218 / 165 / 154, 64 x 512^2 645 / 530 / 532.
+// Tile shapes of plans whose shapes were not set, from the launch's columns
+// and rows over all instances.  Narrow tiles (W <= kStagedMaxW, the staged
+// kernels) while the launch leaves the chip idle, the register kernels' wider
+// ones beyond.  us per launch of the update-and-inverse kernel, W = 1 / 4 / 8:
+// 1 x 256^2 5.9 / 12.9 / 13.7, 8 x 256^2 9.4 / 13.9 / 14.9, 32 x 256^2
+// 22.0 / 21.1 / 20.7, 64 x 256^2 39 / 31.5 / 30.4; W = 1 / 4: 4 x 512^2
+// 14.7 / 15.7, 8 x 512^2 22.4 / 21.4, 64 x 512^2 139 / 128, 1 x 1024^2
+// 20.6 / 27.9, 8 x 1024^2 97 / 68.  Row kernel, small / large shape: 1 x 256^2
+// 4.3 / 5.9 (RB 1 / 8), 64 x 256^2 50 / 22 (RB 1 / 4), 8 x 512^2 20.6 / 17.9
+// (RB 2 / 8), 32 x 512^2 63 / 49, 8 x 1024^2 86 / 59 (RB 1 / 4).
 int ns_default_tiles(NsParams* q, int n, int count) {
   if (!ns_size_supported(n)) return fail(JCFD_ERR_UNSUPPORTED, "spectral grid size not built");
   const long long rows = static_cast<long long>(n) * count, cols = rows / 2;
-  q->w_cols = n >= 512 ? (cols < 8192 ? 1 : 2)
-              : n == 256 ? (cols < 2048 ? 1 : 2)
-                         : (cols < (n == 32 ? 1024 : 512) ? 1 : cols < (n == 128 ? 4096 : 1024) ? (n == 32 ? 1 : 2)
-                                                                : cols < 8192 || n == 128 ? 4 : 8);
-  q->rb_rows = n >= 512 ? 2 : (rows < 512 ? 1 : (rows < 2048 ? 2 : 4));
+  switch (n) {
+    case 32:
+      q->w_cols = cols < 1024 ? 1 : cols < 4096 ? 4 : 8;
+      q->rb_rows = 8;
+      break;
+    case 64:
+      q->w_cols = cols < 1024 ? 1 : cols < 8192 ? 4 : 8;
+      q->rb_rows = rows < 2048 ? 4 : 16;
+      break;
+    case 128:
+      q->w_cols = cols < 1024 ? 1 : cols < 4096 ? 2 : cols < 8192 ? 4 : 8;
+      q->rb_rows = rows < 1024 ? 2 : rows < 4096 ? 4 : 8;
+      break;
+    case 256:
+      q->w_cols = cols < 2048 ? 1 : cols < 4096 ? 2 : 8;
+      q->rb_rows = rows < 512 ? 1 : rows < 1024 ? 2 : 4;
+      break;
+    case 512:
+      q->w_cols = cols < 2048 ? 1 : 8;
+      q->rb_rows = rows < 4096 ? 2 : 8;
+      break;
+    default:
+      q->w_cols = cols < 2048 ? 1 : 4;
+      q->rb_rows = rows < 2048 ? 1 : 4;
+  }
   q->radix = 8;
   return JCFD_OK;
 }

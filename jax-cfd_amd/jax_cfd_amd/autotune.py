@@ -53,7 +53,7 @@ FVM = Tunables(
              'rows_project': {'fvm_rows_project': 1}})
 NS2D = Tunables(
     'spectral',
-    menu={'cols': (1, 2, 4, 8, 16), 'rows': (1, 2, 4)},
+    menu={'cols': (1, 2, 4, 8, 16), 'rows': (1, 2, 4, 8, 16)},
     weights={'cols': {'ns_cols_inverse': 1, 'ns_cols_update_inverse': 4, 'ns_cols_update': 1},
              'rows': {'ns_rows': 5}})
 FVM_MENU = FVM.menu

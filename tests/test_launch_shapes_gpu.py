@@ -81,3 +81,51 @@ def test_spectral_rule_steps_as_one_column_tiles(n, batch):
     w1 = w.clone()
     other.step_slots(w1, slots, 2)
     assert torch.equal(w1[slots.long()], got[slots.long()])
+
+
+# batches above 2^23 cells run in parts: even and uneven splits, with and
+# without a slot list
+@pytest.mark.parametrize("n,batch", [(256, 128), (256, 129), (512, 33)])
+def test_spectral_batches_in_parts_match_lone_instances(n, batch):
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  spec = serving.SpectralFamily(n, _dev()).spec
+  plan, one = _ns2d.Ns2dPlan(spec, batch, _dev()), _ns2d.Ns2dPlan(spec, 1, _dev())
+  gen = torch.Generator(device=_dev()).manual_seed(batch)
+  w = plan.rfft2(torch.randn((batch, n, n), device=_dev(), generator=gen))
+  got = plan.step(w, 34)  # one direct step, one 32-step graph, one direct step
+  perm = torch.randperm(batch, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(_dev())
+  ws = w.clone()
+  plan.step_slots(ws, perm, 34)
+  assert torch.equal(ws, got)
+  for k in (0, batch // 2 - 1, batch // 2, batch - 1):
+    assert torch.equal(got[k], one.step(w[k].contiguous(), 34)), k
+
+
+# every wavefront layout of the column and row kernels, on instances whose
+# forcing list is longer than the registers hold and reaches column n / 2
+@pytest.mark.parametrize("n", [32, 64, 128, 256, 512, 1024])
+def test_spectral_tiles_with_long_forcing_lists(n):
+  import dataclasses
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  spec = dataclasses.replace(
+      serving.SpectralFamily(n, _dev()).spec,
+      forcing=tuple((p % n, c, 3.0 + p, -1.5 * c) for p, c in
+                    ((0, 4), (n - 4, 0), (n // 2, n // 2), (3, n // 2), (n - 1, n // 2 - 1), (5, 7))))
+  plan = _ns2d.Ns2dPlan(spec, 2, _dev())
+  gen = torch.Generator(device=_dev()).manual_seed(n)
+  w = plan.rfft2(torch.randn((2, n, n), device=_dev(), generator=gen))
+  plan.set_tiles(1, 1, 8)
+  want = plan.step(w, 2)
+  for cols, rows in ((2, 2), (4, 4), (8, 8), (16, 16), (8, 2), (16, 4), (2, 8), (4, 2)):
+    try:
+      plan.set_tiles(cols, rows, 8)
+    except NotImplementedError:
+      continue
+    print(f"n={n} cols={cols} rows={rows}", flush=True)
+    assert torch.equal(plan.step(w, 2), want), (cols, rows)
+  # the forcing list itself: the explicit terms of a zero state are the list
+  f = plan.explicit_terms(torch.zeros_like(w))
+  for p, c, re, im in spec.forcing:
+    assert f[1, p, c].item() == complex(re, im)
