@@ -1236,9 +1236,9 @@ struct jcfd_li_plan {
   int n = 0, batch = 1, device = 0;
   int n_layers = 0, hidden = 0, n_logits = 0;
   int cin[JCFD_LI_MAX_LAYERS] = {}, cout[JCFD_LI_MAX_LAYERS] = {};
-  float* w[JCFD_LI_MAX_LAYERS] = {};  // device, li_conv_weight_layout of [tap][cin (first layer: 4)][cout]
+  uint8_t* w[JCFD_LI_MAX_LAYERS] = {};  // device, li_conv_weight_layout of [tap][cin (first layer: 4)][cout]
   float* b[JCFD_LI_MAX_LAYERS] = {};
-  float* w_logits = nullptr;  // the tower's own output layer, padded to 128 channels
+  uint8_t* w_logits = nullptr;  // the tower's own output layer, padded to 128 channels
   float* b_logits = nullptr;
   bool layer_set[JCFD_LI_MAX_LAYERS] = {};
   bool logits_set = false;
@@ -1311,7 +1311,7 @@ int li_ready(const jcfd_li_plan* p) {
 }
 
 int li_upload_layer(const float* w, const float* b, int cin, int cin_dev, int cout, int cout_dev,
-                    float* wd, float* bd) {
+                    uint8_t* wd, float* bd) {
   // (3, 3, cin, cout) host -> [tap][cin_dev][cout_dev], zero padded, then
   // the kernel's operand order
   std::vector<float> wh(static_cast<size_t>(9) * cin_dev * cout_dev, 0.f), bh(cout_dev, 0.f);
@@ -1325,10 +1325,10 @@ int li_upload_layer(const float* w, const float* b, int cin, int cin_dev, int co
     if (!std::isfinite(x)) return fail(JCFD_ERR_INVALID_ARGUMENT, "weights must be finite");
   for (float x : bh)
     if (!std::isfinite(x)) return fail(JCFD_ERR_INVALID_ARGUMENT, "biases must be finite");
-  std::vector<float> wf(wh.size());
+  std::vector<uint8_t> wf(li_conv_weight_bytes(cin_dev, cout_dev));
   li_conv_weight_layout(wh.data(), cin_dev, cout_dev, wf.data());
   int rc;
-  if ((rc = check_hip(hipMemcpy(wd, wf.data(), wf.size() * sizeof(float), hipMemcpyHostToDevice), "copy weights")))
+  if ((rc = check_hip(hipMemcpy(wd, wf.data(), wf.size(), hipMemcpyHostToDevice), "copy weights")))
     return rc;
   return check_hip(hipMemcpy(bd, bh.data(), bh.size() * sizeof(float), hipMemcpyHostToDevice), "copy biases");
 }
@@ -1397,12 +1397,12 @@ int jcfd_li_plan_create(const jcfd_li_config* config, jcfd_li_plan** plan) {
   const size_t nn = static_cast<size_t>(p->n) * p->n * p->batch;
   for (int k = 0; k < c.n_layers && rc == JCFD_OK; ++k) {
     const int cin_dev = k == 0 ? 4 : p->cin[k];
-    if ((rc = device_alloc(&p->w[k], static_cast<size_t>(9) * cin_dev * p->cout[k], &p->bytes))) break;
+    if ((rc = device_alloc(&p->w[k], li_conv_weight_bytes(cin_dev, p->cout[k]), &p->bytes))) break;
     rc = device_alloc(&p->b[k], static_cast<size_t>(p->cout[k]), &p->bytes);
   }
   const int cin_last = c.n_layers == 1 ? 4 : c.hidden_channels;
   if (rc == JCFD_OK &&
-      ((rc = device_alloc(&p->w_logits, static_cast<size_t>(9) * cin_last * kLiCoefChannels, &p->bytes)) ||
+      ((rc = device_alloc(&p->w_logits, li_conv_weight_bytes(cin_last, kLiCoefChannels), &p->bytes)) ||
        (rc = device_alloc(&p->b_logits, static_cast<size_t>(kLiCoefChannels), &p->bytes)) ||
        (c.n_layers > 1 && (rc = device_alloc(&p->act[0], nn * c.hidden_channels, &p->bytes))) ||
        (c.n_layers > 2 && (rc = device_alloc(&p->act[1], nn * c.hidden_channels, &p->bytes))) ||

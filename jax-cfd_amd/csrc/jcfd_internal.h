@@ -237,7 +237,7 @@ struct LiConvArgs {
   int n;
   const float* in;    // (batch, cin, n, n); the first layer: u (batch, n, n)
   const float* in_v;  // the first layer: v (batch, n, n); otherwise null
-  const float* w;     // MFMA operand order (li_conv_weight_layout)
+  const void* w;      // MFMA operand order (li_conv_weight_layout)
   const float* b;     // [cout]
   float* out;         // (batch, cout, n, n)
 };
@@ -255,9 +255,11 @@ struct LiExplicitArgs {
 };
 bool li_conv_supported(int cin, int cout, bool relu);
 int li_launch_conv(const LiConvArgs& a, int cin, int cout, bool relu, int batch, hipStream_t s);
-// Host: weights [tap = 3 kh + kw][cinp][cout] (cinp = input channels padded
-// to a multiple of 4) -> the device layout li_conv3x3 reads (same size).
-void li_conv_weight_layout(const float* w, int cinp, int cout, float* frag);
+// Host: weights [tap = 3 kh + kw][cinp][cout] (the first layer's 2 input
+// channels padded to 4) -> the device layout the convolution kernels read, of
+// li_conv_weight_bytes bytes (hidden and output layers: three bf16 parts).
+void li_conv_weight_layout(const float* w, int cinp, int cout, void* frag);
+size_t li_conv_weight_bytes(int cinp, int cout);
 int li_launch_explicit(const FvmParams& p, const LiExplicitArgs& a, int batch, hipStream_t s);
 int li_launch_interpolate(int n, const float* coef, const float* x, int key, float* out, int batch,
                           hipStream_t s);

@@ -10,19 +10,19 @@
 // faces with them (4 x 4 patches, layers_util.py:324-447) before
 // advect_general (base/advection.py:34-116).  Here:
 //
-//   li_conv3x3    one periodic 3x3 convolution layer as an implicit GEMM on
-//                 the matrix cores (v_mfma_f32_16x16x4_f32, fp32 in, fp32
-//                 accumulate): D[co][px] = sum over (tap, ci) of
-//                 W[tap][ci][co] * x[ci][px + tap], + bias, relu.  A
-//                 workgroup owns 4 rows x 32 columns of pixels (one row per
-//                 wavefront) and every output channel; the input tile with
+//   li_conv3x3_first, li_conv3x3
+//                 one periodic 3x3 convolution layer as an implicit GEMM on
+//                 the matrix cores, D[co][px] = sum over (tap, ci) of
+//                 W[tap][ci][co] * x[ci][px + tap], + bias, relu, with fp32
+//                 accuracy (the first layer on v_mfma_f32_16x16x4_f32, the
+//                 others on v_mfma_f32_16x16x32_bf16 with three-part
+//                 operands).  A workgroup owns 4 rows x 32 columns of
+//                 pixels and up to 64 output channels; the input tile with
 //                 its one-cell periodic halo goes through LDS in chunks of
-//                 16 channels, double-buffered (the next chunk loaded during
-//                 the current chunk's nine taps).  The weights are stored in
-//                 MFMA operand order, so each wavefront reads its A operands
-//                 straight from global memory (cache-resident: every
-//                 workgroup reads the same few hundred KB), one vector load
-//                 per lane for four k-steps, the next step's loads in flight
+//                 32 channels.  The weights are stored in MFMA operand
+//                 order, so each wavefront reads its A operands straight
+//                 from global memory (cache-resident: every workgroup reads
+//                 the same few hundred KB), the next step's loads in flight
 //                 during the current step's products; one barrier per
 //                 chunk.  The tower's output layer is the
 //                 constraint folded in: its 128 channels are the 8
@@ -41,6 +41,7 @@
 // Activations are planar per instance: (batch, channels, n, n) fp32.
 #include <hip/hip_runtime.h>
 
+#include <cstring>
 #include <type_traits>
 #include <utility>
 
@@ -55,35 +56,13 @@ namespace {
 
 constexpr int kThreads = 256;
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Output tile of a convolution workgroup and its LDS halo tile.
 constexpr int kConvRows = 4;                         // one row per wavefront
 constexpr int kConvCols = 32;                        // two 16-pixel MFMA blocks
 constexpr int kHaloW = kConvCols + 2;
 constexpr int kHaloPlane = (kConvRows + 2) * kHaloW;  // 204 words
-constexpr int kHaloPitch = 208;  // plane pitch: 4 channels of a k-step land 16 banks apart
-
-// Weight layout of a convolution layer in MFMA operand order.  K-steps of 4
-// input channels are grouped KG at a time (one KG-wide vector per lane);
-// fragment (tap, group g, channel block cb) holds, for lane l = i + 16 k
-// (the A[i][k] lane of v_mfma_f32_16x16x4_f32), the KG weights
-// W[tap][ci = 4 (g KG + kk) + k][co = 16 cb + i], kk = 0 .. KG-1, at
-// float offset (((tap GPT + g) NCB + cb) 64 + l) KG + kk.
-template <int CINP, int COUT>
-struct ConvFrag {
-  static constexpr int KS = CINP / 4;         // k-steps
-  static constexpr int KG = KS < 4 ? KS : 4;  // k-steps per weight vector
-  static constexpr int GPT = KS / KG;         // groups per tap
-  static constexpr int NCB = COUT / 16;       // output-channel blocks
-  static constexpr int STEPS = 9 * GPT;       // (tap, group) pairs, tap-major
-};
-template <int KG>
-using ConvAVec = std::conditional_t<KG == 4, float4, float>;
-template <int KG>
-__device__ __forceinline__ float conv_acomp(const ConvAVec<KG>& v, int kk) {
-  if constexpr (KG == 4) return kk == 0 ? v.x : (kk == 1 ? v.y : (kk == 2 ? v.z : v.w));
-  else return v;
-}
 
 // Calls f(integral_constant<int, S>) for S = B .. E-1 (a loop the compiler
 // sees fully unrolled, with compile-time step numbers).
@@ -95,118 +74,61 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// v_mfma_f32_16x16x4_f32 operand layout (checked on gfx950): A[i][k] in lane
-// i + 16 k, B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i / 4),
-// register i % 4.  Here i = output channel, j = pixel, k = input channel.
-//
-// The input channels go in chunks of 4 KG (16 for 16 or more channels):
-// the halo tile of one chunk sits in one of two LDS buffers while the next
-// chunk's tile is loaded into registers, so only the first chunk's load is
-// exposed.  Each chunk runs its 9 taps (step s = 9 chunk + tap, weight
-// fragment tap GPT + chunk); every accumulator therefore sums its products
-// chunk by chunk, tap by tap within a chunk, channels in order within a
-// tap.  The steps are unrolled at compile time so that each weight wait
-// counts exactly the loads issued after it: a chunk's halo loads follow
-// the weight prefetch of its chunk's first step and are waited on two
-// steps later (loads and their waits share one counter, in issue order).
-template <int CINP, int COUT, bool RELU, bool FIRST>
-__global__ __launch_bounds__(kThreads) void li_conv3x3(LiConvArgs a) {
-  static_assert(CINP % 4 == 0 && COUT % 16 == 0, "MFMA blocking");
-  using F = ConvFrag<CINP, COUT>;
-  constexpr int NCB = F::NCB, KG = F::KG, GPT = F::GPT, STEPS = F::STEPS;
-  constexpr int CH = 4 * KG;                  // channels per chunk
-  constexpr int CTOT = CH * kHaloPlane;       // halo words per chunk
-  constexpr int HPT = (CTOT + kThreads - 1) / kThreads;
-  constexpr int NBUF = GPT > 1 ? 2 : 1;
-  using AV = ConvAVec<KG>;
-  __shared__ float shalo[NBUF * CH * kHaloPitch];
+// The first layer (u, v; padded to 4 channels): fp32 products, one k-step of
+// v_mfma_f32_16x16x4_f32 per tap.  Operand layout (checked on gfx950):
+// A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k, D[i][j] in lane
+// j + 16 (i / 4), register i % 4; i = output channel, j = pixel, k = input
+// channel.  Its 36 products per output leave it bound by the stores of its
+// activations, so the products stay as they are.  Weight fragment (tap,
+// channel block cb) holds W[tap][ci = k][co = 16 cb + i] of lane i + 16 k at
+// float offset (tap NCB + cb) 64 + lane.
+constexpr int kFirstPitch = 208;  // plane pitch: the 4 channels of a k-step land 16 banks apart
+template <int COUT, bool RELU>
+__global__ __launch_bounds__(kThreads) void li_conv3x3_first(LiConvArgs a) {
+  constexpr int NCB = COUT / 16;
+  __shared__ float shalo[4 * kFirstPitch];
   const int n = a.n;
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int tiles_x = n / kConvCols;
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int i0 = (t / tiles_x) * kConvRows, j0 = (t % tiles_x) * kConvCols;
   const size_t plane = static_cast<size_t>(n) * n;
-  const size_t inst = blockIdx.y;
-  const float* in = a.in + inst * (FIRST ? 1 : CINP) * plane;
-  const float* in_v = FIRST ? a.in_v + inst * plane : nullptr;
-  // fragment (tap GPT + chunk, cb) of this lane at wf[(fragment * NCB + cb) * 64]
-  const AV* wf = reinterpret_cast<const AV*>(a.w) + lane;
-  auto load = [&](int s, AV (&w)[NCB]) {
-    const int sc = s < STEPS ? s : STEPS - 1;  // unconditional: the last prefetch repeats
-    const int fr = (sc % 9) * GPT + sc / 9;
+  const float* in = a.in + blockIdx.y * plane;
+  const float* in_v = a.in_v + blockIdx.y * plane;
+  const float* wf = static_cast<const float*>(a.w) + lane;
+  float w[9][NCB];
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) w[cb] = wf[(fr * NCB + cb) * 64];
-  };
-  // halo tile of chunk g (rows i0-1 .. i0+4, columns j0-1 .. j0+32,
-  // periodic) through registers
-  float hreg[HPT];
-  auto halo_load = [&](int g) {
+  for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
-    for (int k = 0; k < HPT; ++k) {
-      const int e0 = tid + k * kThreads;
-      const int e = (CTOT % kThreads == 0 || e0 < CTOT) ? e0 : CTOT - 1;
-      const int c = g * CH + e / kHaloPlane, r = (e % kHaloPlane) / kHaloW, cc = e % kHaloW;
-      const size_t gi = static_cast<size_t>((i0 - 1 + r) & (n - 1)) * n + ((j0 - 1 + cc) & (n - 1));
-      if constexpr (FIRST) hreg[k] = c == 0 ? in[gi] : (c == 1 ? in_v[gi] : 0.f);
-      else hreg[k] = in[c * plane + gi];
-    }
-  };
-  auto halo_store = [&](int buf) {
-    float* dst = shalo + buf * CH * kHaloPitch;
-#pragma unroll
-    for (int k = 0; k < HPT; ++k) {
-      const int e = tid + k * kThreads;
-      if (CTOT % kThreads == 0 || e < CTOT) dst[(e / kHaloPlane) * kHaloPitch + e % kHaloPlane] = hreg[k];
-    }
-  };
-  // the first step's weights go out first, then chunk 0's halo
-  AV wa[NCB], wb[NCB];
-  load(0, wa);
-  halo_load(0);
-  halo_store(0);
+    for (int cb = 0; cb < NCB; ++cb) w[tap][cb] = wf[(tap * NCB + cb) * 64];
+  if (tid < kHaloPlane) {
+    const int r = tid / kHaloW, cc = tid % kHaloW;
+    const size_t gi = static_cast<size_t>((i0 - 1 + r) & (n - 1)) * n + ((j0 - 1 + cc) & (n - 1));
+    const float x = in[gi], y = in_v[gi];
+    shalo[tid] = x;
+    shalo[kFirstPitch + tid] = y;
+    shalo[2 * kFirstPitch + tid] = 0.f;
+    shalo[3 * kFirstPitch + tid] = 0.f;
+  }
   __syncthreads();
-
   floatx4 acc[NCB][2];
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) acc[cb][0] = acc[cb][1] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int kq = lane / 16, lp = lane % 16;
-  auto step = [&](int s, const AV (&w)[NCB]) {
-    const int tap = s % 9, g = s / 9;
-    const float* bin = shalo + (g % NBUF) * CH * kHaloPitch + (wave + tap / 3) * kHaloW + tap % 3 + lp;
 #pragma unroll
-    for (int kk = 0; kk < KG; ++kk) {
-      const int ci = kk * 4 + kq;
-      const float b0 = bin[ci * kHaloPitch];
-      const float b1 = bin[ci * kHaloPitch + 16];
+  for (int tap = 0; tap < 9; ++tap) {
+    const float* bin = shalo + kq * kFirstPitch + (wave + tap / 3) * kHaloW + tap % 3 + lp;
+    const float b0 = bin[0], b1 = bin[16];
 #pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) {
-        const float av = conv_acomp<KG>(w[cb], kk);
-        acc[cb][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b0, acc[cb][0], 0, 0, 0);
-        acc[cb][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b1, acc[cb][1], 0, 0, 0);
-      }
+    for (int cb = 0; cb < NCB; ++cb) {
+      acc[cb][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[tap][cb], b0, acc[cb][0], 0, 0, 0);
+      acc[cb][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[tap][cb], b1, acc[cb][1], 0, 0, 0);
     }
-  };
-  // step s computes with one register set while the other receives step
-  // s + 1's weights (the sets alternate, so no copy waits for a load)
-  auto run = [&](auto sc, AV (&cur)[NCB], AV (&nxt)[NCB]) {
-    constexpr int s = decltype(sc)::value;
-    load(s + 1, nxt);
-    if constexpr (s % 9 == 0 && s / 9 + 1 < GPT) halo_load(s / 9 + 1);
-    step(s, cur);
-    if constexpr (s % 9 == 8 && s / 9 + 1 < GPT) {
-      halo_store((s / 9 + 1) % NBUF);  // its buffer's last reader was chunk s/9 - 1
-      __syncthreads();
-    }
-  };
-  static_for<0, STEPS>([&](auto sc) {
-    if constexpr (decltype(sc)::value % 2 == 0) run(sc, wa, wb);
-    else run(sc, wb, wa);
-  });
-
+  }
   // out[co][i0 + wave][j0 + px] = act(acc + b[co])
-  float* out = a.out + inst * COUT * plane + static_cast<size_t>(i0 + wave) * n + j0;
+  float* out = a.out + blockIdx.y * COUT * plane + static_cast<size_t>(i0 + wave) * n + j0;
 #pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) {
+  for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int co = cb * 16 + 4 * kq + r;
@@ -216,6 +138,238 @@ __global__ __launch_bounds__(kThreads) void li_conv3x3(LiConvArgs a) {
         float x = acc[cb][pb][r] + bias;
         if constexpr (RELU) x = fmaxf(x, 0.f);
         out[co * plane + pb * 16 + lp] = x;
+      }
+    }
+}
+
+// Shape of a hidden or output layer: k-steps of 32 (one bf16 MFMA deep), the
+// input channels in chunks of CH.  A k-step is one tap of 32 channels, or,
+// for 16 input channels, two taps (the ninth tap's partner has zero weights).
+template <int CIN, int COUT>
+struct ConvSplit {
+  static constexpr int CH = CIN < 32 ? CIN : 32;      // channels per chunk
+  static constexpr int CHUNKS = CIN / CH;
+  static constexpr int TPS = 32 / CH;                 // taps per k-step
+  static constexpr int SPC = (9 + TPS - 1) / TPS;     // k-steps per chunk
+  static constexpr int STEPS = SPC * CHUNKS;
+  static constexpr int CO = COUT < 64 ? COUT : 64;    // output channels per workgroup
+  static constexpr int CW = CO == 64 ? 2 : 1;         // wavefronts across them
+  static constexpr int PW = 4 / CW;                   // wavefronts across the 128 pixels
+  static constexpr int NCB = CO / 16 / CW;            // 16-channel blocks per wavefront
+  static constexpr int NPB = 8 / PW;                  // 16-pixel blocks per wavefront
+};
+
+// Hidden and output layers.  fp32 products on the bf16 matrix cores: each
+// operand is the exact sum of three bf16 parts, x = x0 + x1 + x2 (each part
+// the rounding of what the ones before it leave; 3 x 8 bits hold fp32's 24),
+// and x w is summed from the six part products of relative size above 2^-25
+// (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0; a bf16 product is exact in
+// fp32), accumulated in fp32.  What is left out, x1 w2 + x2 w1 + x2 w2, is at
+// most 2^-25 of x w, under the fp32 rounding of the sum itself.  Against 64 bits
+// whole towers (n 32 to 256, 16 to 64 channels, 3 and 7 layers, inputs of scale
+// 1 and 1e-3) err 0.29 to 0.60 as much, rms, as with v_mfma_f32_16x16x4_f32
+// products, 0.40 in the mean, because each sum is rounded once per 32 products.
+//
+// What bounds it is the matrix cores: six v_mfma_f32_16x16x32_bf16 (16 cycles
+// each) do the work of eight v_mfma_f32_16x16x4_f32 (32 cycles each).  256^2,
+// 64 -> 64 channels: 50 us (99 of the 154 TFLOP/s a large fp32 product reaches)
+// with fp32 products, 27 us so (1050 TFLOP/s of part products; a large bf16
+// product reaches 1130); 64 -> 128: 94 and 49 us.
+//
+// A workgroup owns 4 rows x 32 columns of pixels and 64 output channels, a
+// wavefront 64 pixels x 32 channels of them: 12 B fragments from LDS and 6 A
+// fragments from global memory (L1/L2-resident, stored in operand order, the
+// next step's in flight) feed 48 MFMA, half the rate either path can give.
+// The pixels' parts sit in LDS as [part][8 channels][pixel][channel], so a
+// fragment read is 16 consecutive 16-byte words per 16 lanes; the split is
+// made once per workgroup, when a chunk of 32 channels is staged, and the
+// second chunk is loaded while the first is used.
+//
+// A value of magnitude 2^127 or more, an infinity or a NaN has no such split
+// (its first part would be infinite): a workgroup that meets one among its
+// inputs sums its outputs again from the fp32 values, one product at a time.
+template <int CIN, int COUT, bool RELU>
+__global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
+  using F = ConvSplit<CIN, COUT>;
+  constexpr int CH = F::CH, NCB = F::NCB, NPB = F::NPB, STEPS = F::STEPS;
+  constexpr int KG = CH / 8;                            // groups of 8 channels per chunk
+  constexpr int ITEMS = KG * kHaloPlane;                // (pixel, group) pairs staged per chunk
+  constexpr int HPT = (ITEMS + kThreads - 1) / kThreads;
+  constexpr int NBUF = F::CHUNKS > 1 ? 2 : 1;
+  constexpr int ZC = COUT / F::CO;
+  __shared__ bf16x8 shalo[NBUF][3][ITEMS];
+  const int n = a.n;
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int tiles_x = n / kConvCols;
+  const int t = xcd_tile(blockIdx.x, gridDim.x) / ZC, z = xcd_tile(blockIdx.x, gridDim.x) % ZC;
+  const int i0 = (t / tiles_x) * kConvRows, j0 = (t % tiles_x) * kConvCols;
+  const size_t plane = static_cast<size_t>(n) * n;
+  const float* in = a.in + blockIdx.y * CIN * plane;
+  const int cw = wave % F::CW, pw = wave / F::CW;
+  const int cb0 = z * (F::CO / 16) + cw * NCB;          // first channel block of this wavefront
+  // fragment (step, channel block, part) at wf[((step COUT/16 + block) 3 + part) 64]
+  const bf16x8* wf = static_cast<const bf16x8*>(a.w) + cb0 * 3 * 64;
+  const unsigned ulane = lane;
+  auto load = [&](int s, bf16x8 (&w)[NCB][3]) {
+    const int sc = s < STEPS ? s : STEPS - 1;  // unconditional: the last prefetch repeats
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[cb][q] = (wf + ((sc * (COUT / 16) + cb) * 3 + q) * 64)[ulane];
+  };
+  // halo tile of chunk g (rows i0-1 .. i0+4, columns j0-1 .. j0+32, periodic)
+  float hreg[HPT][8];
+  bool wild = false;
+  auto halo_load = [&](int g) {
+#pragma unroll
+    for (int k = 0; k < HPT; ++k) {
+      const int e0 = tid + k * kThreads;
+      const int e = e0 < ITEMS ? e0 : ITEMS - 1;
+      const int kg = e / kHaloPlane, px = e % kHaloPlane, r = px / kHaloW, cc = px % kHaloW;
+      const unsigned off = static_cast<unsigned>(kg * 8 * plane) + ((i0 - 1 + r) & (n - 1)) * n + ((j0 - 1 + cc) & (n - 1));
+#pragma unroll
+      for (int c = 0; c < 8; ++c) hreg[k][c] = (in + (g * CH + c) * plane)[off];
+    }
+  };
+  auto halo_store = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < HPT; ++k) {
+      const int e = tid + k * kThreads;
+      bf16x8 p0, p1, p2;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float x = hreg[k][c];
+        wild = wild || !(fabsf(x) < 0x1p127f);
+        const __bf16 x0 = static_cast<__bf16>(x);
+        const float r1 = x - static_cast<float>(x0);
+        const __bf16 x1 = static_cast<__bf16>(r1);
+        p0[c] = x0;
+        p1[c] = x1;
+        p2[c] = static_cast<__bf16>(r1 - static_cast<float>(x1));
+      }
+      if (ITEMS % kThreads == 0 || e < ITEMS) {
+        shalo[buf][0][e] = p0;
+        shalo[buf][1][e] = p1;
+        shalo[buf][2][e] = p2;
+      }
+    }
+  };
+  bf16x8 wa[NCB][3], wb[NCB][3];
+  load(0, wa);
+  halo_load(0);
+  halo_store(0);
+  __syncthreads();
+
+  floatx4 acc[NCB][NPB];
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+    for (int pb = 0; pb < NPB; ++pb) acc[cb][pb] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int kq = lane / 16, lp = lane % 16;
+  // pixel block pb of this wavefront: tile pixel 16 (pw NPB + pb), two to a row
+  auto block_row = [&](int pb) { return (pw * NPB + pb) / 2; };
+  const int kg = kq % KG;
+  const int lbase = kg * kHaloPlane + lp + block_row(0) * kHaloW;
+  auto step = [&](int s, const bf16x8 (&w)[NCB][3]) {
+    const int g = s / F::SPC, t0 = (s % F::SPC) * F::TPS;
+    const int o0 = (t0 / 3) * kHaloW + t0 % 3;
+    int off = lbase + o0;
+    if constexpr (F::TPS == 2) {
+      const int t1 = t0 + 1 < 9 ? t0 + 1 : 8;
+      off = lbase + (kq < 2 ? o0 : (t1 / 3) * kHaloW + t1 % 3);
+    }
+    bf16x8 x[NPB][3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int pb = 0; pb < NPB; ++pb)
+        x[pb][q] = shalo[g % NBUF][q][off + (pb / 2) * kHaloW + (pb % 2) * 16];
+    // The step's six part products, small ones first, in accumulators of
+    // their own, which are then added to the sums: one rounding of each sum
+    // per step (summing all six into it measured 10 % more error).
+    constexpr int PX[6] = {2, 0, 1, 1, 0, 0}, PWT[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+      floatx4 part[NPB];
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int pb = 0; pb < NPB; ++pb)
+          part[pb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              w[cb][PWT[q]], x[pb][PX[q]], q == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : part[pb], 0, 0, 0);
+#pragma unroll
+      for (int pb = 0; pb < NPB; ++pb) {
+        acc[cb][pb] += part[pb];
+        // an empty use: the additions are not moved behind the last step,
+        // which would keep every step's part products until there
+        asm volatile("" : "+v"(acc[cb][pb]));
+      }
+    }
+  };
+  // step s computes with one register set while the other receives step
+  // s + 1's weights (the sets alternate, so no copy waits for a load)
+  auto run = [&](auto sc, bf16x8 (&cur)[NCB][3], bf16x8 (&nxt)[NCB][3]) {
+    constexpr int s = decltype(sc)::value;
+    constexpr int g = s / F::SPC;
+    load(s + 1, nxt);
+    if constexpr (s % F::SPC == 0 && g + 1 < F::CHUNKS) halo_load(g + 1);
+    step(s, cur);
+    if constexpr (s % F::SPC == F::SPC - 1 && g + 1 < F::CHUNKS) {
+      halo_store((g + 1) % NBUF);  // its buffer's last reader was chunk g - 1
+      __syncthreads();
+    }
+  };
+  static_for<0, STEPS>([&](auto sc) {
+    if constexpr (decltype(sc)::value % 2 == 0) run(sc, wa, wb);
+    else run(sc, wb, wa);
+  });
+
+  if (__syncthreads_or(wild)) {
+#pragma unroll 1
+    for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll 1
+      for (int pb = 0; pb < NPB; ++pb)
+#pragma unroll 1
+        for (int r = 0; r < 4; ++r) {
+          const int b = cb0 + cb, i = i0 + (pw * NPB + pb) / 2, j = j0 + (pb % 2) * 16 + lp;
+          float sum = 0.f;
+#pragma unroll 1
+          for (int tap = 0; tap < 9; ++tap)
+#pragma unroll 1
+            for (int ci = 0; ci < CIN; ++ci) {
+              const int s = (ci / CH) * F::SPC + tap / F::TPS, k = (tap % F::TPS) * CH + ci % CH;
+              const __bf16* wp = static_cast<const __bf16*>(a.w) +
+                                 (((s * (COUT / 16) + b) * 3) * 64 + 4 * kq + r + 16 * (k / 8)) * 8 + k % 8;
+              const float w = static_cast<float>(wp[0]) +
+                              (static_cast<float>(wp[512]) + static_cast<float>(wp[1024]));
+              sum = __builtin_fmaf(w, in[ci * plane + static_cast<size_t>((i + tap / 3 - 1) & (n - 1)) * n +
+                                         ((j + tap % 3 - 1) & (n - 1))], sum);
+            }
+          // one element of a register array by a run-time index
+#pragma unroll
+          for (int c2 = 0; c2 < NCB; ++c2)
+#pragma unroll
+            for (int p2 = 0; p2 < NPB; ++p2)
+#pragma unroll
+              for (int r2 = 0; r2 < 4; ++r2)
+                if (c2 == cb && p2 == pb && r2 == r) acc[c2][p2][r2] = sum;
+        }
+  }
+
+  // out[co][i0 + row][j0 + px] = act(acc + b[co])
+  float* out = a.out + blockIdx.y * COUT * plane + static_cast<size_t>(i0) * n + j0;
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int co = (cb0 + cb) * 16 + 4 * kq + r;
+      const float bias = a.b[co];
+#pragma unroll
+      for (int pb = 0; pb < NPB; ++pb) {
+        float x = acc[cb][pb][r] + bias;
+        if constexpr (RELU) x = fmaxf(x, 0.f);
+        out[co * plane + block_row(pb) * n + (pb % 2) * 16 + lp] = x;
       }
     }
   }
@@ -327,23 +481,30 @@ __global__ __launch_bounds__(kThreads) void li_interpolate(const float* __restri
 }
 
 // ---- launchers ------------------------------------------------------------
-template <int CINP, int COUT, bool RELU, bool FIRST>
-int conv_launch(const LiConvArgs& a, int batch, hipStream_t s) {
+template <int COUT, bool RELU>
+int first_launch(const LiConvArgs& a, int batch, hipStream_t s) {
   const dim3 grid((a.n / kConvCols) * (a.n / kConvRows), batch);
-  hipLaunchKernelGGL((li_conv3x3<CINP, COUT, RELU, FIRST>), grid, dim3(kThreads), 0, s, a);
-  return check_hip(hipGetLastError(), "li_conv3x3");
+  hipLaunchKernelGGL((li_conv3x3_first<COUT, RELU>), grid, dim3(kThreads), 0, s, a);
+  return check_hip(hipGetLastError(), "li_conv3x3_first");
 }
 
 template <int COUT>
 int conv_first(const LiConvArgs& a, bool relu, int batch, hipStream_t s) {
-  return relu ? conv_launch<4, COUT, true, true>(a, batch, s) : conv_launch<4, COUT, false, true>(a, batch, s);
+  return relu ? first_launch<COUT, true>(a, batch, s) : first_launch<COUT, false>(a, batch, s);
 }
 
-template <int CINP>
+template <int CIN, int COUT, bool RELU>
+int conv_launch(const LiConvArgs& a, int batch, hipStream_t s) {
+  const dim3 grid((a.n / kConvCols) * (a.n / kConvRows) * (COUT / ConvSplit<CIN, COUT>::CO), batch);
+  hipLaunchKernelGGL((li_conv3x3<CIN, COUT, RELU>), grid, dim3(kThreads), 0, s, a);
+  return check_hip(hipGetLastError(), "li_conv3x3");
+}
+
+template <int CIN>
 int conv_hidden(const LiConvArgs& a, int cout, bool relu, int batch, hipStream_t s) {
-  if (relu && cout == CINP) return conv_launch<CINP, CINP, true, false>(a, batch, s);
-  if (!relu && cout == kLiCoefChannels) return conv_launch<CINP, kLiCoefChannels, false, false>(a, batch, s);
-  return fail(JCFD_ERR_UNSUPPORTED, "convolution " + std::to_string(CINP) + " -> " + std::to_string(cout) +
+  if (relu && cout == CIN) return conv_launch<CIN, CIN, true>(a, batch, s);
+  if (!relu && cout == kLiCoefChannels) return conv_launch<CIN, kLiCoefChannels, false>(a, batch, s);
+  return fail(JCFD_ERR_UNSUPPORTED, "convolution " + std::to_string(CIN) + " -> " + std::to_string(cout) +
                                         (relu ? " (relu)" : "") + " not built");
 }
 
@@ -363,18 +524,55 @@ int interpolate_launch(const float* coef, const float* x, int key, float* out, i
 
 }  // namespace
 
-void li_conv_weight_layout(const float* w, int cinp, int cout, float* frag) {
-  // the ConvFrag layout: k-step groups of up to 4, fragments tap-major
-  const int ks = cinp / 4, kg = ks < 4 ? ks : 4, gpt = ks / kg, ncb = cout / 16;
-  for (int tap = 0; tap < 9; ++tap)
-    for (int g = 0; g < gpt; ++g)
+namespace {
+float from_bf16(uint16_t b) {
+  const uint32_t u = static_cast<uint32_t>(b) << 16;
+  float x;
+  std::memcpy(&x, &u, sizeof(x));
+  return x;
+}
+// Nearest bf16 (ties to even) of a finite x; the largest ones, whose nearest
+// is infinite, are cut off instead.
+uint16_t to_bf16(float x) {
+  uint32_t u;
+  std::memcpy(&u, &x, sizeof(u));
+  const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+  return static_cast<uint16_t>((r & 0x7f80u) == 0x7f80u ? u >> 16 : r);
+}
+}  // namespace
+
+size_t li_conv_weight_bytes(int cinp, int cout) {
+  if (cinp == 4) return static_cast<size_t>(9) * cinp * cout * sizeof(float);
+  const int ch = cinp < 32 ? cinp : 32, tps = 32 / ch;
+  return static_cast<size_t>((9 + tps - 1) / tps) * (cinp / ch) * 32 * cout * 3 * sizeof(uint16_t);
+}
+
+void li_conv_weight_layout(const float* w, int cinp, int cout, void* out) {
+  auto weight = [&](int tap, int ci, int co) { return w[(static_cast<size_t>(tap) * cinp + ci) * cout + co]; };
+  const int ncb = cout / 16;
+  if (cinp == 4) {  // li_conv3x3_first
+    float* frag = static_cast<float*>(out);
+    for (int tap = 0; tap < 9; ++tap)
       for (int cb = 0; cb < ncb; ++cb)
-        for (int l = 0; l < 64; ++l)
-          for (int kk = 0; kk < kg; ++kk) {
-            const int ci = (g * kg + kk) * 4 + l / 16, co = cb * 16 + l % 16;
-            frag[(((static_cast<size_t>(tap) * gpt + g) * ncb + cb) * 64 + l) * kg + kk] =
-                w[(static_cast<size_t>(tap) * cinp + ci) * cout + co];
+        for (int l = 0; l < 64; ++l) frag[(tap * ncb + cb) * 64 + l] = weight(tap, l / 16, cb * 16 + l % 16);
+    return;
+  }
+  // li_conv3x3: fragment (step, channel block, part), lane l, element e is
+  // k = 8 (l / 16) + e of the step, output channel l % 16 of the block
+  uint16_t* frag = static_cast<uint16_t*>(out);
+  const int ch = cinp < 32 ? cinp : 32, tps = 32 / ch, spc = (9 + tps - 1) / tps;
+  for (int s = 0; s < spc * (cinp / ch); ++s)
+    for (int cb = 0; cb < ncb; ++cb)
+      for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e) {
+          const int k = 8 * (l / 16) + e, tap = (s % spc) * tps + k / ch, ci = (s / spc) * ch + k % ch;
+          float x = tap < 9 ? weight(tap, ci, cb * 16 + l % 16) : 0.f;
+          for (int q = 0; q < 3; ++q) {
+            const uint16_t part = to_bf16(x);
+            frag[(((static_cast<size_t>(s) * ncb + cb) * 3 + q) * 64 + l) * 8 + e] = part;
+            x -= from_bf16(part);
           }
+        }
 }
 
 bool li_conv_supported(int cin, int cout, bool relu) {
