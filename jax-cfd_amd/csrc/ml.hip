@@ -398,7 +398,9 @@ __device__ __forceinline__ float li_dot(const float* __restrict__ c, size_t plan
 
 // Explicit terms of the learned self-advection step for rows [i0, i0+RB):
 // k = (-div(aligned_c * aligned_v) + nu lap) + f, per component, with the
-// fluxes of advect_general (advection.py:81-116, _advect_aligned 34-78).
+// fluxes of advect_general (advection.py:81-116, _advect_aligned 34-78), for
+// the components blockIdx.z, blockIdx.z + gridDim.z, ..  The coefficients are
+// what it reads, 512 B per cell; see explicit_launch for the row blocks.
 template <int N, int RB>
 __global__ __launch_bounds__(kThreads) void li_explicit(FvmParams p, LiExplicitArgs a) {
   constexpr int ROWS = RB + 4;  // u, v rows i0-2 .. i0+RB+1
@@ -432,7 +434,7 @@ __global__ __launch_bounds__(kThreads) void li_explicit(FvmParams p, LiExplicitA
     return cval * vval;
   };
 #pragma unroll 1
-  for (int comp = 0; comp < 2; ++comp) {
+  for (int comp = blockIdx.z; comp < 2; comp += gridDim.z) {
     const float* sc = comp == 0 ? su : sv;  // the advected component
     const int* key = a.key + 4 * comp;      // x face: (c, velocity), y face: (c, velocity)
     const float* vx = su;                   // velocity of the x faces: u
@@ -508,10 +510,18 @@ int conv_hidden(const LiConvArgs& a, int cout, bool relu, int batch, hipStream_t
                                         (relu ? " (relu)" : "") + " not built");
 }
 
+// Launches of up to 2^17 cells leave CUs idle in the row blocks that suit
+// larger ones: they take one row (whose x faces a neighbour forms again, from
+// the cached coefficients) and one component per workgroup.  us, several rows
+// and both components / one of each: 256^2 18.0 / 6.1, 64^2 7.0 / 3.8,
+// 8 x 128^2 14.0 / 12.9; 4 x 256^2 24.0 / 26.9, 512^2 28.7 / 30.8.
 template <int N>
 int explicit_launch(const FvmParams& p, const LiExplicitArgs& a, int batch, hipStream_t s) {
   constexpr int RB = N <= 256 ? 4 : 2;
-  hipLaunchKernelGGL((li_explicit<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, p, a);
+  if (static_cast<long long>(N) * N * batch <= 1 << 17)
+    hipLaunchKernelGGL((li_explicit<N, 1>), dim3(N, batch, 2), dim3(kThreads), 0, s, p, a);
+  else
+    hipLaunchKernelGGL((li_explicit<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, p, a);
   return check_hip(hipGetLastError(), "li_explicit");
 }
 

@@ -65,3 +65,16 @@ def test_tower_values_without_a_split(hidden, value):
     ok = torch.isfinite(w)
     if ok.any():
       assert float((g[ok] - w[ok]).abs().max()) <= 1e-5 * float(w[ok].abs().max())
+
+
+def test_explicit_row_blocks_agree():
+  # 9 x 128^2 takes four rows and both components per workgroup, 128^2 one of each
+  n, batch = 128, 9
+  params, v0 = ml._case(n, 16, 1, seed=5)
+  step = ml._model(n, params, 16, 1)[0]
+  u, v = (torch.as_tensor(x.data, device=ml._dev()).repeat(batch, 1, 1) for x in v0)
+  u[3] *= 0.5
+  many, one = step.plan(ml._dev(), batch).step(u, v, 1), step.plan(ml._dev())
+  for b in (0, 3, 8):
+    for got, want in zip(many, one.step(u[b], v[b], 1)):
+      assert torch.equal(got[b], want)
