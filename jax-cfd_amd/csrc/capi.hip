@@ -302,7 +302,7 @@ struct jcfd_fvm_plan {
   float* rhs = nullptr;
   int* status_host = nullptr;  // pinned, 4 ints
   bool tiles_set = false;  // set_tiles pinned the shapes; otherwise each launch's size picks them
-  bool cg_persistent = false;  // one cooperative launch per CG solve (opt-in: slower, see the header)
+  bool cg_persistent = true;  // one cooperative launch per CG solve where the device holds it
   int cg_maxiter = 0;
   int cg_last_iterations = 0;
   // CG implicit diffusion (diffusion == JCFD_DIFFUSION_IMPLICIT_CG), same buffers
@@ -396,6 +396,9 @@ int cg_alloc(jcfd_fvm_plan* p) {
       (rc = device_alloc(&c.part_rr[0], nb, &p->bytes)) ||
       (rc = device_alloc(&c.part_rr[1], nb, &p->bytes)) ||
       (rc = device_alloc(&c.part_pap, nb, &p->bytes)) || (rc = device_alloc(&c.part_bb, nb, &p->bytes)) ||
+      (rc = device_alloc(&c.msg_pap, static_cast<size_t>(cg_sum_messages()), &p->bytes)) ||
+      (rc = device_alloc(&c.msg_rr, static_cast<size_t>(cg_sum_messages()), &p->bytes)) ||
+      (rc = device_alloc(&c.msg_edge, 2 * nb * p->params.n, &p->bytes)) ||
       (rc = device_alloc(&c.status, 4, &p->bytes)))
     return rc;
   if ((rc = check_hip(hipHostMalloc(reinterpret_cast<void**>(&p->status_host), 4 * sizeof(int),
@@ -449,7 +452,7 @@ int cg_persistent_solve(jcfd_fvm_plan* p, float rtol, float atol, int maxiter, b
       (rc = check_hip(hipStreamSynchronize(s), "cg status sync")))
     return rc;
   if (p->status_host[3] || !p->status_host[0])
-    return fail(JCFD_ERR_DEVICE, "persistent CG: a grid barrier timed out");
+    return fail(JCFD_ERR_DEVICE, "persistent CG: a message between workgroups did not arrive");
   *iterations = p->status_host[1];
   return JCFD_OK;
 }
@@ -748,6 +751,8 @@ int jcfd_fvm_plan_destroy(jcfd_fvm_plan* p) {
                     static_cast<void*>(p->cg.ap), static_cast<void*>(p->cg.part_rr[0]),
                     static_cast<void*>(p->cg.part_rr[1]), static_cast<void*>(p->cg.part_pap),
                     static_cast<void*>(p->cg.part_bb), static_cast<void*>(p->cg.status),
+                    static_cast<void*>(p->cg.msg_pap), static_cast<void*>(p->cg.msg_rr),
+                    static_cast<void*>(p->cg.msg_edge),
                     static_cast<void*>(p->rhs)})
     if (ptr != nullptr) (void)hipFree(ptr);
   if (p->status_host) (void)hipHostFree(p->status_host);

@@ -9,9 +9,9 @@
 // periodic 5-point Laplacian of finite_differences.laplacian
 // (finite_differences.py:127-133).
 //
-// Each iteration is two steps over row blocks, as two kernels or, where the
-// device can hold all the row blocks at once, as one cooperative launch for
-// the whole solve with a grid barrier between the steps (cg_persistent):
+// The whole solve is one cooperative launch where the device can hold all the
+// row blocks at once (cg_persistent); otherwise, or where a caller asks for it,
+// each iteration is two kernels over row blocks:
 //   cg_direction  p_k = r_k + beta_k p_{k-1} (rows +-1 halo recomputed in
 //                 LDS), Ap = L p_k, per-block partial <p, Ap>; convergence is
 //                 tested here against the reduced <r_k, r_k>.
@@ -36,25 +36,43 @@ namespace {
 
 constexpr int kThreads = 256;
 
+constexpr int kMaxBlocks = 256;  // row blocks of the largest grids
+constexpr int kMsgCopies = 8;
 constexpr int kWaves = kThreads / 64;
 static_assert(kWaves == 4, "block sums combine four wavefronts");
 
-// Workgroup sums of K values at once: a butterfly across each wavefront's 64
-// lanes (every lane ends with the same bits: each step adds the same two
-// numbers in both lanes of a pair), then the four wavefront sums combined
-// as (w0 + w1) + (w2 + w3).  One barrier pair for all K sums; the order is
-// fixed, so every workgroup gets the same result from the same inputs.
-// red holds K * kWaves floats.
+// Sum over a wavefront's 64 lanes by the butterfly l ^ 32, 16, 8, 4, 2, 1 (every
+// lane ends with the same bits: each step adds the same two numbers in both
+// lanes of a pair).  The exchanges are register moves, not LDS permutes, which
+// take some 100 cycles each in the serial chain of an iteration: lane swaps for
+// 32 and 16, then rotations within rows of 16 lanes and quad permutes (after
+// the step of 8 the values repeat every 8 lanes, so a rotation by 4 is l ^ 4).
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  const int b = __float_as_int(x);
+  return __int_as_float(__builtin_amdgcn_update_dpp(b, b, CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_sum(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  x = x + dpp<0x128>(x);  // rotate by 8
+  x = x + dpp<0x124>(x);  // rotate by 4
+  x = x + dpp<0x4E>(x);   // quad 2 3 0 1
+  return x + dpp<0xB1>(x);  // quad 1 0 3 2
+}
+
+// Workgroup sums of K values at once: each wavefront's sum, then the four
+// wavefront sums combined as (w0 + w1) + (w2 + w3).  One barrier for all K
+// sums; the order is fixed, so every workgroup gets the same result from the
+// same inputs.  red holds K * kWaves floats, which another barrier must
+// separate from their next use.
 template <int K>
 __device__ __forceinline__ void block_sums(float (&v)[K], float* red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int q = 0; q < K; ++q) {
-    float x = v[q];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x = x + __shfl_xor(x, o, 64);
-    v[q] = x;
-  }
+  for (int q = 0; q < K; ++q) v[q] = wave_sum(v[q]);
   if (lane == 0) {
 #pragma unroll
     for (int q = 0; q < K; ++q) red[q * kWaves + wave] = v[q];
@@ -63,7 +81,6 @@ __device__ __forceinline__ void block_sums(float (&v)[K], float* red) {
 #pragma unroll
   for (int q = 0; q < K; ++q)
     v[q] = (red[q * kWaves] + red[q * kWaves + 1]) + (red[q * kWaves + 2] + red[q * kWaves + 3]);
-  __syncthreads();  // red may be written again
 }
 
 __device__ __forceinline__ float block_sum(float v, float* red) {
@@ -76,6 +93,16 @@ __device__ __forceinline__ float tol2(const FvmParams& p, float bs, float rtol, 
   const float a = (rtol * rtol) * bs;
   const float b = atol * atol;
   return a > b ? a : b;
+}
+
+// Word of workgroup b's sum in copy `copy` of the sums (one copy per XCD).
+__device__ __forceinline__ int sum_slot(int copy, int b) { return copy * kMaxBlocks + b; }
+
+// This block's messages of the one-launch solve: none sent yet.
+template <int N>
+__device__ __forceinline__ void clear_messages(const CgBuffers& c) {
+  for (int e = threadIdx.x; e < 2 * N; e += kThreads) c.msg_edge[2 * blockIdx.x * N + e] = 0;
+  if (threadIdx.x < kMsgCopies) c.msg_rr[sum_slot(threadIdx.x, blockIdx.x)] = c.msg_pap[sum_slot(threadIdx.x, blockIdx.x)] = 0;
 }
 
 template <int N, int RB>
@@ -92,14 +119,14 @@ __global__ __launch_bounds__(kThreads) void cg_init(const float* __restrict__ rh
     rr = rr + b * b;
   }
   const float s = block_sum(rr, red);
+  clear_messages<N>(c);
   if (threadIdx.x == 0) {
     c.part_rr[0][blockIdx.x] = s;
     c.part_bb[blockIdx.x] = s;
     if (blockIdx.x == 0) {
       c.status[0] = 0;
       c.status[1] = 0;
-      c.status[2] = 0;  // grid-barrier arrivals of the persistent solve
-      c.status[3] = 0;  // grid-barrier timeout
+      c.status[3] = 0;  // a message of the one-launch solve did not arrive
     }
   }
 }
@@ -132,13 +159,13 @@ __global__ __launch_bounds__(kThreads) void cg_init_helmholtz(FvmParams p, const
     sums[1] = sums[1] + bc * bc;
   }
   block_sums<2>(sums, red);
+  clear_messages<N>(c);
   if (threadIdx.x == 0) {
     c.part_rr[0][blockIdx.x] = sums[0];
     c.part_bb[blockIdx.x] = sums[1];
     if (blockIdx.x == 0) {
       c.status[0] = 0;
       c.status[1] = 0;
-      c.status[2] = 0;
       c.status[3] = 0;
     }
   }
@@ -204,7 +231,7 @@ __device__ __forceinline__ bool direction_body(const FvmParams& p, const CgBuffe
     c.ap[(i0 + r) * N + j] = ap;
     pap = pap + pc * ap;
   }
-  const float s = block_sum(pap, red);
+  const float s = block_sum(pap, red + 3 * kWaves);
   if (threadIdx.x == 0) c.part_pap[blockIdx.x] = s;
   return false;
 }
@@ -212,7 +239,7 @@ __device__ __forceinline__ bool direction_body(const FvmParams& p, const CgBuffe
 template <int N, int RB>
 __global__ __launch_bounds__(kThreads) void cg_direction(FvmParams p, CgBuffers c, int k, float rtol,
                                                          float atol, int maxiter) {
-  __shared__ float red[3 * kWaves];
+  __shared__ float red[4 * kWaves];
   __shared__ float pt[(RB + 2) * N];  // p_k rows i0-1 .. i0+RB
   direction_body<N, RB, false>(p, c, k, rtol, atol, maxiter, 0.f, red, pt);
 }
@@ -221,7 +248,7 @@ template <int N, int RB>
 __global__ __launch_bounds__(kThreads) void cg_direction_helmholtz(FvmParams p, CgBuffers c, int k,
                                                                    float rtol, float atol, int maxiter,
                                                                    float coef) {
-  __shared__ float red[3 * kWaves];
+  __shared__ float red[4 * kWaves];
   __shared__ float pt[(RB + 2) * N];
   direction_body<N, RB, true>(p, c, k, rtol, atol, maxiter, coef, red, pt);
 }
@@ -260,71 +287,196 @@ __device__ __forceinline__ void update_body(const CgBuffers& c, int k, float* re
     c.r[idx] = rn;
     rr = rr + rn * rn;
   }
-  const float s = block_sum(rr, red);
+  const float s = block_sum(rr, red + 2 * kWaves);
   if (threadIdx.x == 0) c.part_rr[(k + 1) & 1][blockIdx.x] = s;
 }
 
 template <int N, int RB>
 __global__ __launch_bounds__(kThreads) void cg_update(CgBuffers c, int k) {
-  __shared__ float red[2 * kWaves];
+  __shared__ float red[3 * kWaves];
   if (c.status[0]) return;
   update_body<N, RB>(c, k, red);
 }
 
-// Polls of a grid barrier before a workgroup gives up (seconds of waiting;
-// a barrier of a healthy launch completes in microseconds).
-constexpr unsigned kBarrierSpinLimit = 1u << 24;
-
-// Grid-wide barrier of a cooperative launch (every workgroup resident at
-// once): the arrival counter grows by one per workgroup and barrier, and the
-// workgroups of barrier number b wait until it reaches target = b *
-// gridDim.x.  The agent-scope release of the arrival and the acquire after
-// the wait make every workgroup's earlier global writes visible to all the
-// others (the caches of every XCD included), as a kernel boundary would.
-// Bounded: a workgroup that polls kBarrierSpinLimit times raises the timeout
-// flag and returns false, so a broken launch ends with an error, not a hang.
-__device__ __forceinline__ bool grid_barrier(unsigned* count, int* timeout, unsigned target, int* s_ok) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int ok = 1;
-    __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    unsigned spins = 0;
-    // wrap-safe: the count may pass 2^32 in very long solves
-    while (static_cast<int>(target - __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) > 0) {
-      __builtin_amdgcn_s_sleep(2);
-      if (++spins > kBarrierSpinLimit) {
-        __hip_atomic_store(timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ok = 0;
-        break;
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    *s_ok = ok;
-  }
-  __syncthreads();
-  return *s_ok != 0;
+// Messages of the one-launch solve: a float and the iteration it belongs to
+// in one 64-bit word, written and read as relaxed agent-scope atomics.  Value
+// and tag arrive together, so a reader that sees the tag has the value and
+// nothing needs a fence: no cache is written back or invalidated.  The tags of
+// a solve are 1, 2, ..; cg_init clears the words.
+__device__ __forceinline__ void send(unsigned long long* m, int tag, float x) {
+  __hip_atomic_store(m, (static_cast<unsigned long long>(static_cast<unsigned>(tag)) << 32) | __float_as_uint(x),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The whole solve in one cooperative launch: the iterations of cg_direction
-// and cg_update with a grid barrier in place of each kernel boundary.  Every
-// workgroup computes the same reduced gamma (same partials, same order), so
-// all of them stop at the same iteration; the per-workgroup arithmetic is
-// that of the two-kernel form, so results are bitwise the same.
+// Polls of a message before a workgroup gives up (seconds of waiting; a
+// message of a healthy launch arrives within microseconds).
+constexpr int kSpinLimit = 1 << 21;
+
+// Waits until all K messages carry `tag`; their values into x.  Bounded: false
+// after kSpinLimit polls, so a broken launch ends with an error, not a hang.
+template <int K>
+__device__ __forceinline__ bool receive(unsigned long long* const (&m)[K], int tag, float (&x)[K]) {
+  for (int spins = 0; spins < kSpinLimit; ++spins) {
+    unsigned long long w[K];
+    bool all = true;
+#pragma unroll
+    for (int q = 0; q < K; ++q) w[q] = __hip_atomic_load(m[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+      all = all && static_cast<unsigned>(w[q] >> 32) == static_cast<unsigned>(tag);
+      x[q] = __uint_as_float(static_cast<unsigned>(w[q]));
+    }
+    if (all) return true;
+  }
+  return false;
+}
+
+// The whole solve in one cooperative launch (every workgroup resident at
+// once).  A workgroup keeps its rows of x, r, p and the rows of r and p beside
+// them in registers; per iteration it exchanges two sums with every other
+// workgroup (<p, Ap>, then <r, r>) and the edge rows of r with its neighbours.
+// Every workgroup adds the same sums in the same order, so all of them stop at
+// the same iteration, and each sum and update has the order of the
+// two-kernel form: results are bitwise the same.
+//
+// One buffer per message suffices: a workgroup sends message k + 1 of a kind
+// only after it has every workgroup's message of the other kind that was
+// sent after they read message k.
+//
+// What bounds it is the way of two messages through memory per iteration,
+// about 1.5 us each.  The words of the sums are read by every workgroup: each
+// is sent in 8 copies, one for the workgroups of each XCD (workgroups go to the
+// XCDs in turn), as the readers of one word wait for each other (us per solve
+// of 468 iterations at 256^2 with 1 / 4 / 8 / 16 / 64 copies: 2255 / 1855 / 1780
+// / 1968 / 2327).  us per solve, two kernels per iteration / one launch: 64^2
+// 946 / 395 (117 iterations), 256^2 3600 / 1780 (468), 512^2 7720 / 4700 (943),
+// 1024^2 22470 / 11370 (1904).  With a counter and fences as grid barrier in
+// place of the messages an iteration took 21.7 us at 256^2.
 template <int N, int RB, bool HELM>
 __global__ __launch_bounds__(kThreads) void cg_persistent(FvmParams p, CgBuffers c, float rtol, float atol,
                                                           int maxiter, float coef) {
-  __shared__ float red[3 * kWaves];
-  __shared__ float pt[(RB + 2) * N];
-  __shared__ int s_ok;
-  unsigned* count = reinterpret_cast<unsigned*>(&c.status[2]);
-  unsigned target = 0;
+  constexpr int NB = N / RB, TOT = RB * N;
+  constexpr int PU = (TOT + kThreads - 1) / kThreads;    // cells per thread
+  constexpr int PH = (2 * N + kThreads - 1) / kThreads;  // neighbour cells per thread: rows i0 - 1 and i0 + RB
+  static_assert(NB <= kThreads && NB <= kMaxBlocks, "one message of each workgroup per thread");
+  __shared__ float red[5 * kWaves];  // one area per sum of an iteration
+  __shared__ float pt[(RB + 2) * N];  // p_k rows i0-1 .. i0+RB
+  __shared__ int s_fail;
+  const int tid = threadIdx.x, blk = blockIdx.x, i0 = blk * RB;
+  // edge rows of block b: first row at 2 b, last row at 2 b + 1 (one row: the first)
+  auto edge = [&](int b, int last, int j) { return c.msg_edge + ((2 * b + (RB > 1 ? last : 0)) * N + j); };
+  float x[PU], rv[PU], pv[PU], av[PU], hr[PH], hp[PH];
+  unsigned long long* from[1 + PH];  // this thread's messages: a workgroup's sum, neighbour cells
+  unsigned long long* pap_from[1] = {c.msg_pap + sum_slot(blk % kMsgCopies, tid < NB ? tid : NB - 1)};
+  from[0] = c.msg_rr + sum_slot(blk % kMsgCopies, tid < NB ? tid : NB - 1);
+#pragma unroll
+  for (int q = 0; q < PU; ++q) {
+    const int e = min(tid + q * kThreads, TOT - 1);
+    x[q] = c.x[i0 * N + e];
+    rv[q] = c.r[i0 * N + e];
+    pv[q] = 0.f;
+    av[q] = 0.f;
+  }
+#pragma unroll
+  for (int q = 0; q < PH; ++q) {
+    const int e = min(tid + q * kThreads, 2 * N - 1), below = e / N, j = e % N;
+    const int gi = (below ? i0 + RB : i0 - 1) & (N - 1);
+    hr[q] = c.r[gi * N + j];
+    hp[q] = 0.f;
+    from[1 + q] = edge((below ? blk + 1 : blk + NB - 1) % NB, !below, j);
+  }
+  if (tid == 0) s_fail = 0;
+  __syncthreads();
+  float gamma = 0.f, gamma_prev = 0.f, limit = 0.f;
+  bool done = false;
   for (int k = 0;; ++k) {
-    if (direction_body<N, RB, HELM>(p, c, k, rtol, atol, maxiter, coef, red, pt)) break;
-    target += gridDim.x;
-    if (!grid_barrier(count, &c.status[3], target, &s_ok)) break;
-    update_body<N, RB>(c, k, red);
-    target += gridDim.x;
-    if (!grid_barrier(count, &c.status[3], target, &s_ok)) break;
+    // gamma_k = <r_k, r_k> (and <b, b>, once)
+    if (k == 0) {
+      float sums[2] = {0.f, 0.f};
+      if (tid < NB) {
+        sums[0] = sums[0] + c.part_rr[0][tid];
+        sums[1] = sums[1] + c.part_bb[tid];
+      }
+      block_sums<2>(sums, red);
+      gamma = sums[0];
+      limit = tol2(p, sums[1], rtol, atol);
+    } else {
+      float in[1 + PH];
+      if (!receive(from, k, in)) s_fail = 1;
+#pragma unroll
+      for (int q = 0; q < PH; ++q) hr[q] = in[1 + q];
+      float sums[1] = {0.f};
+      if (tid < NB) sums[0] = sums[0] + in[0];
+      block_sums<1>(sums, red);
+      if (s_fail) break;
+      gamma = sums[0];
+    }
+    if (!(gamma > limit && k < maxiter)) {
+      done = true;
+      if (blk == 0 && tid == 0) {
+        c.status[0] = 1;
+        c.status[1] = k;
+      }
+      break;
+    }
+    const float beta = (k == 0) ? 0.f : gamma / gamma_prev;
+    gamma_prev = gamma;
+#pragma unroll
+    for (int q = 0; q < PU; ++q) {
+      const int e = tid + q * kThreads;
+      pv[q] = rv[q] + beta * pv[q];
+      if (TOT % kThreads == 0 || e < TOT) pt[N + e] = pv[q];
+    }
+#pragma unroll
+    for (int q = 0; q < PH; ++q) {
+      const int e = tid + q * kThreads;
+      hp[q] = hr[q] + beta * hp[q];
+      if (2 * N % kThreads == 0 || e < 2 * N) pt[(e / N ? (RB + 1) * N : 0) + e % N] = hp[q];
+    }
+    __syncthreads();
+    float pap = 0.f;
+#pragma unroll
+    for (int q = 0; q < PU; ++q) {
+      const int e = tid + q * kThreads;
+      if (TOT % kThreads != 0 && e >= TOT) break;
+      const int j = e % N;
+      const float* row = pt + (e / N + 1) * N;
+      const float pc = row[j];
+      const float lap = lap5(p, pc, row[j - N], row[j + N], row[(j - 1) & (N - 1)], row[(j + 1) & (N - 1)]);
+      av[q] = HELM ? pc - coef * lap : lap;
+      pap = pap + pc * av[q];
+    }
+    const float mine = block_sum(pap, red + 2 * kWaves);
+    if (tid < kMsgCopies) send(c.msg_pap + sum_slot(tid, blk), k + 1, mine);
+    float in[1];
+    if (!receive(pap_from, k + 1, in)) s_fail = 1;
+    float sums[1] = {0.f};
+    if (tid < NB) sums[0] = sums[0] + in[0];
+    block_sums<1>(sums, red + 3 * kWaves);
+    if (s_fail) break;
+    const float alpha = gamma / sums[0];
+    float rr = 0.f;
+#pragma unroll
+    for (int q = 0; q < PU; ++q) {
+      const int e = tid + q * kThreads;
+      if (TOT % kThreads != 0 && e >= TOT) break;
+      x[q] = x[q] + alpha * pv[q];
+      rv[q] = rv[q] - alpha * av[q];
+      rr = rr + rv[q] * rv[q];
+      if (e < N) send(edge(blk, 0, e), k + 1, rv[q]);
+      if (RB > 1 && e >= (RB - 1) * N) send(edge(blk, 1, e - (RB - 1) * N), k + 1, rv[q]);
+    }
+    const float next = block_sum(rr, red + 4 * kWaves);
+    if (tid < kMsgCopies) send(c.msg_rr + sum_slot(tid, blk), k + 1, next);
+  }
+  if (!done) {
+    if (tid == 0) __hip_atomic_store(&c.status[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < PU; ++q) {
+    const int e = tid + q * kThreads;
+    if (TOT % kThreads == 0 || e < TOT) c.x[i0 * N + e] = x[q];
   }
 }
 
@@ -380,7 +532,8 @@ struct CgOps {
 
 }  // namespace
 
-int cg_blocks(int n) { return n >= 512 ? 256 : n; }
+int cg_blocks(int n) { return n >= 512 ? kMaxBlocks : n; }
+int cg_sum_messages() { return kMsgCopies * kMaxBlocks; }
 
 int cg_launch_init(const FvmParams& p, const float* rhs, const CgBuffers& c, float, float, int,
                    hipStream_t s) {

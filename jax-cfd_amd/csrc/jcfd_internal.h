@@ -98,9 +98,14 @@ struct CgBuffers {
   float* part_rr[2];   // per-block partial sums of r.r (by parity)
   float* part_pap;     // per-block partial sums of p.Ap
   float* part_bb;      // per-block partial sums of b.b
-  int* status;         // [0] done flag, [1] iterations run, [2] grid-barrier arrivals, [3] barrier timeout
+  // one-launch solve: 64-bit words of a value and the iteration it belongs to
+  unsigned long long* msg_pap;   // per XCD and block: <p, Ap>
+  unsigned long long* msg_rr;    // per XCD and block: <r, r>
+  unsigned long long* msg_edge;  // per block: first and last row of r
+  int* status;         // [0] done flag, [1] iterations run, [3] a message did not arrive
 };
 int cg_blocks(int n);
+int cg_sum_messages();  // words of msg_pap and of msg_rr
 int cg_launch_init(const FvmParams& p, const float* rhs, const CgBuffers& c, float rtol, float atol,
                    int maxiter, hipStream_t s);
 // The whole solve (after cg_launch_init / cg_launch_init_helmholtz) as one

@@ -113,8 +113,8 @@ class FvmPlan:
                'jcfd_fvm_plan_set_graphs')
 
   def set_cg_persistent(self, enabled: bool):
-    """CG solves as one cooperative launch, or two launches per iteration
-    (default, faster on MI355X); same results."""
+    """CG solves as one cooperative launch (default, where the device holds
+    it), or two launches per iteration; same results."""
     _lib.check(self._lib.jcfd_fvm_plan_set_cg_persistent(self._handle, int(bool(enabled))),
                'jcfd_fvm_plan_set_cg_persistent')
 
