@@ -75,8 +75,7 @@ class Grid:
   @property
   def cell_faces(self) -> Tuple[Tuple[float, ...], ...]:
     d = self.ndim
-    offsets = (np.eye(d) + np.ones([d, d])) / 2.
-    return tuple(tuple(float(o) for o in offset) for offset in offsets)
+    return tuple(tuple(1.0 if i == j else 0.5 for j in range(d)) for i in range(d))
 
   def stagger(self, v):
     return tuple(GridArray(u, o, self) for u, o in zip(v, self.cell_faces))
