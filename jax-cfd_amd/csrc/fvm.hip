@@ -281,12 +281,26 @@ struct MarchLds {
   static constexpr int bytes = vs + N * 4;
 };
 
+// Threads of a marching workgroup: four wavefronts, each thread one cell in 256
+// of a row.  A row of 1024 takes a thread per cell: its ring of 8 rows (64 KB)
+// leaves room for one workgroup per CU, which then has to bring all of the
+// CU's wavefronts itself (1024^2: 15.2 us in 256 workgroups of 4 rows; one row
+// per workgroup with its 6 staged rows, 80 KB of LDS and 8 wavefronts per CU,
+// took 29.4).
+template <int N>
+constexpr int kMarchThreads = N == 1024 ? 1024 : kThreads;
+// Tiles that march: 16 rows and more, and at 1024 4 rows and more, where
+// RB + 5 staged rows with their fluxes would fill the LDS.
+template <int N, int RB>
+constexpr bool kMarches = RB >= 16 || (N == 1024 && RB >= 4);
+
 template <int N, int RB, int R = 8, int CONV = JCFD_CONVECT_VAN_LEER>
 __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, const FvmBuffers& b,
                                                         int i0, int tid, char* smem) {
   using L = MarchLds<N, RB>;
-  constexpr int H = N / 2, K = L::K, FB = L::FB, CPT = N / kThreads;
-  static_assert(N % kThreads == 0 && RB % FB == 0, "march shape");
+  constexpr int NT = kMarchThreads<N>;
+  constexpr int H = N / 2, K = L::K, FB = L::FB, CPT = N / NT;
+  static_assert(N % NT == 0 && RB % FB == 0, "march shape");
   float* su = lds_at<float>(smem, L::su);
   float* sv = lds_at<float>(smem, L::sv);
   float* fy = lds_at<float>(smem, L::fy);
@@ -299,14 +313,14 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
   const RingWindow<N, K> w{su, sv};
   // ring row a holds global row i0 - 3 + a
   auto grow = [&](int a) { return (i0 - 3 + a) & (N - 1); };
-  TwiddleStage<N, 1, kThreads> tsn;
-  TwiddleStage<H, 2, kThreads> tsh;
+  TwiddleStage<N, 1, NT> tsn;
+  TwiddleStage<H, 2, NT> tsh;
   tsn.load(b.tw, tid);
   tsh.load(b.tw, tid);
   float fx_prev[CPT], gx_prev[CPT], us_prev[CPT], fxj[CPT];
 #pragma unroll
-  for (int c = 0; c < CPT; ++c) fxj[c] = p.has_forcing ? b.fx[tid + c * kThreads] : 0.f;
-  staged<5 * N, 8, kThreads>(
+  for (int c = 0; c < CPT; ++c) fxj[c] = p.has_forcing ? b.fx[tid + c * NT] : 0.f;
+  staged<5 * N, 8, NT>(
       tid,
       [&](int e) {
         const int g = grow(e / N) * N + e % N;
@@ -322,7 +336,7 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
   __syncthreads();
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
-    const int j = tid + c * kThreads;
+    const int j = tid + c * NT;
     fx_prev[c] = face_fx_u<CONV>(w, 2, j, p);  // x face below the first u row (i0 - 1)
     gx_prev[c] = face_fx_v<CONV>(w, 3, j, p);  // x face below the first v row (i0)
     us_prev[c] = 0.f;
@@ -337,14 +351,14 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
     if (more) {
 #pragma unroll
       for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * kThreads;
+        const int j = tid + c * NT;
         pu[c] = b.u[grow(a + 3) * N + j];
         pv[c] = b.v[grow(a + 3) * N + j];
       }
     }
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
-      const int j = tid + c * kThreads;
+      const int j = tid + c * NT;
       fy[j] = face_fy_u<CONV>(w, a, j, p);
       if (vrow) gy[j] = face_fy_v<CONV>(w, a, j, p);
     }
@@ -352,7 +366,7 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
     float us_cur[CPT];
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
-      const int j = tid + c * kThreads;
+      const int j = tid + c * NT;
       const int jm = (j - 1) & (N - 1);
       const float fx_next = face_fx_u<CONV>(w, a + 1, j, p);
       const float adv_u = -(over_step(fx_next - fx_prev[c], p.dx, p.rcp_dx) +
@@ -378,7 +392,7 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
       const int d = s - 1;  // div row i0 + d
 #pragma unroll
       for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * kThreads;
+        const int j = tid + c * NT;
         // div u* (finite_differences.py:136-143)
         const float ddx = over_step(us_cur[c] - us_prev[c], p.dx, p.rcp_dx);
         const float ddy = over_step(vs[j] - vs[(j - 1) & (N - 1)], p.dy, p.rcp_dy);
@@ -390,7 +404,7 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
     if (more) {
 #pragma unroll
       for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * kThreads;
+        const int j = tid + c * NT;
         su[((a + 3) & (K - 1)) * N + j] = pu[c];
         sv[((a + 3) & (K - 1)) * N + j] = pv[c];
       }
@@ -398,8 +412,8 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
     __syncthreads();
     if (vrow && (s - 1) % FB == FB - 1) {
       const int d0 = s - FB;  // first div row of this batch
-      lds_fft_waves<H, FB, kThreads, 1, H, false, kRowRadix<N, R>>(zb, twh, tid);
-      for (int e = tid; e < FB * H; e += kThreads) {
+      lds_fft_waves<H, FB, NT, 1, H, false, kRowRadix<N, R>>(zb, twh, tid);
+      for (int e = tid; e < FB * H; e += NT) {
         const int r = e / H, k = e % H;
         b.spec[(i0 + d0 + r) * H + k] = r2c_combine(zb + r * H, k, H, twn[k]);
       }
@@ -420,7 +434,7 @@ __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, cons
   }
 
 template <int N, int RB, int R = 8>
-__global__ __launch_bounds__(kThreads) void fvm_rows_forward_march(FvmParams p, FvmBuffers b) {
+__global__ __launch_bounds__(kMarchThreads<N>) void fvm_rows_forward_march(FvmParams p, FvmBuffers b) {
   __shared__ __align__(16) char smem[MarchLds<N, RB>::bytes];
   const FvmBuffers bi = fvm_instance(b, N);
   const int i0 = xcd_tile(blockIdx.x, gridDim.x) * RB;
@@ -846,13 +860,17 @@ template <> struct Tiles<1024> { static constexpr int RB = 1; };
 //   rows-forward   1 x 256^2  5.5 / 9.6 (RB 1 / 4);   128 x 256^2 116 / 90 / 68 (RB 1 / 4 / 16)
 //                  1 x 512^2  9.5 / 11.0 (RB 1 / 2);   64 x 512^2 277 / 228 / 155 (RB 1 / 2 / 16)
 //                  8 x 256^2  11.6 / 10.9 / 11.9 (RB 1 / 2 / 4)
+//                  1 x 1024^2 29.4 / 15.2 / 23.3 (RB 1 / 4 / 8)
+//                  2 x 1024^2 55.7 / 27.9 / 24.3 (RB 1 / 4 / 8)
+//                  4 x 1024^2 105 / 55.7 / 49.2 / 42.9 (RB 1 / 4 / 8 / 16)
+//                  16 x 1024^2 401 / 180 / 162 / 154 (RB 1 / 8 / 16 / 32)
 //   Poisson cols   1 x 256^2  4.2 / 9.3 (W 1 / 8);     128 x 256^2 45.8 / 23.2 / 22.6 (W 1 / 8 / 4)
 //                  1 x 1024^2 11.2 / 18.9 (W 1 / 4);   16 x 1024^2 75 / 59 (W 1 / 4)
 //   rows-project   1 x 256^2  3.0 / 3.8 (RB 1 / 4);    128 x 256^2 36 / 26 (RB 1 / 4)
 template <int N>
 void auto_tiles(FvmParams* p, int count) {
   const long long R = static_cast<long long>(N) * count, C = R / 2;
-  if (N == 1024) p->rb_fwd = 1;
+  if (N == 1024) p->rb_fwd = R < 2048 ? 4 : (R < 4096 ? 8 : (R < 16384 ? 16 : 32));
   else if ((N == 512 && R >= 8192) || (N == 256 && R >= 12288)) p->rb_fwd = 16;  // marching form
   else if (N <= 128 && R >= 16384) p->rb_fwd = 8;
   else p->rb_fwd = R < 1024 ? 1 : (R < 4096 ? 2 : 4);
@@ -879,11 +897,11 @@ bool one_row(int count) {
 // FFTs' rounding.
 constexpr int kTileLdsMax = 96 * 1024;
 
-// rows_forward tiles 1..8 stage RB + 5 rows at once; 16 and 32 march (n >= 256).
+// rows_forward tiles that do not march stage RB + 5 rows at once.
 template <int N, int RB>
 constexpr bool fwd_ok() {
-  if constexpr (RB >= 16)
-    return N >= kThreads && N <= 512 && RB <= N / 8 && MarchLds<N, RB>::bytes <= kTileLdsMax;
+  if constexpr (kMarches<N, RB>)
+    return N >= kThreads && RB <= N / 8 && MarchLds<N, RB>::bytes <= (N == 1024 ? 112 * 1024 : kTileLdsMax);
   else
     return RB <= N / 4 && RowsForwardLds<N, RB, 0>::bytes <= kTileLdsMax;
 }
@@ -903,8 +921,9 @@ template <int N, int T, int R>
 int launch_variant(int which, const FvmParams& p, const FvmBuffers& b, hipStream_t s) {
   if (which == 0) {
     if constexpr (fwd_ok<N, T>()) {
-      if constexpr (T >= 16)
-        hipLaunchKernelGGL((fvm_rows_forward_march<N, T, R>), dim3(N / T, nb(b)), dim3(kThreads), 0, s, p, b);
+      if constexpr (kMarches<N, T>)
+        hipLaunchKernelGGL((fvm_rows_forward_march<N, T, R>), dim3(N / T, nb(b)), dim3(kMarchThreads<N>), 0, s,
+                           p, b);
       else
         hipLaunchKernelGGL((fvm_rows_forward<N, T, 0, R>), dim3(N / T, nb(b)), dim3(kThreads), 0, s, p, b);
       return JCFD_OK;

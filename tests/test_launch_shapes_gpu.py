@@ -129,3 +129,19 @@ def test_spectral_tiles_with_long_forcing_lists(n):
   f = plan.explicit_terms(torch.zeros_like(w))
   for p, c, re, im in spec.forcing:
     assert f[1, p, c].item() == complex(re, im)
+
+
+# rows of 1024 march with a thread per cell: every tile, scheme and batch
+# against one-row tiles, which stage their rows
+@pytest.mark.parametrize("convect", [0, 1, 2, 3])
+@pytest.mark.parametrize("batch", [1, 2])
+def test_fvm_marching_rows_of_1024(convect, batch):
+  plan, u, v = _fvm(1024, batch, convect=convect)
+  if batch == 1:
+    u, v = u[0], v[0]
+  plan.set_tiles(1, 1, 1, 8)
+  want = plan.step(u, v, 2)
+  for rows in (4, 8, 16, 32):
+    plan.set_tiles(rows, 1, 1, 8)
+    got = plan.step(u, v, 2)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), rows
