@@ -625,7 +625,7 @@ def _fvm_plan_kernel_key(kname, n, batch, tiles):
     march = rb >= (4 if n == 1024 else 16)
     name = (f"fvm_rows_forward_march<{n}, {rb}, {radix}>" if march
             else f"fvm_rows_forward<{n}, {rb}, 0, {radix}>")
-    return f"{name} grid={batch * n // rb * (1024 if march and n == 1024 else 256)}"
+    return f"{name} grid={batch * n // rb * (n if march else 256)}"
   if kname == "fvm_poisson_cols":
     w = tiles["poisson_cols"]
     return f"fvm_poisson_cols<{n}, {w}, {radix}> grid={batch * (n // 2) // w * 256}"

@@ -104,13 +104,12 @@ __device__ __forceinline__ T* lds_at(char* smem, int offset) {
   return reinterpret_cast<T*>(smem + offset);
 }
 
-// The same rows held in a ring of K slots: local row a lives in slot a % K.
-template <int N, int K>
-struct RingWindow {
-  const float* su;
-  const float* sv;
-  __device__ __forceinline__ float U(int a, int j) const { return su[(a & (K - 1)) * N + (j & (N - 1))]; }
-  __device__ __forceinline__ float V(int a, int j) const { return sv[(a & (K - 1)) * N + (j & (N - 1))]; }
+// The cells around one cell held in registers: rows -1 .. 2, columns -1 .. 2
+// relative to it (every index is a compile-time constant after inlining).
+struct CellWindow {
+  float u[4][4], v[4][4];
+  __device__ __forceinline__ float U(int a, int j) const { return u[a + 1][j + 1]; }
+  __device__ __forceinline__ float V(int a, int j) const { return v[a + 1][j + 1]; }
 };
 
 // Face fluxes of the convection term, each evaluated once per face.  With
@@ -260,166 +259,193 @@ struct RowsForwardLds {
 };
 
 // Marching variant of kernel A (full step only), for n >= 256: a workgroup
-// walks RB rows i0-1 .. i0+RB-1 one at a time over a ring of 8 staged rows of
-// u and v (each row read once per workgroup, plus a 4-row halo), fetching
-// the next row into registers while the current row is computed.  x-face
-// fluxes carry over from row to row in registers; y-face fluxes and v* of
-// the current row go through LDS for the column neighbours; div rows collect
-// FB at a time and are transformed together.  Same per-cell arithmetic as
+// walks rows i0-1 .. i0+RB-1 one at a time, each thread keeping the cells
+// around its own (CellWindow) in registers.  Per row it reads one new row of
+// u and v from global memory (the next one in flight during the row's work)
+// and, of that row, its neighbours' columns through LDS.  The y faces of a row
+// are formed one row ahead and the divergence one row behind, so that what
+// the columns exchange -- the new row, y-face fluxes, v* -- is written in one
+// step and read in the next: double-buffered, one barrier per row.  x-face
+// fluxes carry over from row to row in registers; div rows collect FB at a
+// time and are transformed together.  Same per-cell arithmetic as
 // rows_forward_body, so the same results bit for bit.
+//
+// What bounds it is the arithmetic of the four limited faces per cell (some 300
+// instructions, four cycles each).  rows-forward, us, with a ring of 8 rows in
+// LDS (34 LDS reads per cell, three barriers per row) / so: 128 x 256^2 70 / 64,
+// 64 x 512^2 162 / 132, 16 x 1024^2 154 / 149, 1024^2 15.2 / 14.6.
 template <int N, int RB>
 struct MarchLds {
-  static constexpr int H = N / 2, K = 8, FB = 4;
+  static constexpr int H = N / 2, FB = 4;
   static constexpr int twn = 0;                  // float2[N]
   static constexpr int twh = twn + N * 8;        // float2[H]
   static constexpr int zb = twh + H * 8;         // float2[FB * H]: div rows, then FFTs
-  static constexpr int su = zb + FB * H * 8;     // float[K * N]: ring of u rows
-  static constexpr int sv = su + K * N * 4;      // float[K * N]: ring of v rows
-  static constexpr int fy = sv + K * N * 4;      // float[N]: y-face fluxes of u, current row
-  static constexpr int gy = fy + N * 4;          // float[N]: y-face fluxes of v, current row
-  static constexpr int vs = gy + N * 4;          // float[N]: v* of the current row
-  static constexpr int bytes = vs + N * 4;
+  static constexpr int ex = zb + FB * H * 8;     // float[2][5 * N]: exchanged rows, by step parity
+  static constexpr int bytes = ex + 2 * 5 * N * 4;
 };
 
-// Threads of a marching workgroup: four wavefronts, each thread one cell in 256
-// of a row.  A row of 1024 takes a thread per cell: its ring of 8 rows (64 KB)
-// leaves room for one workgroup per CU, which then has to bring all of the
-// CU's wavefronts itself (1024^2: 15.2 us in 256 workgroups of 4 rows; one row
-// per workgroup with its 6 staged rows, 80 KB of LDS and 8 wavefronts per CU,
-// took 29.4).
+// Threads of a marching workgroup: one per cell of a row.
 template <int N>
-constexpr int kMarchThreads = N == 1024 ? 1024 : kThreads;
+constexpr int kMarchThreads = N < kThreads ? kThreads : N;
 // Tiles that march: 16 rows and more, and at 1024 4 rows and more, where
-// RB + 5 staged rows with their fluxes would fill the LDS.
+// RB + 5 staged rows with their fluxes would fill the LDS (1024^2, one row per
+// workgroup with its 6 staged rows, 80 KB of LDS and 8 wavefronts per CU:
+// 29.4 us; marching 15.2).
 template <int N, int RB>
 constexpr bool kMarches = RB >= 16 || (N == 1024 && RB >= 4);
 
-template <int N, int RB, int R = 8, int CONV = JCFD_CONVECT_VAN_LEER>
+template <int N, int RB, int R = 8, int CONV = JCFD_CONVECT_VAN_LEER, int NT = kMarchThreads<N>>
 __device__ __forceinline__ void rows_forward_march_body(const FvmParams& p, const FvmBuffers& b,
                                                         int i0, int tid, char* smem) {
   using L = MarchLds<N, RB>;
-  constexpr int NT = kMarchThreads<N>;
-  constexpr int H = N / 2, K = L::K, FB = L::FB, CPT = N / NT;
+  constexpr int H = N / 2, FB = L::FB, CPT = N / NT;
   static_assert(N % NT == 0 && RB % FB == 0, "march shape");
-  float* su = lds_at<float>(smem, L::su);
-  float* sv = lds_at<float>(smem, L::sv);
-  float* fy = lds_at<float>(smem, L::fy);
-  float* gy = lds_at<float>(smem, L::gy);
-  float* vs = lds_at<float>(smem, L::vs);
   float2* zb = lds_at<float2>(smem, L::zb);
   float* zf = reinterpret_cast<float*>(zb);
   float2* twn = lds_at<float2>(smem, L::twn);
   float2* twh = lds_at<float2>(smem, L::twh);
-  const RingWindow<N, K> w{su, sv};
-  // ring row a holds global row i0 - 3 + a
-  auto grow = [&](int a) { return (i0 - 3 + a) & (N - 1); };
+  // exchanged rows of step parity q: u, v of the window's new row, y-face
+  // fluxes of u and v of the row the step finishes, v* of the row before it
+  auto row_of = [&](int q, int k) { return lds_at<float>(smem, L::ex) + ((q & 1) * 5 + k) * N; };
+  // window row a holds global row i0 - 3 + a
+  auto grow = [&](int a) { return ((i0 - 3 + a) & (N - 1)) * N; };
   TwiddleStage<N, 1, NT> tsn;
   TwiddleStage<H, 2, NT> tsh;
   tsn.load(b.tw, tid);
   tsh.load(b.tw, tid);
-  float fx_prev[CPT], gx_prev[CPT], us_prev[CPT], fxj[CPT];
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) fxj[c] = p.has_forcing ? b.fx[tid + c * NT] : 0.f;
-  staged<5 * N, 8, NT>(
-      tid,
-      [&](int e) {
-        const int g = grow(e / N) * N + e % N;
-        return make_float2(b.u[g], b.v[g]);
-      },
-      [&](int e, float2 x) {
-        const int a = e / N, j = e % N;
-        su[(a & (K - 1)) * N + j] = x.x;
-        sv[(a & (K - 1)) * N + j] = x.y;
-      });
-  tsn.store(twn, tid);
-  tsh.store(twh, tid);
-  __syncthreads();
+  CellWindow w[CPT];
+  float fx_prev[CPT], gx_prev[CPT], fy[CPT], gy[CPT], fxj[CPT], us1[CPT], us2[CPT], vs1[CPT], pu[CPT], pv[CPT];
+  int jm[CPT], jp[CPT], jq[CPT];  // columns j - 1, j + 1, j + 2
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     const int j = tid + c * NT;
-    fx_prev[c] = face_fx_u<CONV>(w, 2, j, p);  // x face below the first u row (i0 - 1)
-    gx_prev[c] = face_fx_v<CONV>(w, 3, j, p);  // x face below the first v row (i0)
-    us_prev[c] = 0.f;
+    jm[c] = (j - 1) & (N - 1);
+    jp[c] = (j + 1) & (N - 1);
+    jq[c] = (j + 2) & (N - 1);
+    fxj[c] = p.has_forcing ? b.fx[j] : 0.f;
+    // rows 0 .. 3: the window of row 1
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* ur = b.u + grow(r);
+      const float* vr = b.v + grow(r);
+      w[c].u[r][0] = ur[jm[c]];
+      w[c].u[r][1] = ur[j];
+      w[c].u[r][2] = ur[jp[c]];
+      w[c].u[r][3] = ur[jq[c]];
+      w[c].v[r][0] = vr[jm[c]];
+      w[c].v[r][1] = vr[j];
+      w[c].v[r][2] = vr[jp[c]];
+      w[c].v[r][3] = vr[jq[c]];
+    }
+    pu[c] = b.u[grow(4) + j];
+    pv[c] = b.v[grow(4) + j];
+    us1[c] = us2[c] = vs1[c] = gx_prev[c] = 0.f;
   }
-  // step s: cells of ring row a = s + 2 (global row i0 - 1 + s); u for every
-  // s, v and div for s >= 1.  Reads ring rows a - 1 .. a + 2.
-  for (int s = 0; s <= RB; ++s) {
-    const int a = s + 2;
-    const bool vrow = s >= 1;
-    const bool more = s < RB;
-    float pu[CPT], pv[CPT];
-    if (more) {
+  tsn.store(twn, tid);
+  tsh.store(twh, tid);
+  // the x face below the first u row (i0 - 1), that row's y faces, and row 4
 #pragma unroll
-      for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * NT;
-        pu[c] = b.u[grow(a + 3) * N + j];
-        pv[c] = b.v[grow(a + 3) * N + j];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      const int j = tid + c * NT;
-      fy[j] = face_fy_u<CONV>(w, a, j, p);
-      if (vrow) gy[j] = face_fy_v<CONV>(w, a, j, p);
-    }
-    __syncthreads();
-    float us_cur[CPT];
+  for (int c = 0; c < CPT; ++c) {
+    const int j = tid + c * NT;
+    fx_prev[c] = face_fx_u<CONV>(w[c], 1, 0, p);
+    fy[c] = face_fy_u<CONV>(w[c], 1, 0, p);
+    gy[c] = 0.f;
+    row_of(0, 0)[j] = pu[c];
+    row_of(0, 1)[j] = pv[c];
+    row_of(0, 2)[j] = fy[c];
+    row_of(0, 3)[j] = 0.f;
+  }
+  // div row i0 + d from v* of parity q, u* of its row (us1) and the one below
+  auto div_row = [&](int d, int q) {
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
-      const int j = tid + c * NT;
-      const int jm = (j - 1) & (N - 1);
-      const float fx_next = face_fx_u<CONV>(w, a + 1, j, p);
-      const float adv_u = -(over_step(fx_next - fx_prev[c], p.dx, p.rcp_dx) +
-                            over_step(fy[j] - fy[jm], p.dy, p.rcp_dy));
-      const float ku = add_diffusion_forcing<false>(w, a, j, p, fxj[c], adv_u);
-      us_cur[c] = w.U(a, j) + p.dt * ku;
-      fx_prev[c] = fx_next;
-      if (vrow) {
-        const float gx_next = face_fx_v<CONV>(w, a + 1, j, p);
-        const float adv_v = -(over_step(gx_next - gx_prev[c], p.dx, p.rcp_dx) +
-                              over_step(gy[j] - gy[jm], p.dy, p.rcp_dy));
-        const float kv = add_diffusion_forcing<true>(w, a, j, p, 0.f, adv_v);
-        const float vst = w.V(a, j) + p.dt * kv;
-        gx_prev[c] = gx_next;
-        vs[j] = vst;
-        const int gi = i0 - 1 + s;
-        b.us[gi * N + j] = us_cur[c];
-        b.vs[gi * N + j] = vst;
-      }
+      // div u* (finite_differences.py:136-143)
+      const float ddx = over_step(us1[c] - us2[c], p.dx, p.rcp_dx);
+      const float ddy = over_step(vs1[c] - row_of(q, 4)[jm[c]], p.dy, p.rcp_dy);
+      zf[(d % FB) * N + tid + c * NT] = ddx + ddy;
     }
-    __syncthreads();  // v* row complete; y-face rows read
-    if (vrow) {
-      const int d = s - 1;  // div row i0 + d
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * NT;
-        // div u* (finite_differences.py:136-143)
-        const float ddx = over_step(us_cur[c] - us_prev[c], p.dx, p.rcp_dx);
-        const float ddy = over_step(vs[j] - vs[(j - 1) & (N - 1)], p.dy, p.rcp_dy);
-        zf[(d % FB) * N + j] = ddx + ddy;
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) us_prev[c] = us_cur[c];
-    if (more) {
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * NT;
-        su[((a + 3) & (K - 1)) * N + j] = pu[c];
-        sv[((a + 3) & (K - 1)) * N + j] = pv[c];
-      }
-    }
-    __syncthreads();
-    if (vrow && (s - 1) % FB == FB - 1) {
-      const int d0 = s - FB;  // first div row of this batch
+    if (d % FB == FB - 1) {
+      __syncthreads();
       lds_fft_waves<H, FB, NT, 1, H, false, kRowRadix<N, R>>(zb, twh, tid);
       for (int e = tid; e < FB * H; e += NT) {
         const int r = e / H, k = e % H;
-        b.spec[(i0 + d0 + r) * H + k] = r2c_combine(zb + r * H, k, H, twn[k]);
+        b.spec[(i0 + d + 1 - FB + r) * H + k] = r2c_combine(zb + r * H, k, H, twn[k]);
       }
-      // zb is written again only after the next step's first barrier
+      // zb is written again only after the next step's barrier
+    }
+  };
+  // step s: cells of window row a = s + 2 (global row i0 - 1 + s); u for every
+  // s, v for s >= 1; div of the row before for s >= 2
+#pragma unroll 1
+  for (int s = 0; s <= RB; ++s) {
+    const int a = s + 2;
+    __syncthreads();  // the rows of parity s are complete, those of s + 1 read
+    float qu[CPT], qv[CPT];
+    if (s < RB) {
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) {
+        qu[c] = b.u[grow(a + 3) + tid + c * NT];
+        qv[c] = b.v[grow(a + 3) + tid + c * NT];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      // the window moves up one row
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          w[c].u[r][k] = w[c].u[r + 1][k];
+          w[c].v[r][k] = w[c].v[r + 1][k];
+        }
+      const float* ur = row_of(s, 0);
+      const float* vr = row_of(s, 1);
+      w[c].u[3][0] = ur[jm[c]];
+      w[c].u[3][1] = pu[c];
+      w[c].u[3][2] = ur[jp[c]];
+      w[c].u[3][3] = ur[jq[c]];
+      w[c].v[3][0] = vr[jm[c]];
+      w[c].v[3][1] = pv[c];
+      w[c].v[3][2] = vr[jp[c]];
+      w[c].v[3][3] = vr[jq[c]];
+    }
+    if (s >= 2) div_row(s - 2, s);
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      const int j = tid + c * NT;
+      const float fx_next = face_fx_u<CONV>(w[c], 1, 0, p);
+      const float adv_u = -(over_step(fx_next - fx_prev[c], p.dx, p.rcp_dx) +
+                            over_step(fy[c] - row_of(s, 2)[jm[c]], p.dy, p.rcp_dy));
+      const float ku = add_diffusion_forcing<false>(w[c], 0, 0, p, fxj[c], adv_u);
+      us2[c] = us1[c];
+      us1[c] = w[c].U(0, 0) + p.dt * ku;
+      fx_prev[c] = fx_next;
+      const float gx_next = face_fx_v<CONV>(w[c], 1, 0, p);
+      if (s >= 1) {
+        const float adv_v = -(over_step(gx_next - gx_prev[c], p.dx, p.rcp_dx) +
+                              over_step(gy[c] - row_of(s, 3)[jm[c]], p.dy, p.rcp_dy));
+        const float kv = add_diffusion_forcing<true>(w[c], 0, 0, p, 0.f, adv_v);
+        vs1[c] = w[c].V(0, 0) + p.dt * kv;
+        const int gi = (i0 - 1 + s) * N + j;
+        b.us[gi] = us1[c];
+        b.vs[gi] = vs1[c];
+        row_of(s + 1, 4)[j] = vs1[c];
+      }
+      gx_prev[c] = gx_next;
+      if (s < RB) {
+        fy[c] = face_fy_u<CONV>(w[c], 1, 0, p);
+        gy[c] = face_fy_v<CONV>(w[c], 1, 0, p);
+        pu[c] = qu[c];
+        pv[c] = qv[c];
+        row_of(s + 1, 0)[j] = pu[c];
+        row_of(s + 1, 1)[j] = pv[c];
+        row_of(s + 1, 2)[j] = fy[c];
+        row_of(s + 1, 3)[j] = gy[c];
+      }
     }
   }
+  __syncthreads();
+  div_row(RB - 1, RB + 1);
 }
 
 // The convection scheme is a template argument of the stencil bodies, chosen
@@ -860,10 +886,10 @@ template <> struct Tiles<1024> { static constexpr int RB = 1; };
 //   rows-forward   1 x 256^2  5.5 / 9.6 (RB 1 / 4);   128 x 256^2 116 / 90 / 68 (RB 1 / 4 / 16)
 //                  1 x 512^2  9.5 / 11.0 (RB 1 / 2);   64 x 512^2 277 / 228 / 155 (RB 1 / 2 / 16)
 //                  8 x 256^2  11.6 / 10.9 / 11.9 (RB 1 / 2 / 4)
-//                  1 x 1024^2 29.4 / 15.2 / 23.3 (RB 1 / 4 / 8)
-//                  2 x 1024^2 55.7 / 27.9 / 24.3 (RB 1 / 4 / 8)
-//                  4 x 1024^2 105 / 55.7 / 49.2 / 42.9 (RB 1 / 4 / 8 / 16)
-//                  16 x 1024^2 401 / 180 / 162 / 154 (RB 1 / 8 / 16 / 32)
+//                  1 x 1024^2 29.4 / 14.6 / 22.5 (RB 1 / 4 / 8)
+//                  2 x 1024^2 55.7 / 22.4 / 23.8 (RB 1 / 4 / 8)
+//                  4 x 1024^2 105 / 40.0 / 44.3 / 40.1 (RB 1 / 4 / 8 / 16)
+//                  16 x 1024^2 400 / 154 / 153 / 149 (RB 1 / 4 / 16 / 32)
 //   Poisson cols   1 x 256^2  4.2 / 9.3 (W 1 / 8);     128 x 256^2 45.8 / 23.2 / 22.6 (W 1 / 8 / 4)
 //                  1 x 1024^2 11.2 / 18.9 (W 1 / 4);   16 x 1024^2 75 / 59 (W 1 / 4)
 //   rows-project   1 x 256^2  3.0 / 3.8 (RB 1 / 4);    128 x 256^2 36 / 26 (RB 1 / 4)
@@ -901,7 +927,7 @@ constexpr int kTileLdsMax = 96 * 1024;
 template <int N, int RB>
 constexpr bool fwd_ok() {
   if constexpr (kMarches<N, RB>)
-    return N >= kThreads && RB <= N / 8 && MarchLds<N, RB>::bytes <= (N == 1024 ? 112 * 1024 : kTileLdsMax);
+    return N >= kThreads && RB <= N / 8 && MarchLds<N, RB>::bytes <= kTileLdsMax;
   else
     return RB <= N / 4 && RowsForwardLds<N, RB, 0>::bytes <= kTileLdsMax;
 }
@@ -1186,7 +1212,7 @@ __device__ __forceinline__ void group_tile(const FvmGroupDesc& d, int tile, int 
   if constexpr (PHASE == 0) {
     const FvmParams& p = d.p;
     if constexpr (G::kMarch) {
-#define JCFD_GMARCH(C) rows_forward_march_body<N, G::RB_FWD, 8, C>(d.p, d.b, tile * G::RB_FWD, tid, smem)
+#define JCFD_GMARCH(C) rows_forward_march_body<N, G::RB_FWD, 8, C, kThreads>(d.p, d.b, tile * G::RB_FWD, tid, smem)
       JCFD_CONVECT_DISPATCH(JCFD_GMARCH)
 #undef JCFD_GMARCH
     } else {
