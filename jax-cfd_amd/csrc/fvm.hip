@@ -43,8 +43,6 @@ namespace {
 
 constexpr int kThreads = 256;
 
-__device__ __forceinline__ float sgnf(float x) { return (x > 0.f) ? 1.f : ((x < 0.f) ? -1.f : x); }
-
 // Radix schedule of the packed row transforms (length n/2).  A row kernel
 // transforms a handful of rows per workgroup (4 per marching batch, RB or
 // RB + 1 per row tile), often one per wavefront: radix-8 passes then keep
@@ -55,16 +53,37 @@ __device__ __forceinline__ float sgnf(float x) { return (x > 0.f) ? 1.f : ((x < 
 template <int N, int R>
 constexpr int kRowRadix = (R == 8 && N <= 512) ? 4 : R;
 
+// x / d for normal d up to 2^126 and |x| <= d: one Newton step makes
+// v_rcp_f32 (1 ulp) the rounded reciprocal, and one remainder step then the
+// rounded quotient (Markstein's theorem, as over_step): 5 instructions and the
+// reciprocal, where the IEEE sequence with its scaling takes 11 and the
+// reciprocal.  Below |x| = 2^-100 the remainder underflows and the result is
+// within an ulp; above d = 2^126 the reciprocal is flushed and the result 0.
+__device__ __forceinline__ float ratio(float x, float d) {
+  const float r0 = __builtin_amdgcn_rcpf(d);
+  const float r = __builtin_fmaf(__builtin_fmaf(-d, r0, 1.f), r0, r0);
+  const float q = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
+}
+
+// 0.5 a + 0.5 b: the halves are exact, so a fused sum rounds like the plain one.
+__device__ __forceinline__ float mean2(float a, float b) { return __builtin_fmaf(0.5f, b, 0.5f * a); }
+
 // Van Leer flux correction (advection.py:284-334 for one face):
 // pre = 0.5 (1 - (dt/h)|U|)|U|;  phi = num (sgn den + sgn num) den / D,
-// D = |den| + |num| if |den| > 0 else 1.
+// D = |den| + |num| if |den| > 0 else 1.  The marching stencil is bound by
+// these instructions (some 300 per cell, four cycles each), so:
+//   - D is the larger of |den| + |num| and the smallest normal number: at den =
+//     0 the quotient is 0 either way;
+//   - num (sgn den + sgn num) is 2 t with t = +-num, den's sign folded in,
+//     where t is positive (the signs agree), else 0 t, which keeps the NaN of
+//     an infinity: five instructions where two signs took ten.
 __device__ __forceinline__ float vl_correction(float U, float num_pos, float num_neg, float den,
                                                float dt_over_h) {
   const float num = (U > 0.f) ? num_pos : num_neg;
-  const float aden = fabsf(den);
-  const float dnn = (aden > 0.f) ? (aden + fabsf(num)) : 1.0f;
-  const float inv = den / dnn;
-  const float phi = (num * (sgnf(den) + sgnf(num))) * inv;
+  const float inv = ratio(den, fmaxf(fabsf(den) + fabsf(num), 0x1p-126f));
+  const float t = __uint_as_float(__float_as_uint(num) ^ (__float_as_uint(den) & 0x80000000u));
+  const float phi = (t * ((t <= 0.f) ? 0.f : 2.f)) * inv;
   const float av = fabsf(U);
   const float pre = (0.5f * (1.f - dt_over_h * av)) * av;
   return pre * phi;
@@ -128,19 +147,19 @@ template <int CONV, typename WIN>
 __device__ __forceinline__ float face_fx_u(const WIN& w, int a, int j, const FvmParams& p) {
   const float h = p.dt_over_dx;
   if constexpr (CONV == JCFD_CONVECT_LINEAR) {  // u and its velocity both at the face
-    const float Uf = 0.5f * w.U(a - 1, j) + 0.5f * w.U(a, j);
+    const float Uf = mean2(w.U(a - 1, j), w.U(a, j));
     return Uf * Uf;
   }
   if constexpr (CONV == JCFD_CONVECT_UPWIND) {  // upwind u times the face velocity
-    const float Uf = 0.5f * w.U(a - 1, j) + 0.5f * w.U(a, j);
+    const float Uf = mean2(w.U(a - 1, j), w.U(a, j));
     return ((Uf > 0.f) ? w.U(a - 1, j) : w.U(a, j)) * Uf;
   }
   if constexpr (CONV == JCFD_CONVECT_VAN_LEER_LIMITERS) {
     const int c = a - 1;  // face between rows c and c + 1
-    const float Uf = 0.5f * w.U(c, j) + 0.5f * w.U(c + 1, j);
+    const float Uf = mean2(w.U(c, j), w.U(c + 1, j));
     return vll_flux(w.U(c - 1, j), w.U(c, j), w.U(c + 1, j), w.U(c + 2, j), Uf, h);
   }
-  const float Uf = 0.5f * w.U(a - 1, j) + 0.5f * w.U(a, j);
+  const float Uf = mean2(w.U(a - 1, j), w.U(a, j));
   return vl_flux(Uf, w.U(a - 1, j), w.U(a, j), w.U(a - 2, j), w.U(a - 1, j), w.U(a, j), w.U(a + 1, j), h);
 }
 
@@ -148,20 +167,20 @@ template <int CONV, typename WIN>
 __device__ __forceinline__ float face_fy_u(const WIN& w, int lr, int b, const FvmParams& p) {
   const float h = p.dt_over_dy;
   if constexpr (CONV == JCFD_CONVECT_LINEAR) {  // (u at the face) * (v at the face)
-    const float cf = 0.5f * w.U(lr, b) + 0.5f * w.U(lr, b + 1);
-    const float Vf = 0.5f * w.V(lr, b) + 0.5f * w.V(lr + 1, b);
+    const float cf = mean2(w.U(lr, b), w.U(lr, b + 1));
+    const float Vf = mean2(w.V(lr, b), w.V(lr + 1, b));
     return cf * Vf;
   }
   if constexpr (CONV == JCFD_CONVECT_UPWIND) {
-    const float Vf = 0.5f * w.V(lr, b) + 0.5f * w.V(lr + 1, b);
+    const float Vf = mean2(w.V(lr, b), w.V(lr + 1, b));
     return ((Vf > 0.f) ? w.U(lr, b) : w.U(lr, b + 1)) * Vf;
   }
   if constexpr (CONV == JCFD_CONVECT_VAN_LEER_LIMITERS) {
-    const float Vf = 0.5f * w.V(lr, b) + 0.5f * w.V(lr + 1, b);
+    const float Vf = mean2(w.V(lr, b), w.V(lr + 1, b));
     return vll_flux(w.U(lr, b - 1), w.U(lr, b), w.U(lr, b + 1), w.U(lr, b + 2), Vf, h);
   }
   const int a = lr + 1;
-  const float Vf = 0.5f * w.V(a - 1, b) + 0.5f * w.V(a, b);
+  const float Vf = mean2(w.V(a - 1, b), w.V(a, b));
   return vl_flux(Vf, w.U(a - 1, b), w.U(a - 1, b + 1), w.U(a, b - 1), w.U(a, b), w.U(a, b + 1),
                  w.U(a, b + 2), h);
 }
@@ -171,20 +190,20 @@ __device__ __forceinline__ float face_fx_v(const WIN& w, int a, int j, const Fvm
   const float h = p.dt_over_dx;
   const int c = a - 1;
   if constexpr (CONV == JCFD_CONVECT_LINEAR) {  // (v at the face) * (u at the face)
-    const float cf = 0.5f * w.V(c, j) + 0.5f * w.V(c + 1, j);
-    const float Uf = 0.5f * w.U(c, j) + 0.5f * w.U(c, j + 1);
+    const float cf = mean2(w.V(c, j), w.V(c + 1, j));
+    const float Uf = mean2(w.U(c, j), w.U(c, j + 1));
     return cf * Uf;
   }
   if constexpr (CONV == JCFD_CONVECT_UPWIND) {
-    const float Uf = 0.5f * w.U(c, j) + 0.5f * w.U(c, j + 1);
+    const float Uf = mean2(w.U(c, j), w.U(c, j + 1));
     return ((Uf > 0.f) ? w.V(c, j) : w.V(c + 1, j)) * Uf;
   }
   if constexpr (CONV == JCFD_CONVECT_VAN_LEER_LIMITERS) {
-    const float Uf = 0.5f * w.U(c, j) + 0.5f * w.U(c, j + 1);
+    const float Uf = mean2(w.U(c, j), w.U(c, j + 1));
     return vll_flux(w.V(c - 1, j), w.V(c, j), w.V(c + 1, j), w.V(c + 2, j), Uf, h);
   }
   const int b = j + 1;
-  const float Uf = 0.5f * w.U(c, b - 1) + 0.5f * w.U(c, b);
+  const float Uf = mean2(w.U(c, b - 1), w.U(c, b));
   return vl_flux(Uf, w.V(c, b - 1), w.V(c + 1, b - 1), w.V(c - 1, b), w.V(c, b), w.V(c + 1, b),
                  w.V(c + 2, b), h);
 }
@@ -193,19 +212,19 @@ template <int CONV, typename WIN>
 __device__ __forceinline__ float face_fy_v(const WIN& w, int lr, int j, const FvmParams& p) {
   const float h = p.dt_over_dy;
   if constexpr (CONV == JCFD_CONVECT_LINEAR) {  // v and its velocity both at the face
-    const float Vf = 0.5f * w.V(lr, j) + 0.5f * w.V(lr, j + 1);
+    const float Vf = mean2(w.V(lr, j), w.V(lr, j + 1));
     return Vf * Vf;
   }
   if constexpr (CONV == JCFD_CONVECT_UPWIND) {
-    const float Vf = 0.5f * w.V(lr, j) + 0.5f * w.V(lr, j + 1);
+    const float Vf = mean2(w.V(lr, j), w.V(lr, j + 1));
     return ((Vf > 0.f) ? w.V(lr, j) : w.V(lr, j + 1)) * Vf;
   }
   if constexpr (CONV == JCFD_CONVECT_VAN_LEER_LIMITERS) {
-    const float Vf = 0.5f * w.V(lr, j) + 0.5f * w.V(lr, j + 1);
+    const float Vf = mean2(w.V(lr, j), w.V(lr, j + 1));
     return vll_flux(w.V(lr, j - 1), w.V(lr, j), w.V(lr, j + 1), w.V(lr, j + 2), Vf, h);
   }
   const int b = j + 1;
-  const float Vf = 0.5f * w.V(lr, b - 1) + 0.5f * w.V(lr, b);
+  const float Vf = mean2(w.V(lr, b - 1), w.V(lr, b));
   return vl_flux(Vf, w.V(lr, b - 1), w.V(lr, b), w.V(lr, b - 2), w.V(lr, b - 1), w.V(lr, b),
                  w.V(lr, b + 1), h);
 }
@@ -270,10 +289,11 @@ struct RowsForwardLds {
 // time and are transformed together.  Same per-cell arithmetic as
 // rows_forward_body, so the same results bit for bit.
 //
-// What bounds it is the arithmetic of the four limited faces per cell (some 300
+// What bounds it is the arithmetic of the four limited faces per cell (some 250
 // instructions, four cycles each).  rows-forward, us, with a ring of 8 rows in
-// LDS (34 LDS reads per cell, three barriers per row) / so: 128 x 256^2 70 / 64,
-// 64 x 512^2 162 / 132, 16 x 1024^2 154 / 149, 1024^2 15.2 / 14.6.
+// LDS (34 LDS reads per cell, three barriers per row) / so / with the shorter
+// limiter of vl_correction: 128 x 256^2 70 / 64 / 56, 64 x 512^2 162 / 132 / 115,
+// 16 x 1024^2 154 / 149 / 127, 1024^2 15.2 / 14.6 / 13.0.
 template <int N, int RB>
 struct MarchLds {
   static constexpr int H = N / 2, FB = 4;
@@ -883,21 +903,21 @@ template <> struct Tiles<1024> { static constexpr int RB = 1; };
 // R = rows and C = packed spectrum columns over all instances.  us per launch,
 // small shape / fixed default (RB 4, 4, 4, 2, 1 for 64..1024; W 8, 8, 8, 8, 4)
 // / largest-useful shape:
-//   rows-forward   1 x 256^2  5.5 / 9.6 (RB 1 / 4);   128 x 256^2 116 / 90 / 68 (RB 1 / 4 / 16)
-//                  1 x 512^2  9.5 / 11.0 (RB 1 / 2);   64 x 512^2 277 / 228 / 155 (RB 1 / 2 / 16)
-//                  8 x 256^2  11.6 / 10.9 / 11.9 (RB 1 / 2 / 4)
-//                  1 x 1024^2 29.4 / 14.6 / 22.5 (RB 1 / 4 / 8)
-//                  2 x 1024^2 55.7 / 22.4 / 23.8 (RB 1 / 4 / 8)
-//                  4 x 1024^2 105 / 40.0 / 44.3 / 40.1 (RB 1 / 4 / 8 / 16)
-//                  16 x 1024^2 400 / 154 / 153 / 149 (RB 1 / 4 / 16 / 32)
+//   rows-forward   1 x 256^2  5.5 / 9.6 (RB 1 / 4);   128 x 256^2 102 / 80 / 56 (RB 1 / 4 / 16)
+//                  8 x 256^2  10.6 / 10.0 / 10.5 (RB 1 / 2 / 4)
+//                  24 x 256^2 21.3 / 22.1, 32 x 256^2 26.3 / 22.2 (RB 4 / 16)
+//                  1 x 512^2  9.5 / 11.0 (RB 1 / 2);   64 x 512^2 247 / 237 / 115 (RB 1 / 4 / 16)
+//                  4 x 512^2  18.7 / 22.8, 8 x 512^2 32.8 / 23.5 (RB 4 / 16)
+//                  1 x 1024^2 27.0 / 13.0 / 19.8 (RB 1 / 4 / 8)
+//                  16 x 1024^2 364 / 133 / 133 / 127 (RB 1 / 4 / 16 / 32)
 //   Poisson cols   1 x 256^2  4.2 / 9.3 (W 1 / 8);     128 x 256^2 45.8 / 23.2 / 22.6 (W 1 / 8 / 4)
 //                  1 x 1024^2 11.2 / 18.9 (W 1 / 4);   16 x 1024^2 75 / 59 (W 1 / 4)
 //   rows-project   1 x 256^2  3.0 / 3.8 (RB 1 / 4);    128 x 256^2 36 / 26 (RB 1 / 4)
 template <int N>
 void auto_tiles(FvmParams* p, int count) {
   const long long R = static_cast<long long>(N) * count, C = R / 2;
-  if (N == 1024) p->rb_fwd = R < 2048 ? 4 : (R < 4096 ? 8 : (R < 16384 ? 16 : 32));
-  else if ((N == 512 && R >= 8192) || (N == 256 && R >= 12288)) p->rb_fwd = 16;  // marching form
+  if (N == 1024) p->rb_fwd = R < 16384 ? 4 : 32;
+  else if ((N == 512 && R >= 4096) || (N == 256 && R >= 8192)) p->rb_fwd = 16;  // marching form
   else if (N <= 128 && R >= 16384) p->rb_fwd = 8;
   else p->rb_fwd = R < 1024 ? 1 : (R < 4096 ? 2 : 4);
   int w = 1;
