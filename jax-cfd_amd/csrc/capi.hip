@@ -440,8 +440,10 @@ int cg_iterate(jcfd_fvm_plan* p, int maxiter, int first, int* iterations, hipStr
 
 // The solve as one cooperative launch (cg_launch_persistent) when enabled
 // and the device holds it: reads the status once at the end.  Returns
-// JCFD_ERR_UNSUPPORTED, with nothing launched, when the caller should run
-// the chunked two-kernel form instead.
+// JCFD_ERR_UNSUPPORTED when the caller should run the chunked two-kernel form
+// instead, from a new cg_init: nothing was launched, or a workgroup gave up
+// waiting for another's message (the launch had to share the GPU with other
+// processes' such launches, and not all of its workgroups ran).
 int cg_persistent_solve(jcfd_fvm_plan* p, float rtol, float atol, int maxiter, bool helm, float coef,
                         int* iterations, hipStream_t s) {
   if (!p->cg_persistent) return JCFD_ERR_UNSUPPORTED;
@@ -451,8 +453,7 @@ int cg_persistent_solve(jcfd_fvm_plan* p, float rtol, float atol, int maxiter, b
                                      s), "cg status")) ||
       (rc = check_hip(hipStreamSynchronize(s), "cg status sync")))
     return rc;
-  if (p->status_host[3] || !p->status_host[0])
-    return fail(JCFD_ERR_DEVICE, "persistent CG: a message between workgroups did not arrive");
+  if (p->status_host[3] || !p->status_host[0]) return JCFD_ERR_UNSUPPORTED;
   *iterations = p->status_host[1];
   return JCFD_OK;
 }
@@ -464,6 +465,8 @@ int cg_solve(jcfd_fvm_plan* p, hipStream_t s) {
   if (rc) return rc;
   rc = cg_persistent_solve(p, rtol, atol, p->cg_maxiter, false, 0.f, &p->cg_last_iterations, s);
   if (rc != JCFD_ERR_UNSUPPORTED) return rc;
+  if (p->cg_persistent && (rc = cg_launch_init(p->params, p->rhs, p->cg, rtol, atol, p->cg_maxiter, s)))
+    return rc;
   return cg_iterate(p, p->cg_maxiter, kCgChunk, &p->cg_last_iterations, s, [&](int k, hipStream_t st) {
     return cg_launch_iteration(p->params, p->cg, k, rtol, atol, p->cg_maxiter, st);
   });
@@ -484,7 +487,9 @@ int cg_diffuse(jcfd_fvm_plan* p, float* u, float* v, hipStream_t s) {
     if (rc == JCFD_OK) {
       rc = cg_persistent_solve(p, rtol, atol, p->diff_maxiter, true, p->diff_coef,
                                &p->diff_last_iterations[m], s);
-      if (rc == JCFD_ERR_UNSUPPORTED)
+      if (rc == JCFD_ERR_UNSUPPORTED &&
+          (rc = p->cg_persistent ? cg_launch_init_helmholtz(p->params, comps[m], p->cg, p->diff_coef, s)
+                                 : JCFD_OK) == JCFD_OK)
         rc = cg_iterate(p, p->diff_maxiter, kDiffusionFirstChunk, &p->diff_last_iterations[m], s,
                         [&](int k, hipStream_t st) {
                           return cg_launch_iteration_helmholtz(p->params, p->cg, k, rtol, atol,

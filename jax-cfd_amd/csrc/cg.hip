@@ -308,12 +308,12 @@ __device__ __forceinline__ void send(unsigned long long* m, int tag, float x) {
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Polls of a message before a workgroup gives up (seconds of waiting; a
+// Polls of a message before a workgroup gives up (about a second of waiting; a
 // message of a healthy launch arrives within microseconds).
-constexpr int kSpinLimit = 1 << 21;
+constexpr int kSpinLimit = 1 << 20;
 
 // Waits until all K messages carry `tag`; their values into x.  Bounded: false
-// after kSpinLimit polls, so a broken launch ends with an error, not a hang.
+// after kSpinLimit polls, so a launch whose workgroups do not all run ends.
 template <int K>
 __device__ __forceinline__ bool receive(unsigned long long* const (&m)[K], int tag, float (&x)[K]) {
   for (int spins = 0; spins < kSpinLimit; ++spins) {
