@@ -53,12 +53,16 @@ constexpr int kThreads = 256;
 template <int N, int R>
 constexpr int kRowRadix = (R == 8 && N <= 512) ? 4 : R;
 
-// x / d for normal d up to 2^126 and |x| <= d: one Newton step makes
-// v_rcp_f32 (1 ulp) the rounded reciprocal, and one remainder step then the
-// rounded quotient (Markstein's theorem, as over_step): 5 instructions and the
+// x / d for normal d up to 2^126 and |x| <= d: 5 instructions and the
 // reciprocal, where the IEEE sequence with its scaling takes 11 and the
-// reciprocal.  Below |x| = 2^-100 the remainder underflows and the result is
-// within an ulp; above d = 2^126 the reciprocal is flushed and the result 0.
+// reciprocal.  v_rcp_f32 (1 ulp), after one Newton step, is the rounded
+// reciprocal for all but 33 (divisor, estimate) pairs of a binade, and the
+// remainder step then gives the rounded quotient (Markstein's theorem, as
+// over_step), for those pairs too but for the divisor of 24 one bits with an
+// estimate beside the rounded one; v_rcp_f32 rounds that one correctly (gfx950:
+// every divisor significand with 64 dividends, and every dividend of that
+// divisor, equal x / d).  Below |x| = 2^-100 the remainder underflows and the
+// result is within an ulp.
 __device__ __forceinline__ float ratio(float x, float d) {
   const float r0 = __builtin_amdgcn_rcpf(d);
   const float r = __builtin_fmaf(__builtin_fmaf(-d, r0, 1.f), r0, r0);
@@ -73,15 +77,22 @@ __device__ __forceinline__ float mean2(float a, float b) { return __builtin_fmaf
 // pre = 0.5 (1 - (dt/h)|U|)|U|;  phi = num (sgn den + sgn num) den / D,
 // D = |den| + |num| if |den| > 0 else 1.  The marching stencil is bound by
 // these instructions (some 300 per cell, four cycles each), so:
-//   - D is the larger of |den| + |num| and the smallest normal number: at den =
-//     0 the quotient is 0 either way;
+//   - the quotient is ratio's for D in its range [2^-126, 2^126]; a wavefront
+//     that meets another D (differences of 8e37 and more, their infinite sum,
+//     subnormal ones; D = 0 with its den = 0 gives 0 either way) divides there
+//     (eight steps of 128 x 256^2 872 us without the test, 876 with it);
 //   - num (sgn den + sgn num) is 2 t with t = +-num, den's sign folded in,
 //     where t is positive (the signs agree), else 0 t, which keeps the NaN of
 //     an infinity: five instructions where two signs took ten.
 __device__ __forceinline__ float vl_correction(float U, float num_pos, float num_neg, float den,
                                                float dt_over_h) {
   const float num = (U > 0.f) ? num_pos : num_neg;
-  const float inv = ratio(den, fmaxf(fabsf(den) + fabsf(num), 0x1p-126f));
+  const float sum = fabsf(den) + fabsf(num);
+  const float d = __builtin_amdgcn_fmed3f(sum, 0x1p-126f, 0x1p126f);
+  float inv = ratio(den, d);
+  if (__builtin_expect(sum != d, 0)) {
+    if (fabsf(den) > 0.f) inv = den / sum;
+  }
   const float t = __uint_as_float(__float_as_uint(num) ^ (__float_as_uint(den) & 0x80000000u));
   const float phi = (t * ((t <= 0.f) ? 0.f : 2.f)) * inv;
   const float av = fabsf(U);
