@@ -140,6 +140,14 @@ int jcfd_fvm_plan_set_graphs(jcfd_fvm_plan* plan, int32_t enabled);
  * convergence flag read every 64 iterations (7.6 us).  No counterpart in the
  * reference; same results. */
 int jcfd_fvm_plan_set_cg_persistent(jcfd_fvm_plan* plan, int32_t enabled);
+/* A workgroup of the one-launch solve polls for a message this often (0 to
+ * 2^20, the default: about a second), then gives up; the solve then runs again
+ * in the other form, and the plan stays with that form for its next 256 solves
+ * (doubled, to 2^14, by give-ups in a row; set_cg_persistent ends the wait). */
+int jcfd_fvm_plan_set_cg_polls(jcfd_fvm_plan* plan, int32_t polls);
+/* CG solves of the plan so far: counts[0] in one launch, [1] in two launches
+ * per iteration, [2] given up in the first form (and counted in [1]). */
+int jcfd_fvm_cg_solves(const jcfd_fvm_plan* plan, int64_t* counts);
 
 /* Tile shapes and FFT radix schedule of the three step kernels.  No
  * counterpart in the reference (XLA picks its own kernels); set by the

@@ -292,6 +292,14 @@ int run_steps(GraphCache& graphs, const void* k, const void* k2, const void* k4,
 
 using namespace jcfd;
 
+// Polls of a message of the one-launch CG solve: about a second of waiting,
+// where a healthy launch's messages arrive within microseconds.
+constexpr int kCgPolls = 1 << 20;
+// Solves a plan stays in the two-launch form after a give-up, doubled by each
+// that follows without a one-launch solve in between: a second of waiting then
+// costs each of them 4 ms at most, as much as the form itself.
+constexpr int kCgRest = 256, kCgRestMost = 1 << 14;
+
 struct jcfd_fvm_plan {
   jcfd_fvm_config cfg;
   FvmParams params;
@@ -303,6 +311,10 @@ struct jcfd_fvm_plan {
   int* status_host = nullptr;  // pinned, 4 ints
   bool tiles_set = false;  // set_tiles pinned the shapes; otherwise each launch's size picks them
   bool cg_persistent = true;  // one cooperative launch per CG solve where the device holds it
+  int cg_polls = kCgPolls;    // of a message, before its workgroup gives up
+  int cg_rest = 0;            // solves left in the two-launch form after a give-up
+  int cg_rest_next = kCgRest;
+  int64_t cg_solves[3] = {0, 0, 0};  // in one launch, in two launches per iteration, given up
   int cg_maxiter = 0;
   int cg_last_iterations = 0;
   // CG implicit diffusion (diffusion == JCFD_DIFFUSION_IMPLICIT_CG), same buffers
@@ -438,38 +450,53 @@ int cg_iterate(jcfd_fvm_plan* p, int maxiter, int first, int* iterations, hipStr
   return rc;
 }
 
-// The solve as one cooperative launch (cg_launch_persistent) when enabled
-// and the device holds it: reads the status once at the end.  Returns
-// JCFD_ERR_UNSUPPORTED when the caller should run the chunked two-kernel form
-// instead, from a new cg_init: nothing was launched, or a workgroup gave up
-// waiting for another's message (the launch had to share the GPU with other
-// processes' such launches, and not all of its workgroups ran).
-int cg_persistent_solve(jcfd_fvm_plan* p, float rtol, float atol, int maxiter, bool helm, float coef,
-                        int* iterations, hipStream_t s) {
-  if (!p->cg_persistent) return JCFD_ERR_UNSUPPORTED;
-  int rc = cg_launch_persistent(p->params, p->cg, rtol, atol, maxiter, helm, coef, s);
+// A CG solve: init(s) sets it up, then one cooperative launch
+// (cg_launch_persistent) runs it where that is enabled and the device takes it,
+// else iterate(k, s), two launches per iteration, with a first chunk of `first`.
+// A launch whose workgroups do not all run (it had to share the GPU with other
+// processes' such launches) ends with a workgroup giving up: the solve then
+// starts again from init in the other form, and the plan stays with that form
+// for a while (kCgRest).
+template <typename Init, typename Iterate>
+int cg_run(jcfd_fvm_plan* p, float rtol, float atol, int maxiter, bool helm, float coef, int first,
+           int* iterations, hipStream_t s, Init init, Iterate iterate) {
+  int rc = init(s);
   if (rc) return rc;
-  if ((rc = check_hip(hipMemcpyAsync(p->status_host, p->cg.status, 4 * sizeof(int), hipMemcpyDeviceToHost,
-                                     s), "cg status")) ||
-      (rc = check_hip(hipStreamSynchronize(s), "cg status sync")))
-    return rc;
-  if (p->status_host[3] || !p->status_host[0]) return JCFD_ERR_UNSUPPORTED;
-  *iterations = p->status_host[1];
-  return JCFD_OK;
+  if (p->cg_persistent && p->cg_rest > 0) {
+    --p->cg_rest;
+  } else if (p->cg_persistent) {
+    rc = cg_launch_persistent(p->params, p->cg, rtol, atol, maxiter, helm, coef, p->cg_polls, s);
+    if (rc != JCFD_OK && rc != JCFD_ERR_UNSUPPORTED) return rc;
+    if (rc == JCFD_OK) {
+      if ((rc = check_hip(hipMemcpyAsync(p->status_host, p->cg.status, 4 * sizeof(int), hipMemcpyDeviceToHost,
+                                         s), "cg status")) ||
+          (rc = check_hip(hipStreamSynchronize(s), "cg status sync")))
+        return rc;
+      if (p->status_host[0] && !p->status_host[3]) {
+        *iterations = p->status_host[1];
+        p->cg_rest_next = kCgRest;
+        ++p->cg_solves[0];
+        return JCFD_OK;
+      }
+      ++p->cg_solves[2];
+      p->cg_rest = p->cg_rest_next;
+      p->cg_rest_next = std::min(2 * p->cg_rest_next, kCgRestMost);
+      if ((rc = init(s))) return rc;
+    }
+  }
+  ++p->cg_solves[1];
+  return cg_iterate(p, maxiter, first, iterations, s, iterate);
 }
 
 // CG on p->rhs into p->cg.x (solve_cg).
 int cg_solve(jcfd_fvm_plan* p, hipStream_t s) {
   const float rtol = static_cast<float>(p->cfg.cg_rtol), atol = static_cast<float>(p->cfg.cg_atol);
-  int rc = cg_launch_init(p->params, p->rhs, p->cg, rtol, atol, p->cg_maxiter, s);
-  if (rc) return rc;
-  rc = cg_persistent_solve(p, rtol, atol, p->cg_maxiter, false, 0.f, &p->cg_last_iterations, s);
-  if (rc != JCFD_ERR_UNSUPPORTED) return rc;
-  if (p->cg_persistent && (rc = cg_launch_init(p->params, p->rhs, p->cg, rtol, atol, p->cg_maxiter, s)))
-    return rc;
-  return cg_iterate(p, p->cg_maxiter, kCgChunk, &p->cg_last_iterations, s, [&](int k, hipStream_t st) {
-    return cg_launch_iteration(p->params, p->cg, k, rtol, atol, p->cg_maxiter, st);
-  });
+  return cg_run(
+      p, rtol, atol, p->cg_maxiter, false, 0.f, kCgChunk, &p->cg_last_iterations, s,
+      [&](hipStream_t st) { return cg_launch_init(p->params, p->rhs, p->cg, rtol, atol, p->cg_maxiter, st); },
+      [&](int k, hipStream_t st) {
+        return cg_launch_iteration(p->params, p->cg, k, rtol, atol, p->cg_maxiter, st);
+      });
 }
 
 // diffusion.solve_cg (diffusion.py:137-167) in place on both components of
@@ -483,19 +510,12 @@ int cg_diffuse(jcfd_fvm_plan* p, float* u, float* v, hipStream_t s) {
   const size_t bytes = sizeof(float) * static_cast<size_t>(p->params.n) * p->params.n;
   float* comps[2] = {u, v};
   for (int m = 0; m < 2; ++m) {
-    int rc = cg_launch_init_helmholtz(p->params, comps[m], p->cg, p->diff_coef, s);
-    if (rc == JCFD_OK) {
-      rc = cg_persistent_solve(p, rtol, atol, p->diff_maxiter, true, p->diff_coef,
-                               &p->diff_last_iterations[m], s);
-      if (rc == JCFD_ERR_UNSUPPORTED &&
-          (rc = p->cg_persistent ? cg_launch_init_helmholtz(p->params, comps[m], p->cg, p->diff_coef, s)
-                                 : JCFD_OK) == JCFD_OK)
-        rc = cg_iterate(p, p->diff_maxiter, kDiffusionFirstChunk, &p->diff_last_iterations[m], s,
-                        [&](int k, hipStream_t st) {
-                          return cg_launch_iteration_helmholtz(p->params, p->cg, k, rtol, atol,
-                                                               p->diff_maxiter, p->diff_coef, st);
-                        });
-    }
+    int rc = cg_run(
+        p, rtol, atol, p->diff_maxiter, true, p->diff_coef, kDiffusionFirstChunk, &p->diff_last_iterations[m], s,
+        [&](hipStream_t st) { return cg_launch_init_helmholtz(p->params, comps[m], p->cg, p->diff_coef, st); },
+        [&](int k, hipStream_t st) {
+          return cg_launch_iteration_helmholtz(p->params, p->cg, k, rtol, atol, p->diff_maxiter, p->diff_coef, st);
+        });
     if (rc == JCFD_OK)
       rc = check_hip(hipMemcpyAsync(comps[m], p->cg.x, bytes, hipMemcpyDeviceToDevice, s),
                      "copy diffused component");
@@ -781,6 +801,22 @@ int jcfd_fvm_plan_set_graphs(jcfd_fvm_plan* p, int32_t enabled) {
 int jcfd_fvm_plan_set_cg_persistent(jcfd_fvm_plan* p, int32_t enabled) {
   if (p == nullptr) return fail(JCFD_ERR_INVALID_ARGUMENT, "null plan");
   p->cg_persistent = enabled != 0;
+  p->cg_rest = 0;
+  p->cg_rest_next = kCgRest;
+  return JCFD_OK;
+}
+
+int jcfd_fvm_plan_set_cg_polls(jcfd_fvm_plan* p, int32_t polls) {
+  if (p == nullptr) return fail(JCFD_ERR_INVALID_ARGUMENT, "null plan");
+  if (polls < 0 || polls > kCgPolls)
+    return fail(JCFD_ERR_INVALID_ARGUMENT, "polls must be 0 to " + std::to_string(kCgPolls));
+  p->cg_polls = polls;
+  return JCFD_OK;
+}
+
+int jcfd_fvm_cg_solves(const jcfd_fvm_plan* p, int64_t* counts) {
+  if (p == nullptr || counts == nullptr) return fail(JCFD_ERR_INVALID_ARGUMENT, "null argument");
+  for (int k = 0; k < 3; ++k) counts[k] = p->cg_solves[k];
   return JCFD_OK;
 }
 

@@ -308,27 +308,26 @@ __device__ __forceinline__ void send(unsigned long long* m, int tag, float x) {
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Polls of a message before a workgroup gives up (about a second of waiting; a
-// message of a healthy launch arrives within microseconds).
-constexpr int kSpinLimit = 1 << 20;
-
 // Waits until all K messages carry `tag`; their values into x.  Bounded: false
-// after kSpinLimit polls, so a launch whose workgroups do not all run ends.
+// after `polls` polls, so a launch whose workgroups do not all run ends (0: one
+// poll that no message satisfies).
 template <int K>
-__device__ __forceinline__ bool receive(unsigned long long* const (&m)[K], int tag, float (&x)[K]) {
-  for (int spins = 0; spins < kSpinLimit; ++spins) {
+__device__ __forceinline__ bool receive(unsigned long long* const (&m)[K], int tag, float (&x)[K], int polls) {
+  const unsigned want = polls > 0 ? static_cast<unsigned>(tag) : ~0u;
+  bool all;
+  unsigned left = polls;
+  do {
     unsigned long long w[K];
-    bool all = true;
+    all = true;
 #pragma unroll
     for (int q = 0; q < K; ++q) w[q] = __hip_atomic_load(m[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int q = 0; q < K; ++q) {
-      all = all && static_cast<unsigned>(w[q] >> 32) == static_cast<unsigned>(tag);
+      all = all && static_cast<unsigned>(w[q] >> 32) == want;
       x[q] = __uint_as_float(static_cast<unsigned>(w[q]));
     }
-    if (all) return true;
-  }
-  return false;
+  } while (!all && left-- != 0);
+  return all;
 }
 
 // The whole solve in one cooperative launch (every workgroup resident at
@@ -354,7 +353,7 @@ __device__ __forceinline__ bool receive(unsigned long long* const (&m)[K], int t
 // place of the messages an iteration took 21.7 us at 256^2.
 template <int N, int RB, bool HELM>
 __global__ __launch_bounds__(kThreads) void cg_persistent(FvmParams p, CgBuffers c, float rtol, float atol,
-                                                          int maxiter, float coef) {
+                                                          int maxiter, float coef, int polls) {
   constexpr int NB = N / RB, TOT = RB * N;
   constexpr int PU = (TOT + kThreads - 1) / kThreads;    // cells per thread
   constexpr int PH = (2 * N + kThreads - 1) / kThreads;  // neighbour cells per thread: rows i0 - 1 and i0 + RB
@@ -402,7 +401,7 @@ __global__ __launch_bounds__(kThreads) void cg_persistent(FvmParams p, CgBuffers
       limit = tol2(p, sums[1], rtol, atol);
     } else {
       float in[1 + PH];
-      if (!receive(from, k, in)) s_fail = 1;
+      if (!receive(from, k, in, polls)) s_fail = 1;
 #pragma unroll
       for (int q = 0; q < PH; ++q) hr[q] = in[1 + q];
       float sums[1] = {0.f};
@@ -449,7 +448,7 @@ __global__ __launch_bounds__(kThreads) void cg_persistent(FvmParams p, CgBuffers
     const float mine = block_sum(pap, red + 2 * kWaves);
     if (tid < kMsgCopies) send(c.msg_pap + sum_slot(tid, blk), k + 1, mine);
     float in[1];
-    if (!receive(pap_from, k + 1, in)) s_fail = 1;
+    if (!receive(pap_from, k + 1, in, polls)) s_fail = 1;
     float sums[1] = {0.f};
     if (tid < NB) sums[0] = sums[0] + in[0];
     block_sums<1>(sums, red + 3 * kWaves);
@@ -502,9 +501,10 @@ struct CgOps {
     return check_hip(hipGetLastError(), "cg_init_helmholtz");
   }
   // The whole solve as one cooperative launch (N / RB workgroups, all
-  // resident).  JCFD_ERR_UNSUPPORTED when the device cannot hold them.
+  // resident).  JCFD_ERR_UNSUPPORTED when the device cannot hold them or
+  // refuses the launch.
   static int persistent(const FvmParams& p, const CgBuffers& c, float rtol, float atol, int maxiter,
-                        bool helm, float coef, hipStream_t s) {
+                        bool helm, float coef, int polls, hipStream_t s) {
     const void* fn = helm ? reinterpret_cast<const void*>(&cg_persistent<N, RB, true>)
                           : reinterpret_cast<const void*>(&cg_persistent<N, RB, false>);
     int dev = 0, coop = 0, cus = 0, per_cu = 0, rc;
@@ -517,9 +517,10 @@ struct CgOps {
     if (!coop || per_cu * cus < N / RB) return JCFD_ERR_UNSUPPORTED;
     FvmParams pp = p;
     CgBuffers cc = c;
-    void* args[] = {&pp, &cc, &rtol, &atol, &maxiter, &coef};
-    return check_hip(hipLaunchCooperativeKernel(fn, dim3(N / RB), dim3(kThreads), args, 0, s),
-                     "cg_persistent");
+    void* args[] = {&pp, &cc, &rtol, &atol, &maxiter, &coef, &polls};
+    if (hipLaunchCooperativeKernel(fn, dim3(N / RB), dim3(kThreads), args, 0, s) == hipSuccess) return JCFD_OK;
+    (void)hipGetLastError();  // nothing was launched: the caller's other form reports what is wrong, if it persists
+    return JCFD_ERR_UNSUPPORTED;
   }
   static int iteration_helmholtz(const FvmParams& p, const CgBuffers& c, int k, float rtol, float atol,
                                  int maxiter, float coef, hipStream_t s) {
@@ -562,14 +563,14 @@ int cg_launch_iteration(const FvmParams& p, const CgBuffers& c, int k, float rto
 }
 
 int cg_launch_persistent(const FvmParams& p, const CgBuffers& c, float rtol, float atol, int maxiter,
-                         bool helm, float coef, hipStream_t s) {
+                         bool helm, float coef, int polls, hipStream_t s) {
   switch (p.n) {
-    case 32: return CgOps<32>::persistent(p, c, rtol, atol, maxiter, helm, coef, s);
-    case 64: return CgOps<64>::persistent(p, c, rtol, atol, maxiter, helm, coef, s);
-    case 128: return CgOps<128>::persistent(p, c, rtol, atol, maxiter, helm, coef, s);
-    case 256: return CgOps<256>::persistent(p, c, rtol, atol, maxiter, helm, coef, s);
-    case 512: return CgOps<512>::persistent(p, c, rtol, atol, maxiter, helm, coef, s);
-    case 1024: return CgOps<1024>::persistent(p, c, rtol, atol, maxiter, helm, coef, s);
+    case 32: return CgOps<32>::persistent(p, c, rtol, atol, maxiter, helm, coef, polls, s);
+    case 64: return CgOps<64>::persistent(p, c, rtol, atol, maxiter, helm, coef, polls, s);
+    case 128: return CgOps<128>::persistent(p, c, rtol, atol, maxiter, helm, coef, polls, s);
+    case 256: return CgOps<256>::persistent(p, c, rtol, atol, maxiter, helm, coef, polls, s);
+    case 512: return CgOps<512>::persistent(p, c, rtol, atol, maxiter, helm, coef, polls, s);
+    case 1024: return CgOps<1024>::persistent(p, c, rtol, atol, maxiter, helm, coef, polls, s);
     default: return fail(JCFD_ERR_UNSUPPORTED, "CG grid size not built");
   }
 }

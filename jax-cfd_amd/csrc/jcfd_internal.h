@@ -109,10 +109,12 @@ int cg_sum_messages();  // words of msg_pap and of msg_rr
 int cg_launch_init(const FvmParams& p, const float* rhs, const CgBuffers& c, float rtol, float atol,
                    int maxiter, hipStream_t s);
 // The whole solve (after cg_launch_init / cg_launch_init_helmholtz) as one
-// cooperative launch; JCFD_ERR_UNSUPPORTED (no error recorded) when the
-// device cannot keep all its workgroups resident.
+// cooperative launch; JCFD_ERR_UNSUPPORTED (no error recorded, nothing
+// launched) when the device cannot keep all its workgroups resident or refuses
+// the launch.  A workgroup polls `polls` times for a message, then gives up
+// (status[3]).
 int cg_launch_persistent(const FvmParams& p, const CgBuffers& c, float rtol, float atol, int maxiter,
-                         bool helm, float coef, hipStream_t s);
+                         bool helm, float coef, int polls, hipStream_t s);
 // One CG iteration k (two kernels); a no-op once converged.
 int cg_launch_iteration(const FvmParams& p, const CgBuffers& c, int k, float rtol, float atol,
                         int maxiter, hipStream_t s);

@@ -124,6 +124,8 @@ _SIGNATURES = {
     "jcfd_ns2d_plan_set_graphs": (ctypes.c_int, [_P, ctypes.c_int32]),
     "jcfd_fvm_plan_set_graphs": (ctypes.c_int, [_P, ctypes.c_int32]),
     "jcfd_fvm_plan_set_cg_persistent": (ctypes.c_int, [_P, ctypes.c_int32]),
+    "jcfd_fvm_plan_set_cg_polls": (ctypes.c_int, [_P, ctypes.c_int32]),
+    "jcfd_fvm_cg_solves": (ctypes.c_int, [_P, ctypes.POINTER(ctypes.c_int64)]),
     "jcfd_ns2d_step": (ctypes.c_int, [_P, _P, _P, ctypes.c_int64, _P]),
     "jcfd_ns2d_explicit_terms": (ctypes.c_int, [_P, _P, _P, _P]),
     "jcfd_ns2d_time_kernels": (ctypes.c_int, [_P, _P, ctypes.c_int32,

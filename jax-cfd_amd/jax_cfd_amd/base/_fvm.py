@@ -118,6 +118,19 @@ class FvmPlan:
     _lib.check(self._lib.jcfd_fvm_plan_set_cg_persistent(self._handle, int(bool(enabled))),
                'jcfd_fvm_plan_set_cg_persistent')
 
+  def set_cg_polls(self, polls: int):
+    """Polls of a message of the one-launch CG solve before its workgroup gives
+    up and the solve runs in two launches per iteration."""
+    _lib.check(self._lib.jcfd_fvm_plan_set_cg_polls(self._handle, int(polls)),
+               'jcfd_fvm_plan_set_cg_polls')
+
+  @property
+  def cg_solves(self) -> dict:
+    """CG solves so far, by form."""
+    c = (ctypes.c_int64 * 3)()
+    _lib.check(self._lib.jcfd_fvm_cg_solves(self._handle, c), 'jcfd_fvm_cg_solves')
+    return dict(zip(('one_launch', 'two_launches', 'given_up'), (int(x) for x in c)))
+
   @property
   def tiles(self) -> dict:
     """Tile shapes and radix schedule of the step kernels."""
