@@ -1975,8 +1975,10 @@ int jcfd_fvm_group_launch_shape(const jcfd_fvm_group* g, int32_t* grid, int32_t*
 
 // ------------------------------------------------------------ spectral path
 namespace {
+constexpr size_t kNsPartCells = size_t(8) << 20;  // cells stepped together, see ns_run
+
 // nsteps CN-RK4 steps of `count` instances (slots, or 0..count-1) from
-// w_in to w_out (external layout; may alias): the state is moved into the
+// w_in to w_out (external layout; may alias or overlap): the state is moved into the
 // plan's internal-layout buffer, stepped in place there (graph replay when
 // enabled) and moved back.
 int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slots, int count,
@@ -1989,9 +1991,15 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
   // part all its steps: the spectra one kernel writes are then still cached
   // when the next reads them (512^2: 17.1 us per instance and step at 32
   // instances, 18.5 at 16, 19.1 at 64).
-  constexpr size_t kPartCells = size_t(8) << 20;
-  const int most = static_cast<int>(std::max<size_t>(1, kPartCells / (n * n)));
+  const int most = static_cast<int>(std::max<size_t>(1, kNsPartCells / (n * n)));
   const int parts = (count + most - 1) / most;
+  // Parts are read in as they come where that reads what the caller gave: an
+  // output that overlaps the input (other than being it) holds earlier parts'
+  // results by then, so everything is read in first.
+  const float2 *in_end = w_in + count * ext, *out_end = w_out + count * ext;
+  const bool read_first = parts > 1 && w_in != w_out && w_in < out_end && w_out < in_end;
+  int rc;
+  if (read_first && (rc = ns_launch_state_convert(p->n, true, w_in, p->ws, slots, count, s))) return rc;
   for (int k = 0; k < parts; ++k) {
     const int first = static_cast<int>(static_cast<int64_t>(count) * k / parts);
     const int m = static_cast<int>(static_cast<int64_t>(count) * (k + 1) / parts) - first;
@@ -2010,12 +2018,10 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
     b.h = p->h + o * ext;
     b.g = p->g + o * 4 * half;
     b.pbuf = p->pbuf + o * half;
-    int rc;
-    if ((rc = ns_launch_state_convert(p->n, true, w_in + o * ext, p->ws + o * ext, sl, m, s))) return rc;
-    if ((rc = ns_launch_step(p->n, stages, ns, b, m, s))) return rc;
-    if ((rc = run_steps(p->graphs, b.u_out, nullptr, sl, m, nsteps - 1, s,
-                        [&](hipStream_t gs) { return ns_launch_step(p->n, stages, ns, b, m, gs); })))
-      return rc;
+    auto step = [&](hipStream_t gs) { return ns_launch_step(p->n, stages, ns, b, m, gs); };
+    if (!read_first && (rc = ns_launch_state_convert(p->n, true, w_in + o * ext, p->ws + o * ext, sl, m, s))) return rc;
+    if ((rc = step(s))) return rc;
+    if ((rc = run_steps(p->graphs, b.u_out, nullptr, sl, m, nsteps - 1, s, step))) return rc;
     if ((rc = ns_launch_state_convert(p->n, false, p->ws + o * ext, w_out + o * ext, sl, m, s))) return rc;
   }
   return JCFD_OK;

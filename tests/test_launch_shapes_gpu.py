@@ -102,6 +102,27 @@ def test_spectral_batches_in_parts_match_lone_instances(n, batch):
     assert torch.equal(got[k], one.step(w[k].contiguous(), 34)), k
 
 
+# an output that overlaps the input: nothing is written before all is read
+@pytest.mark.parametrize("batch,shift", [(9, 1), (9, -1), (17, 4)])
+def test_spectral_parts_with_overlapping_output(batch, shift):
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  n = 1024
+  plan = _ns2d.Ns2dPlan(serving.SpectralFamily(n, _dev()).spec, batch, _dev())
+  gen = torch.Generator(device=_dev()).manual_seed(batch)
+  w = plan.rfft2(torch.randn((batch, n, n), device=_dev(), generator=gen))
+  want = plan.step(w, 2)
+  both = torch.zeros((batch + abs(shift), n, n // 2 + 1), dtype=torch.complex64, device=_dev())
+  first, second = both[:batch], both[abs(shift):]
+  src, dst = (first, second) if shift > 0 else (second, first)
+  src.copy_(w)
+  plan.step(src, 2, out=dst)
+  assert torch.equal(dst, want)
+  same = w.clone()
+  plan.step(same, 2, out=same)
+  assert torch.equal(same, want)
+
+
 # every wavefront layout of the column and row kernels, on instances whose
 # forcing list is longer than the registers hold and reaches column n / 2
 @pytest.mark.parametrize("n", [32, 64, 128, 256, 512, 1024])
