@@ -265,7 +265,7 @@ constexpr int kGraphChunk = 32;
 // graph cache when it is enabled (keyed by k..k4), the rest directly on s.
 template <typename Step>
 int run_steps(GraphCache& graphs, const void* k, const void* k2, const void* k4, int k3,
-              int64_t nsteps, hipStream_t s, Step&& step) {
+              int64_t nsteps, hipStream_t s, Step&& step, bool use_graphs = true) {
   auto chunk_of = [&](int len) {
     return [&step, len](hipStream_t gs) {
       for (int i = 0; i < len; ++i) {
@@ -277,7 +277,7 @@ int run_steps(GraphCache& graphs, const void* k, const void* k2, const void* k4,
   };
   int64_t remaining = nsteps;
   int rc;
-  if (graphs.enabled && remaining >= kGraphChunk) {
+  if (graphs.enabled && use_graphs && remaining >= kGraphChunk) {
     if ((rc = graphs.run(k, k2, k4, k3, kGraphChunk, remaining / kGraphChunk, s, chunk_of(kGraphChunk))))
       return rc;
     remaining %= kGraphChunk;
@@ -1993,6 +1993,10 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
   // instances, 18.5 at 16, 19.1 at 64).
   const int most = static_cast<int>(std::max<size_t>(1, kNsPartCells / (n * n)));
   const int parts = (count + most - 1) / most;
+  // Graph replay saves 2 to 4 % of a part's steps (65 steps of 64 x 512^2, two
+  // parts: 67.1 against 68.7 ms).  Every part has graphs of its own; more parts
+  // than half the cache holds would replace each other's on every call.
+  const bool graphs = parts <= GraphCache::kMaxGraphs / 2;
   // Parts are read in as they come where that reads what the caller gave: an
   // output that overlaps the input (other than being it) holds earlier parts'
   // results by then, so everything is read in first.
@@ -2021,7 +2025,7 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
     auto step = [&](hipStream_t gs) { return ns_launch_step(p->n, stages, ns, b, m, gs); };
     if (!read_first && (rc = ns_launch_state_convert(p->n, true, w_in + o * ext, p->ws + o * ext, sl, m, s))) return rc;
     if ((rc = step(s))) return rc;
-    if ((rc = run_steps(p->graphs, b.u_out, nullptr, sl, m, nsteps - 1, s, step))) return rc;
+    if ((rc = run_steps(p->graphs, b.u_out, nullptr, sl, m, nsteps - 1, s, step, graphs))) return rc;
     if ((rc = ns_launch_state_convert(p->n, false, p->ws + o * ext, w_out + o * ext, sl, m, s))) return rc;
   }
   return JCFD_OK;

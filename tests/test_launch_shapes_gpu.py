@@ -123,6 +123,21 @@ def test_spectral_parts_with_overlapping_output(batch, shift):
   assert torch.equal(same, want)
 
 
+# more parts than have graphs of their own
+def test_spectral_batch_in_many_parts():
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  n, batch = 1024, 137
+  spec = serving.SpectralFamily(n, _dev()).spec
+  plan, one = _ns2d.Ns2dPlan(spec, batch, _dev()), _ns2d.Ns2dPlan(spec, 1, _dev())
+  gen = torch.Generator(device=_dev()).manual_seed(batch)
+  w = one.rfft2(torch.randn((n, n), device=_dev(), generator=gen))
+  ws = w[None] * torch.linspace(0.5, 1.5, batch, device=_dev())[:, None, None]
+  got = plan.step(ws, 33)
+  for k in (0, 60, 136):
+    assert torch.equal(got[k], one.step(ws[k].contiguous(), 33)), k
+
+
 # every wavefront layout of the column and row kernels, on instances whose
 # forcing list is longer than the registers hold and reaches column n / 2
 @pytest.mark.parametrize("n", [32, 64, 128, 256, 512, 1024])
