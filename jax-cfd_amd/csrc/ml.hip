@@ -162,10 +162,11 @@ struct ConvSplit {
 // Hidden and output layers.  fp32 products on the bf16 matrix cores: each
 // operand is the exact sum of three bf16 parts, x = x0 + x1 + x2 (each part
 // the rounding of what the ones before it leave; 3 x 8 bits hold fp32's 24),
-// and x w is summed from the six part products of relative size above 2^-25
+// and x w is summed from the six largest part products
 // (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0; a bf16 product is exact in
 // fp32), accumulated in fp32.  What is left out, x1 w2 + x2 w1 + x2 w2, is at
-// most 2^-25 of x w, under the fp32 rounding of the sum itself.  Against 64 bits
+// most 2^-24 of x w (x = w = 1.0038986), one rounding of the product, and far
+// less on average.  Against 64 bits
 // whole towers (n 32 to 256, 16 to 64 channels, 3 and 7 layers, inputs of scale
 // 1 and 1e-3) err 0.29 to 0.60 as much, rms, as with v_mfma_f32_16x16x4_f32
 // products, 0.40 in the mean, because each sum is rounded once per 32 products.
@@ -187,7 +188,9 @@ struct ConvSplit {
 //
 // A value of magnitude 2^127 or more, an infinity or a NaN has no such split
 // (its first part would be infinite): a workgroup that meets one among its
-// inputs sums its outputs again from the fp32 values, one product at a time.
+// inputs forms its outputs from the fp32 values, v_mfma_f32_16x16x4_f32, the
+// weights added up from their parts: the tower's layers at 256^2, 64 channels,
+// all of them so, take 440 us against 184 with splits.
 template <int CIN, int COUT, bool RELU>
 __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
   using F = ConvSplit<CIN, COUT>;
@@ -198,6 +201,7 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
   constexpr int NBUF = F::CHUNKS > 1 ? 2 : 1;
   constexpr int ZC = COUT / F::CO;
   __shared__ bf16x8 shalo[NBUF][3][ITEMS];
+  __shared__ int s_wild[F::CHUNKS][4];  // whether a wavefront staged a value without a split, per chunk
   const int n = a.n;
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -220,7 +224,6 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
   };
   // halo tile of chunk g (rows i0-1 .. i0+4, columns j0-1 .. j0+32, periodic)
   float hreg[HPT][8];
-  bool wild = false;
   auto halo_load = [&](int g) {
 #pragma unroll
     for (int k = 0; k < HPT; ++k) {
@@ -232,7 +235,9 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
       for (int c = 0; c < 8; ++c) hreg[k][c] = (in + (g * CH + c) * plane)[off];
     }
   };
-  auto halo_store = [&](int buf) {
+  auto halo_store = [&](int g) {
+    const int buf = g % NBUF;
+    bool wild = false;
 #pragma unroll
     for (int k = 0; k < HPT; ++k) {
       const int e = tid + k * kThreads;
@@ -240,13 +245,14 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         const float x = hreg[k][c];
-        wild = wild || !(fabsf(x) < 0x1p127f);
         const __bf16 x0 = static_cast<__bf16>(x);
         const float r1 = x - static_cast<float>(x0);
         const __bf16 x1 = static_cast<__bf16>(r1);
+        const float r2 = r1 - static_cast<float>(x1);
+        wild = wild || !(fabsf(x) < 0x1p127f);
         p0[c] = x0;
         p1[c] = x1;
-        p2[c] = static_cast<__bf16>(r1 - static_cast<float>(x1));
+        p2[c] = static_cast<__bf16>(r2);
       }
       if (ITEMS % kThreads == 0 || e < ITEMS) {
         shalo[buf][0][e] = p0;
@@ -254,6 +260,12 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
         shalo[buf][2][e] = p2;
       }
     }
+    const int any = __any(wild);
+    if (lane == 0) s_wild[g][wave] = any;
+  };
+  // after the barrier that follows the chunk's halo_store
+  auto chunk_is_wild = [&](int g) {
+    return __builtin_amdgcn_readfirstlane(s_wild[g][0] | s_wild[g][1] | s_wild[g][2] | s_wild[g][3]) != 0;
   };
   bf16x8 wa[NCB][3], wb[NCB][3];
   load(0, wa);
@@ -316,45 +328,48 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
     if constexpr (s % F::SPC == 0 && g + 1 < F::CHUNKS) halo_load(g + 1);
     step(s, cur);
     if constexpr (s % F::SPC == F::SPC - 1 && g + 1 < F::CHUNKS) {
-      halo_store((g + 1) % NBUF);  // its buffer's last reader was chunk g - 1
+      halo_store(g + 1);  // its buffer's last reader was chunk g - 1
       __syncthreads();
     }
   };
-  static_for<0, STEPS>([&](auto sc) {
-    if constexpr (decltype(sc)::value % 2 == 0) run(sc, wa, wb);
-    else run(sc, wb, wa);
-  });
-
-  if (__syncthreads_or(wild)) {
-#pragma unroll 1
+  bool wild = chunk_is_wild(0);
+  if (!wild) {
+    static_for<0, STEPS>([&](auto sc) {
+      if constexpr (decltype(sc)::value % 2 == 0) run(sc, wa, wb);
+      else run(sc, wb, wa);
+    });
+#pragma unroll
+    for (int g = 1; g < F::CHUNKS; ++g) wild = wild || chunk_is_wild(g);
+  }
+  if (wild) {
+#pragma unroll
     for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll 1
-      for (int pb = 0; pb < NPB; ++pb)
-#pragma unroll 1
-        for (int r = 0; r < 4; ++r) {
-          const int b = cb0 + cb, i = i0 + (pw * NPB + pb) / 2, j = j0 + (pb % 2) * 16 + lp;
-          float sum = 0.f;
-#pragma unroll 1
-          for (int tap = 0; tap < 9; ++tap)
-#pragma unroll 1
-            for (int ci = 0; ci < CIN; ++ci) {
-              const int s = (ci / CH) * F::SPC + tap / F::TPS, k = (tap % F::TPS) * CH + ci % CH;
-              const __bf16* wp = static_cast<const __bf16*>(a.w) +
-                                 (((s * (COUT / 16) + b) * 3) * 64 + 4 * kq + r + 16 * (k / 8)) * 8 + k % 8;
-              const float w = static_cast<float>(wp[0]) +
-                              (static_cast<float>(wp[512]) + static_cast<float>(wp[1024]));
-              sum = __builtin_fmaf(w, in[ci * plane + static_cast<size_t>((i + tap / 3 - 1) & (n - 1)) * n +
-                                         ((j + tap % 3 - 1) & (n - 1))], sum);
-            }
-          // one element of a register array by a run-time index
 #pragma unroll
-          for (int c2 = 0; c2 < NCB; ++c2)
+      for (int pb = 0; pb < NPB; ++pb) acc[cb][pb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // a step's 32 products in eight MFMA of four: k = 8 kq + e in the e-th
+#pragma unroll 1
+    for (int s = 0; s < STEPS; ++s) {
+      const int tap = (s % F::SPC) * F::TPS + (F::TPS == 2 ? kq / 2 : 0);
+      const float* xc = in + ((s / F::SPC) * CH + 8 * kg) * plane;
+      load(s, wa);
 #pragma unroll
-            for (int p2 = 0; p2 < NPB; ++p2)
+      for (int pb = 0; pb < NPB; ++pb) {
+        const int i = (i0 + block_row(pb) + tap / 3 - 1) & (n - 1);
+        const int j = (j0 + (pb % 2) * 16 + lp + tap % 3 - 1) & (n - 1);
+        float x[8];
 #pragma unroll
-              for (int r2 = 0; r2 < 4; ++r2)
-                if (c2 == cb && p2 == pb && r2 == r) acc[c2][p2][r2] = sum;
+        for (int e = 0; e < 8; ++e) x[e] = xc[e * plane + static_cast<size_t>(i) * n + j];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (F::TPS == 2 && tap > 8) x[e] = 0.f;  // the ninth tap's partner: not 0 times an infinity
+#pragma unroll
+          for (int cb = 0; cb < NCB; ++cb)
+            acc[cb][pb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                static_cast<float>(wa[cb][0][e]) + (static_cast<float>(wa[cb][1][e]) + static_cast<float>(wa[cb][2][e])),
+                x[e], acc[cb][pb], 0, 0, 0);
         }
+      }
+    }
   }
 
   // out[co][i0 + row][j0 + px] = act(acc + b[co])

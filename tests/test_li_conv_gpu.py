@@ -67,6 +67,29 @@ def test_tower_values_without_a_split(hidden, value):
       assert float((g[ok] - w[ok]).abs().max()) <= 1e-5 * float(w[ok].abs().max())
 
 
+@pytest.mark.parametrize('n,hidden,layers', [(256, 64, 6), (128, 32, 3), (64, 16, 2)])
+def test_values_without_a_split_cost_a_few_plain_ones(n, hidden, layers):
+  # the fp32 matrix instructions take 2.7 times the time of the six bf16 ones
+  params, v0 = ml._case(n, hidden, layers, seed=3)
+  plan = ml._model(n, params, hidden, layers)[0].plan(ml._dev())
+  plain = tuple(torch.as_tensor(x.data, device=ml._dev()) for x in v0)
+  huge = tuple(x / x.abs().max() * 3e38 for x in plain)
+
+  def best(fields):
+    times = []
+    for _ in range(5):
+      start, end = torch.cuda.Event(True), torch.cuda.Event(True)
+      start.record()
+      for _ in range(10):
+        plan.tower(*fields)
+      end.record()
+      end.synchronize()
+      times.append(start.elapsed_time(end))
+    return min(times)
+
+  assert best(huge) <= 6 * best(plain)
+
+
 def test_explicit_row_blocks_agree():
   # 9 x 128^2 takes four rows and both components per workgroup, 128^2 one of each
   n, batch = 128, 9
