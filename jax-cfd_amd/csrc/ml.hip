@@ -186,11 +186,16 @@ struct ConvSplit {
 // made once per workgroup, when a chunk of 32 channels is staged, and the
 // second chunk is loaded while the first is used.
 //
-// A value of magnitude 2^127 or more, an infinity or a NaN has no such split
-// (its first part would be infinite): a workgroup that meets one among its
-// inputs forms its outputs from the fp32 values, v_mfma_f32_16x16x4_f32, the
-// weights added up from their parts: the tower's layers at 256^2, 64 channels,
-// all of them so, take 440 us against 184 with splits.
+// Values without such a split show in what the first two parts leave: NaN for
+// infinities, NaN and values whose first part is infinite (beyond 2^128 -
+// 2^119), a subnormal number where the third part may end below bf16's 2^-133
+// (values under 2^-110; the matrix cores keep subnormal parts).  A workgroup
+// that meets one among its inputs forms its outputs from the fp32 values,
+// v_mfma_f32_16x16x4_f32, the weights added up from their parts: the tower's
+// layers at 256^2, 64 channels, all of them so, take 440 us against 184 with
+// splits.  (Parts of a weight under 2^-133 are dropped: an output moves by
+// 2^-134 of its inputs' sum at most.)
+constexpr int kNoSplit = 0x297;  // v_cmp_class_f32: NaN, infinite or subnormal
 template <int CIN, int COUT, bool RELU>
 __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
   using F = ConvSplit<CIN, COUT>;
@@ -249,7 +254,7 @@ __global__ __launch_bounds__(kThreads, 2) void li_conv3x3(LiConvArgs a) {
         const float r1 = x - static_cast<float>(x0);
         const __bf16 x1 = static_cast<__bf16>(r1);
         const float r2 = r1 - static_cast<float>(x1);
-        wild = wild || !(fabsf(x) < 0x1p127f);
+        wild = wild || __builtin_amdgcn_classf(r2, kNoSplit);
         p0[c] = x0;
         p1[c] = x1;
         p2[c] = static_cast<__bf16>(r2);

@@ -67,6 +67,21 @@ def test_tower_values_without_a_split(hidden, value):
       assert float((g[ok] - w[ok]).abs().max()) <= 1e-5 * float(w[ok].abs().max())
 
 
+@pytest.mark.parametrize('hidden', [16, 32, 64])
+@pytest.mark.parametrize('scale', [1e-35, 1e-30])
+def test_tower_rounding_of_small_values(hidden, scale):
+  # as test_tower_rounding, on activations near and under the least ones whose
+  # three bf16 parts are normal numbers; no biases, which would cover them
+  n = 64
+  params, v0 = ml._case(n, hidden, 2, seed=3)
+  params = [(w, np.zeros_like(b)) for w, b in params]
+  plan = ml._model(n, params, hidden, 2)[0].plan(ml._dev())
+  u, v = (torch.as_tensor(x.data, device=ml._dev()) * scale for x in v0)
+  got = plan.tower(u, v, coefficients=False)[0, :120].double().cpu()
+  want = _tower(u, v, params)
+  assert float((got - want).norm() / want.norm()) <= 2.0 ** -21
+
+
 @pytest.mark.parametrize('n,hidden,layers', [(256, 64, 6), (128, 32, 3), (64, 16, 2)])
 def test_values_without_a_split_cost_a_few_plain_ones(n, hidden, layers):
   # the fp32 matrix instructions take 2.7 times the time of the six bf16 ones
