@@ -588,21 +588,30 @@ void li_conv_weight_layout(const float* w, int cinp, int cout, void* out) {
     return;
   }
   // li_conv3x3: fragment (step, channel block, part), lane l, element e is
-  // k = 8 (l / 16) + e of the step, output channel l % 16 of the block
+  // k = 8 (l / 16) + e of the step, output channel l % 16 of the block.  The
+  // 8 k x 16 channels of 16 lanes are one contiguous run, split together.
   uint16_t* frag = static_cast<uint16_t*>(out);
   const int ch = cinp < 32 ? cinp : 32, tps = 32 / ch, spc = (9 + tps - 1) / tps;
   for (int s = 0; s < spc * (cinp / ch); ++s)
-    for (int cb = 0; cb < ncb; ++cb)
-      for (int l = 0; l < 64; ++l)
-        for (int e = 0; e < 8; ++e) {
-          const int k = 8 * (l / 16) + e, tap = (s % spc) * tps + k / ch, ci = (s / spc) * ch + k % ch;
-          float x = tap < 9 ? weight(tap, ci, cb * 16 + l % 16) : 0.f;
-          for (int q = 0; q < 3; ++q) {
-            const uint16_t part = to_bf16(x);
-            frag[(((static_cast<size_t>(s) * ncb + cb) * 3 + q) * 64 + l) * 8 + e] = part;
-            x -= from_bf16(part);
-          }
+    for (int k8 = 0; k8 < 4; ++k8) {
+      const int tap = (s % spc) * tps + 8 * k8 / ch, ci = (s / spc) * ch + 8 * k8 % ch;
+      for (int cb = 0; cb < ncb; ++cb) {
+        float x[128] = {};
+        if (tap < 9) {
+          const float* src = w + (static_cast<size_t>(tap) * cinp + ci) * cout + cb * 16;
+          for (int i = 0; i < 16; ++i)
+            for (int e = 0; e < 8; ++e) x[8 * i + e] = src[static_cast<size_t>(e) * cout + i];
         }
+        for (int q = 0; q < 3; ++q) {
+          uint16_t part[128];
+          for (int i = 0; i < 128; ++i) {
+            part[i] = to_bf16(x[i]);
+            x[i] -= from_bf16(part[i]);
+          }
+          std::memcpy(frag + ((static_cast<size_t>(s) * ncb + cb) * 3 + q) * 512 + 128 * k8, part, sizeof(part));
+        }
+      }
+    }
 }
 
 bool li_conv_supported(int cin, int cout, bool relu) {
