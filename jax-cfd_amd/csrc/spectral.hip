@@ -16,10 +16,11 @@
 //   ns_rows           RB rows: four inverse packed real row FFTs, the
 //                     product -(gx vx + gy vy), forward packed real row FFT -> P.
 //   ns_cols_forward   column tile: forward column FFT of P, unpack the DC/
-//                     Nyquist word, 2/3 filter, forcing curl, then either write
-//                     F (explicit-terms seam) or the RK/CN update of (u, h),
-//                     optionally followed directly by the next stage's
-//                     ns_cols_inverse work on the same tile.
+//                     Nyquist word, 2/3 filter, forcing curl, then the RK/CN
+//                     update of (u, h), optionally followed directly by the
+//                     next stage's ns_cols_inverse work on the same tile.
+//   rows_r2c, ns_cols_out and ns_cols_in, rows_c2r   rfft2 and irfft2; the
+//                     explicit-terms seam ends in ns_cols_out.
 //
 // Packed half spectra: word 0 of a row holds (X[0], X[n/2]) of a real row;
 // the column pass of word 0 therefore carries two Hermitian columns, which
@@ -157,13 +158,12 @@ __device__ __forceinline__ float recompute(float x) {
   return x;
 }
 
-// Inverse column transforms of the tile -> G[0..NSPEC): the four derivative
-// spectra (NSPEC = 4: d_x w, d_y w, v_x, v_y) or the field itself (NSPEC = 1),
-// scaled by 1/n^2.  w becomes psi w, psi = -1/laplacian, for the last two, so
+// Inverse column transforms of the tile -> G[0..4): the four derivative
+// spectra (d_x w, d_y w, v_x, v_y), scaled by 1/n^2.  w becomes psi w, psi = -1/laplacian, for the last two, so
 // no second array is held.  Column 0 is the symmetrised pair of the DC and
 // Nyquist columns, s0 + i sh with s(p) = (a(p) + conj a(-p)) / 2, from the two
 // columns in LDS (w0, wn): kx(-p) = -kx(p) (but at 0 and N/2), psi(-p) = psi(p).
-template <int N, int NSPEC, int R, typename TW>
+template <int N, int R, typename TW>
 __device__ __forceinline__ void cols_inverse_body(float2 (&w)[ColShape<N>::E], const TW& tw, const ColLane<N>& ln,
                                                   const ColLds<N>& lds, const NsParams& q,
                                                   float2* __restrict__ g) {
@@ -173,7 +173,7 @@ __device__ __forceinline__ void cols_inverse_body(float2 (&w)[ColShape<N>::E], c
   const float ky = q.ky[ln.c], kyh = q.ky[H];
   const float ay = q.two_pi * ky, ayh = q.two_pi * kyh;
 #pragma unroll 1
-  for (int m = 0; m < NSPEC; ++m) {
+  for (int m = 0; m < 4; ++m) {
     const float jf = recompute(static_cast<float>(ln.j));
     if (m == 2) {
 #pragma unroll
@@ -201,7 +201,7 @@ __device__ __forceinline__ void cols_inverse_body(float2 (&w)[ColShape<N>::E], c
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const float k = along_y ? ay : q.two_pi * lane_kx<N>(q, jf, e);
-      v[e] = NSPEC == 1 ? w[e] : mul_i(sign * k, w[e]);
+      v[e] = mul_i(sign * k, w[e]);
     }
     if (ln.c == 0 && ln.own) {
 #pragma unroll
@@ -212,9 +212,9 @@ __device__ __forceinline__ void cols_inverse_body(float2 (&w)[ColShape<N>::E], c
         const float kx1 = lane_kx<N>(q, jf, e);
         const float kp = sign * (q.two_pi * kx1), km = pm == p ? kp : -kp;
         const float2 a0 = v[e];
-        const float2 b0 = NSPEC == 1 ? z0 : mul_i(along_y ? ay : km, z0);
-        const float2 ah = NSPEC == 1 ? zp : mul_i(along_y ? ayh : kp, zp);
-        const float2 bh = NSPEC == 1 ? zm : mul_i(along_y ? ayh : km, zm);
+        const float2 b0 = mul_i(along_y ? ay : km, z0);
+        const float2 ah = mul_i(along_y ? ayh : kp, zp);
+        const float2 bh = mul_i(along_y ? ayh : km, zm);
         const float2 s0 = make_float2(0.5f * (a0.x + b0.x), 0.5f * (a0.y - b0.y));
         const float2 sh = make_float2(0.5f * (ah.x + bh.x), 0.5f * (ah.y - bh.y));
         v[e] = make_float2(s0.x - sh.y, s0.y + sh.x);  // s0 + i sh
@@ -238,22 +238,18 @@ struct NsColOcc {
   static constexpr int value = N == 1024 ? 2 : 4;
 };
 
-// One wavefront's columns from c0: the state -> the inverse transforms of the
-// four spectra (NSPEC = 4) or of the field (NSPEC = 1); w and g already point
-// at the instance.
-template <int N, int NSPEC, int R>
+// One wavefront's columns from c0: the state (internal layout) -> the inverse
+// transforms of the four spectra; w and g already point at the instance.
+template <int N, int R>
 __device__ __forceinline__ void cols_inverse_tile(const ColLds<N>& lds, const NsParams& q,
                                                   const float2* __restrict__ w, float2* __restrict__ g,
                                                   int c0, int width, int lane) {
   using S = ColShape<N>;
   constexpr int E = S::E, L = S::L, H = N / 2;
   const ColLane<N> ln(c0, width, lane);
-  // the step (NSPEC = 4) reads the internal state, irfft2 (NSPEC = 1) the
-  // caller's array
-  auto at = [&](int p, int c) { return NSPEC == 4 ? six<N>(p, c) : p * (H + 1) + c; };
   float2 wt[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) wt[e] = w[at(ln.j + e * L, ln.c)];
+  for (int e = 0; e < E; ++e) wt[e] = w[six<N>(ln.j + e * L, ln.c)];
   RegTwiddles<N, E, R> tw;
   tw.template load<1>(q.tw, ln.j);
   if (c0 == 0) {
@@ -261,15 +257,15 @@ __device__ __forceinline__ void cols_inverse_tile(const ColLds<N>& lds, const Ns
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         lds.w0[ln.j + e * L] = wt[e];
-        lds.wn[ln.j + e * L] = w[at(ln.j + e * L, H)];
+        lds.wn[ln.j + e * L] = w[six<N>(ln.j + e * L, H)];
       }
     }
     wave_lds_sync();
   }
-  cols_inverse_body<N, NSPEC, R>(wt, tw, ln, lds, q, g);
+  cols_inverse_body<N, R>(wt, tw, ln, lds, q, g);
 }
 
-template <int N, int NSPEC, int R>
+template <int N, int R>
 __global__ __launch_bounds__(1024 / ColShape<N>::E * 8, (NsColOcc<N>::value)) void ns_cols_inverse(
     NsParams q, const float2* __restrict__ w, float2* __restrict__ g, int width) {
   extern __shared__ float4 ns_smem[];
@@ -277,12 +273,15 @@ __global__ __launch_bounds__(1024 / ColShape<N>::E * 8, (NsColOcc<N>::value)) vo
   const ColLds<N> lds(reinterpret_cast<char*>(ns_smem), blockDim.x / 64, wave);
   const int c0 = xcd_tile(blockIdx.x, gridDim.x) * width + wave * ColShape<N>::T;
   const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
-  cols_inverse_tile<N, NSPEC, R>(lds, q, w + inst * static_cast<size_t>(N) * (N / 2 + 1),
-                                        g + inst * NSPEC * static_cast<size_t>(N) * (N / 2), c0, width,
-                                        threadIdx.x % 64);
+  cols_inverse_tile<N, R>(lds, q, w + inst * static_cast<size_t>(N) * (N / 2 + 1),
+                          g + inst * 4 * static_cast<size_t>(N) * (N / 2), c0, width, threadIdx.x % 64);
 }
 
-// Packed real row transforms of a batch of real (N, N) fields.
+// Packed real row transforms of a batch of real (N, N) fields.  Between the
+// passes of rfft2 and irfft2 the packed words lie row by row: both passes then
+// read and write runs of a row (in the step's column tiles, one word wide at
+// 512^2, the row pass stores single words; rfft2 and irfft2 of 64 x 512^2 in
+// those tiles 110 and 103 us, row by row 63 and 64).
 template <int N, int RB>
 __global__ __launch_bounds__(kThreads) void rows_r2c(NsParams q, const float* __restrict__ x,
                                                      float2* __restrict__ pout) {
@@ -308,7 +307,7 @@ __global__ __launch_bounds__(kThreads) void rows_r2c(NsParams q, const float* __
   lds_fft_waves<H, RB, kThreads, 1, H, false>(zb, twh, tid);
   for (int e = tid; e < RB * H; e += kThreads) {
     const int r = e / H, k = e % H;
-    pout[tix<N>(i0 + r, k)] = r2c_combine(zb + r * H, k, H, twn[k]);
+    pout[(i0 + r) * H + k] = r2c_combine(zb + r * H, k, H, twn[k]);
   }
 }
 
@@ -329,7 +328,7 @@ __global__ __launch_bounds__(kThreads) void rows_c2r(NsParams q, const float2* _
       tid,
       [&](int e) {
         const int r = e / H, k = e % H;
-        return F2Triple{pin[tix<N>(i0 + r, k)], pin[tix<N>(i0 + r, (H - k) & (H - 1))], q.tw[k]};
+        return F2Triple{pin[(i0 + r) * H + k], pin[(i0 + r) * H + ((H - k) & (H - 1))], q.tw[k]};
       },
       [&](int e, F2Triple v) { zb[e] = c2r_combine(v.a, v.b, e % H, v.t); });
   tb.store(twh, tid);
@@ -588,17 +587,16 @@ __device__ __forceinline__ float ns_filter(const NsParams& q, int p, int c) {
 }
 
 // One wavefront's columns from c0 of the forward column pass: P's columns ->
-// explicit terms F in the external layout (MODE 0), the RK/CN update of
-// (u, h) in the internal state layout (MODE 1), or the update followed by the
-// next stage's inverse work on the new columns (MODE 2); all pointers already
-// point at the instance.
+// the RK/CN update of (u, h) in the internal state layout (MODE 1), or the
+// update followed by the next stage's inverse work on the new columns (MODE 2);
+// all pointers already point at the instance.
 template <int N, int MODE, int R>
 __device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const NsParams& q,
                                                   const float2* __restrict__ pin, const float2* u_in,
                                                   float2* u_out, float2* h, float2* __restrict__ g,
                                                   int c0, int width, int lane) {
   using S = ColShape<N>;
-  constexpr int E = S::E, L = S::L, T = S::T, H = N / 2, H1 = H + 1;
+  constexpr int E = S::E, L = S::L, T = S::T, H = N / 2;
   constexpr int ES = L * kTw<N>;  // words between a lane's elements, in P, G, u and h
   const ColLane<N> ln(c0, width, lane);
   const int at0 = tix<N>(ln.j, ln.c);  // the lane's element 0 (u and h: six = tix for c < N/2)
@@ -611,25 +609,22 @@ __device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const Ns
   for (int e = 0; e < E; ++e) v[e] = pl[e * ES];
   RegTwiddles<N, E, R> tw;
   tw.template load<1>(q.tw, ln.j);
-  [[maybe_unused]] float2 uo[MODE == 0 ? 1 : E], ho[MODE == 0 ? 1 : E];
-  [[maybe_unused]] float ky = 0.f;
-  if constexpr (MODE != 0) {
-    const float2* ul = u_in + at0;
-    const float2* hl = h + at0;
+  float2 uo[E], ho[E];
+  const float2* ul = u_in + at0;
+  const float2* hl = h + at0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    uo[e] = ul[e * ES];
+    ho[e] = q.read_h ? hl[e * ES] : make_float2(0.f, 0.f);
+  }
+  const float ky = q.ky[ln.c];
+  if (ln.c == 0 && ln.own) {  // (u, h) of the Nyquist column, parked in LDS
+    const float2* uh = u_in + six<N>(ln.j, H);
+    const float2* hh = h + six<N>(ln.j, H);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      uo[e] = ul[e * ES];
-      ho[e] = q.read_h ? hl[e * ES] : make_float2(0.f, 0.f);
-    }
-    ky = q.ky[ln.c];
-    if (ln.c == 0 && ln.own) {  // (u, h) of the Nyquist column, parked in LDS
-      const float2* uh = u_in + six<N>(ln.j, H);
-      const float2* hh = h + six<N>(ln.j, H);
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        lds.wn[ln.j + e * L] = uh[e * L];
-        if (q.read_h) lds.w0[ln.j + e * L] = hh[e * L];
-      }
+      lds.wn[ln.j + e * L] = uh[e * L];
+      if (q.read_h) lds.w0[ln.j + e * L] = hh[e * L];
     }
   }
   float2* x = lds.x;
@@ -646,7 +641,7 @@ __device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const Ns
     const float inv = 1.0f / (1.0f - q.mu * Lc);
     return make_float2(inv * xx.x, inv * xx.y);
   };
-  [[maybe_unused]] const float jf = recompute(static_cast<float>(ln.j));
+  const float jf = recompute(static_cast<float>(ln.j));
 
   if (c0 == 0) {
     // column 0 of tile 0 carries the DC (A) and Nyquist (B) columns:
@@ -674,24 +669,19 @@ __device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const Ns
             if (q.force_idx[2 * t] == p && q.force_idx[2 * t + 1] == H) f = cadd(f, q.force_val[t]);
         return f;
       };
-      if constexpr (MODE == 0) {
+      const float kyh = q.ky[H];
+      float2* hn = h + six<N>(ln.j, H);
+      float2* un = u_out + six<N>(ln.j, H);
 #pragma unroll
-        for (int e = 0; e < E; ++e) u_out[(ln.j + e * L) * H1 + H] = nyquist(ln.j + e * L);
-      } else {
-        const float kyh = q.ky[H];
-        float2* hn = h + six<N>(ln.j, H);
-        float2* un = u_out + six<N>(ln.j, H);
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-          const int p = ln.j + e * L;
-          const float2 h0 = q.read_h ? lds.w0[p] : make_float2(0.f, 0.f);
-          float2 f = nyquist(p);
-          const float2 w = update(lane_kx<N>(q, jf, e), kyh, f, lds.wn[p], h0);
-          hn[e * L] = f;
-          un[e * L] = w;
-          if constexpr (MODE == 2) lds.wn[p] = w;
-        }
+      for (int e = 0; e < E; ++e) {
+        if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+        const int p = ln.j + e * L;
+        const float2 h0 = q.read_h ? lds.w0[p] : make_float2(0.f, 0.f);
+        float2 f = nyquist(p);
+        const float2 w = update(lane_kx<N>(q, jf, e), kyh, f, lds.wn[p], h0);
+        hn[e * L] = f;
+        un[e * L] = w;
+        if constexpr (MODE == 2) lds.wn[p] = w;
       }
     }
   }
@@ -711,25 +701,18 @@ __device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const Ns
         if (e == se) v[e] = cadd(v[e], f);
     }
   }
-  if constexpr (MODE == 0) {
-    if (ln.own) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) u_out[(ln.j + e * L) * H1 + ln.c] = v[e];
-    }
-  } else {
+  for (int e = 0; e < E; ++e) {
+    if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two elements' updates in registers at a time
+    uo[e] = update(lane_kx<N>(q, jf, e), ky, v[e], uo[e], ho[e]);
+  }
+  if (ln.own) {
+    float2* hs = h + at0;
+    float2* us = u_out + at0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two elements' updates in registers at a time
-      uo[e] = update(lane_kx<N>(q, jf, e), ky, v[e], uo[e], ho[e]);
-    }
-    if (ln.own) {
-      float2* hs = h + at0;
-      float2* us = u_out + at0;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        hs[e * ES] = v[e];
-        us[e * ES] = uo[e];
-      }
+      hs[e * ES] = v[e];
+      us[e * ES] = uo[e];
     }
   }
   if constexpr (MODE == 2) {
@@ -740,7 +723,7 @@ __device__ __forceinline__ void cols_forward_tile(const ColLds<N>& lds, const Ns
       }
       wave_lds_sync();
     }
-    cols_inverse_body<N, 4, R>(uo, tw, ln, lds, q, g);
+    cols_inverse_body<N, R>(uo, tw, ln, lds, q, g);
   }
 }
 
@@ -755,8 +738,7 @@ __global__ __launch_bounds__(1024 / ColShape<N>::E * 8, (NsColOcc<N>::value)) vo
   const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
   const size_t ext = static_cast<size_t>(N) * (N / 2 + 1);
   cols_forward_tile<N, MODE, R>(lds, q, pin + inst * static_cast<size_t>(N) * (N / 2),
-                                u_in ? u_in + inst * ext : nullptr, u_out + inst * ext,
-                                h ? h + inst * ext : nullptr,
+                                u_in + inst * ext, u_out + inst * ext, h + inst * ext,
                                 g ? g + inst * 4 * static_cast<size_t>(N) * (N / 2) : nullptr, c0, width,
                                 threadIdx.x % 64);
 }
@@ -1136,12 +1118,104 @@ __global__ __launch_bounds__(kThreads, (StagedWaves<N, W>::value)) void ns_cols_
   const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
   const size_t ext = static_cast<size_t>(N) * (N / 2 + 1);
   staged_forward_tile<N, W, MODE, R>(sm, q, pin + inst * static_cast<size_t>(N) * (N / 2),
-                                   u_in ? u_in + inst * ext : nullptr, u_out + inst * ext,
-                                   h ? h + inst * ext : nullptr,
+                                   u_in + inst * ext, u_out + inst * ext, h + inst * ext,
                                    g ? g + inst * 4 * static_cast<size_t>(N) * (N / 2) : nullptr,
                                    xcd_tile(blockIdx.x, gridDim.x) * W, threadIdx.x);
 }
 
+
+// ---- column kernels of the transforms and the explicit terms -----------------
+// Their external side (rows of n/2 + 1 words) is read and written column by
+// column, so W columns share a workgroup and its cache lines.
+
+// Columns of P -> out in the external layout: the filter and the forcing curl
+// entries of explicit_terms (rfft2 passes neither).  P in the step's column
+// tiles (TILED) or row by row.
+template <int N, int W, bool TILED>
+__global__ __launch_bounds__(kThreads) void ns_cols_out(NsParams q, const float2* __restrict__ pin,
+                                                        float2* __restrict__ out) {
+  constexpr int H = N / 2, H1 = H + 1, PER = (N * W + kThreads - 1) / kThreads;
+  __shared__ float2 buf[N * W];
+  __shared__ float2 tw[N];
+  const int tid = threadIdx.x, c0 = xcd_tile(blockIdx.x, gridDim.x) * W;
+  const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
+  pin += inst * static_cast<size_t>(N) * H;
+  out += inst * static_cast<size_t>(N) * H1;
+  TwiddleStage<N, 1, kThreads> tws;
+  tws.load(q.tw, tid);
+  staged<N * W, PER, kThreads>(
+      tid, [&](int e) { return pin[TILED ? tix<N>(e / W, c0 + e % W) : (e / W) * H + c0 + e % W]; },
+      [&](int e, float2 x) { buf[e] = x; });
+  tws.store(tw, tid);
+  __syncthreads();
+  lds_fft<N, W, kThreads, W, 1, true, false, 8>(buf, tw, tid);
+  // F at (p, c) from its transform: the filter, then the forcing entries
+  auto put = [&](int p, int c, float2 f) {
+    const float m = ns_filter(q, p, c);
+    f = make_float2(f.x * m, f.y * m);
+    for (int t = 0; t < q.n_force; ++t)
+      if (q.force_idx[2 * t] == p && q.force_idx[2 * t + 1] == c) f = cadd(f, q.force_val[t]);
+    out[p * H1 + c] = f;
+  };
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = tid + k * kThreads;
+    if (e >= N * W) break;
+    const int p = e / W, c = c0 + e % W;
+    const float2 y = buf[e];
+    if (c != 0) {
+      put(p, c, y);
+    } else {  // the DC (A) and Nyquist (B) columns
+      const float2 ym = cconj(buf[((N - p) & (N - 1)) * W]);
+      const float2 d = csub(y, ym);
+      put(p, 0, make_float2(0.5f * (y.x + ym.x), 0.5f * (y.y + ym.y)));
+      put(p, H, make_float2(0.5f * d.y, -0.5f * d.x));
+    }
+  }
+}
+
+// Columns of a spectrum in the external layout, scaled by 1/n^2 -> inverse
+// transforms, row by row.
+template <int N, int W>
+__global__ __launch_bounds__(kThreads) void ns_cols_in(NsParams q, const float2* __restrict__ in,
+                                                       float2* __restrict__ pout) {
+  constexpr int H = N / 2, H1 = H + 1, PER = (N * W + kThreads - 1) / kThreads;
+  __shared__ float2 buf[N * W];
+  __shared__ float2 tw[N];
+  __shared__ float2 w0[N], wn[N];  // tile 0: columns 0 and N/2
+  const int tid = threadIdx.x, c0 = xcd_tile(blockIdx.x, gridDim.x) * W;
+  const size_t inst = q.slots ? static_cast<size_t>(q.slots[blockIdx.y]) : blockIdx.y;
+  in += inst * static_cast<size_t>(N) * H1;
+  pout += inst * static_cast<size_t>(N) * H;
+  TwiddleStage<N, 1, kThreads> tws;
+  tws.load(q.tw, tid);
+  staged<N * W, PER, kThreads>(
+      tid, [&](int e) { return in[(e / W) * H1 + c0 + e % W]; },
+      [&](int e, float2 x) {
+        if (c0 + e % W == 0) w0[e / W] = x;
+        else buf[e] = make_float2(x.x * q.inv_nn, x.y * q.inv_nn);
+      });
+  if (c0 == 0)
+    for (int p = tid; p < N; p += kThreads) wn[p] = in[p * H1 + H];
+  tws.store(tw, tid);
+  if (c0 == 0) {
+    __syncthreads();
+    for (int p = tid; p < N; p += kThreads) {
+      const int pm = (N - p) & (N - 1);
+      const float2 s0 = make_float2(0.5f * (w0[p].x + w0[pm].x), 0.5f * (w0[p].y - w0[pm].y));
+      const float2 sh = make_float2(0.5f * (wn[p].x + wn[pm].x), 0.5f * (wn[p].y - wn[pm].y));
+      const float2 s = make_float2(s0.x - sh.y, s0.y + sh.x);  // s0 + i sh
+      buf[p * W] = make_float2(s.x * q.inv_nn, s.y * q.inv_nn);
+    }
+  }
+  __syncthreads();
+  lds_fft<N, W, kThreads, W, 1, true, true, 8>(buf, tw, tid);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = tid + k * kThreads;
+    if (e < N * W) pout[(e / W) * H + c0 + e % W] = buf[e];
+  }
+}
 
 // ---- mixed-size group step ---------------------------------------------------
 // Every item is 1024 complex words of work whatever its grid size (column
@@ -1174,7 +1248,7 @@ __device__ __forceinline__ void ns_group_tile(const NsGroupDesc& d, int tile, in
     const ColLds<N> lds(smem, waves, wave);
     const int c0 = tile * S::W + wave * ColShape<N>::T;
     if constexpr (CLS == 0)
-      cols_inverse_tile<N, 4, 8>(lds, d.q, d.ws, d.g, c0, S::W, tid % 64);
+      cols_inverse_tile<N, 8>(lds, d.q, d.ws, d.g, c0, S::W, tid % 64);
     else
       cols_forward_tile<N, CLS == 2 ? 2 : 1, 8>(lds, d.q, d.pbuf, d.ws, d.ws, d.h, d.g, c0, S::W, tid % 64);
   }
@@ -1252,10 +1326,10 @@ template <> struct NsTiles<256> { static constexpr int W = 8, RB = 2; };
 template <> struct NsTiles<512> { static constexpr int W = 8, RB = 1; };
 template <> struct NsTiles<1024> { static constexpr int W = 4, RB = 1; };
 
-template <int N, int NSPEC, int R>
+template <int N, int R>
 void launch_cols_inverse(int w, const NsParams& q, const float2* in, float2* g, int batch, hipStream_t s) {
   const int waves = col_waves<N>(w);
-  hipLaunchKernelGGL((ns_cols_inverse<N, NSPEC, R>), dim3(N / 2 / w, batch), dim3(64 * waves), col_lds<N>(waves), s,
+  hipLaunchKernelGGL((ns_cols_inverse<N, R>), dim3(N / 2 / w, batch), dim3(64 * waves), col_lds<N>(waves), s,
                      q, in, g, w);
 }
 template <int N, int MODE, int R>
@@ -1278,35 +1352,25 @@ void launch_rows(const NsParams& q, const float2* g, float2* pbuf, int batch, hi
 template <int N>
 struct NsOps {
   static constexpr int W = NsTiles<N>::W, RB = NsTiles<N>::RB;
-  static int cols_inverse(const NsParams& q, const float2* w, float2* g, int batch, hipStream_t s) {
-    launch_cols_inverse<N, 4, 8>(W, q, w, g, batch, s);
-    return check_hip(hipGetLastError(), "ns_cols_inverse");
-  }
-  // The external layout's rows are read and written column by column here,
-  // so many columns share a workgroup (and its cache lines).
   static int rfft2(const NsParams& q, const float* x, float2* out, float2* pbuf, int batch,
                    hipStream_t s) {
     NsParams plain = q;
     plain.smooth = 0;
     plain.n_force = 0;
     hipLaunchKernelGGL((rows_r2c<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, q, x, pbuf);
-    launch_cols_forward<N, 0, 8>(W, plain, pbuf, nullptr, out, nullptr, nullptr, batch, s);
+    hipLaunchKernelGGL((ns_cols_out<N, W, false>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, plain, pbuf, out);
     return check_hip(hipGetLastError(), "rfft2");
   }
   static int irfft2(const NsParams& q, const float2* in, float* x, float2* pbuf, int batch,
                     hipStream_t s) {
-    launch_cols_inverse<N, 1, 8>(W, q, in, pbuf, batch, s);
+    hipLaunchKernelGGL((ns_cols_in<N, W>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, q, in, pbuf);
     hipLaunchKernelGGL((rows_c2r<N, RB>), dim3(N / RB, batch), dim3(kThreads), 0, s, q, pbuf, x);
     return check_hip(hipGetLastError(), "irfft2");
   }
-  static int rows(const NsParams& q, const float2* g, float2* pbuf, int batch, hipStream_t s) {
-    launch_rows<N, (N >= 512 ? RB : 4), 8>(q, g, pbuf, batch, s);
-    return check_hip(hipGetLastError(), "ns_rows");
-  }
   // Forward column transforms of P -> explicit terms F (no update).
   static int explicit_cols(const NsParams& q, const float2* pbuf, float2* out, int batch, hipStream_t s) {
-    launch_cols_forward<N, 0, 8>(W, q, pbuf, nullptr, out, nullptr, nullptr, batch, s);
-    return check_hip(hipGetLastError(), "ns_cols_forward");
+    hipLaunchKernelGGL((ns_cols_out<N, W, true>), dim3(N / 2 / W, batch), dim3(kThreads), 0, s, q, pbuf, out);
+    return check_hip(hipGetLastError(), "explicit terms");
   }
 };
 
@@ -1350,7 +1414,7 @@ int ns_variant(int which, const NsParams& q, const float2* a, const float2* u_in
     return JCFD_OK;
   }
   if (which == 0)
-    launch_cols_inverse<N, 4, R>(T, q, a, g, batch, s);
+    launch_cols_inverse<N, R>(T, q, a, g, batch, s);
   else if (which == 2)
     launch_cols_forward<N, 2, R>(T, q, a, u_in, u_out, h, g, batch, s);
   else
@@ -1407,11 +1471,14 @@ bool ns_tile_on_menu(int which, int tile) {
   }
 }
 
+// The step's kernels of the plan's shapes, in the radix-8 schedule.
 template <int N>
-int ns_explicit_impl(const NsParams& q, const float2* w, float2* out, float2* g, float2* pbuf,
+int ns_explicit_impl(const NsParams& plan, const float2* w, float2* out, float2* g, float2* pbuf,
                      int batch, hipStream_t s) {
-  int rc = NsOps<N>::cols_inverse(q, w, g, batch, s);
-  if (!rc) rc = NsOps<N>::rows(q, g, pbuf, batch, s);
+  NsParams q = plan;
+  q.radix = 8;
+  int rc = ns_launch<N>(0, q, w, nullptr, nullptr, nullptr, g, batch, s);
+  if (!rc) rc = ns_launch<N>(1, q, g, nullptr, nullptr, nullptr, pbuf, batch, s);
   if (!rc) rc = NsOps<N>::explicit_cols(q, pbuf, out, batch, s);
   return rc;
 }
