@@ -7,9 +7,7 @@ the library binds to the HIP runtime torch already loaded (same soname).
 from __future__ import annotations
 
 import ctypes
-import functools
 import os
-import struct
 import threading
 
 import torch  # noqa: F401  (must load before the HIP library; see docstring)
@@ -256,28 +254,16 @@ _PyCapsule_GetPointer = ctypes.pythonapi.PyCapsule_GetPointer
 _PyCapsule_GetPointer.restype = ctypes.c_void_p
 _PyCapsule_GetPointer.argtypes = [ctypes.py_object, ctypes.c_char_p]
 
-_DTYPES = {torch.float32: (2, 32), torch.complex64: (5, 64), torch.int32: (0, 32)}
-_pack_data = struct.Struct("=Q").pack
-_TensorBuffer = ctypes.c_char * 48  # sizeof(jcfd_tensor): the data pointer, then _tensor_tail
-
-
-@functools.lru_cache(maxsize=256)
-def _tensor_tail(shape, dtype, device: int):
-  """jcfd_tensor of a C-contiguous array but for its data pointer, and the
-  shape array it points at."""
-  dims = (ctypes.c_int64 * len(shape))(*shape)
-  code, bits = _DTYPES[dtype]
-  return struct.pack("=iiiBBHQQQ", 10, device, len(shape), code, bits, 1,
-                     ctypes.addressof(dims), 0, 0), dims
+_to_dlpack = torch.utils.dlpack.to_dlpack
 
 
 class dlpack_args:
   """with dlpack_args() as dl: dl(tensor) is a jcfd_tensor* argument, valid
-  inside the block.
+  inside the block: the DLTensor of a DLPack capsule, whose layout jcfd_tensor
+  shares.
 
-  The structure is filled here for plain contiguous GPU tensors (0.5 us; a
-  DLPack capsule 1.1 us) and taken from a DLPack capsule for every other one,
-  whose checks and errors then apply.
+  us for 4 tensors: 1.7; 2.5 with a generator as context manager, 4.6 with the
+  structures filled in here instead of by DLPack.
   """
   __slots__ = ("_keep",)
 
@@ -289,17 +275,8 @@ class dlpack_args:
     self._keep.clear()
 
   def __call__(self, t: torch.Tensor):
-    if (type(t) is torch.Tensor and t.is_cuda and t.dtype in _DTYPES and t.is_contiguous()
-        and not t.is_conj() and not t.is_neg()):
-      shape = t.shape
-      if min(shape, default=0) > 1:  # DLPack rewrites the strides of other dimensions
-        tail = _tensor_tail(shape, t.dtype, t.get_device())
-        arg = _TensorBuffer.from_buffer_copy(_pack_data(t.data_ptr()) + tail[0])
-        self._keep.append((arg, tail, t))
-        return ctypes.addressof(arg)
-    cap = torch.utils.dlpack.to_dlpack(t)
+    cap = _to_dlpack(t)
     self._keep.append(cap)
-    # DLManagedTensor starts with its DLTensor, whose layout jcfd_tensor shares.
     return _PyCapsule_GetPointer(cap, b"dltensor")
 
 
