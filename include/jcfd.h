@@ -472,7 +472,8 @@ int jcfd_ns2d_group_set_graphs(jcfd_ns2d_group* group, int32_t enabled);
 /* nsteps steps of every member instance.  No (plan, slot) and no
  * (w_hat, slot) may appear twice.  Calls on one group must be ordered on one
  * stream, and a plan must not be stepped on another stream meanwhile (the
- * group steps its instances in the plan's internal buffers). */
+ * group steps its instances in the plan's internal buffers).  A single member
+ * steps as jcfd_ns2d_step_slots does. */
 int jcfd_ns2d_group_step(jcfd_ns2d_group* group, const jcfd_ns2d_group_member* members,
                          int32_t n_members, int64_t nsteps, void* stream);
 

@@ -1982,7 +1982,7 @@ constexpr size_t kNsPartCells = size_t(8) << 20;  // cells stepped together, see
 // plan's internal-layout buffer, stepped in place there (graph replay when
 // enabled) and moved back.
 int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slots, int count,
-           int64_t nsteps, hipStream_t s) {
+           int64_t nsteps, hipStream_t s, bool use_graphs = true) {
   const size_t n = static_cast<size_t>(p->n);
   const size_t ext = n * (n / 2 + 1), half = n * (n / 2);
   const int ns = p->n_stages;
@@ -1996,7 +1996,7 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
   // Graph replay saves 2 to 4 % of a part's steps (65 steps of 64 x 512^2, two
   // parts: 67.1 against 68.7 ms).  Every part has graphs of its own; more parts
   // than half the cache holds would replace each other's on every call.
-  const bool graphs = parts <= GraphCache::kMaxGraphs / 2;
+  const bool graphs = use_graphs && parts <= GraphCache::kMaxGraphs / 2;
   // Parts are read in as they come where that reads what the caller gave: an
   // output that overlaps the input (other than being it) holds earlier parts'
   // results by then, so everything is read in first.
@@ -2471,7 +2471,7 @@ int jcfd_ns2d_group_step(jcfd_ns2d_group* g, const jcfd_ns2d_group_member* membe
   if (nsteps < 0) return fail(JCFD_ERR_INVALID_ARGUMENT, "nsteps must be >= 0");
   struct Conv {
     int n, slot_off, count;
-    const jcfd_ns2d_plan* plan;
+    jcfd_ns2d_plan* plan;
     float2* state;
   };
   std::vector<Conv> convs;
@@ -2583,6 +2583,12 @@ int jcfd_ns2d_group_step(jcfd_ns2d_group* g, const jcfd_ns2d_group_member* membe
     g->bytes[2] += packed + 2 * ext + 2 * ext + 4 * packed;
     g->bytes[3] += packed + 2 * ext + 2 * ext;
   }
+  // One member: its plan's own step, whose kernels and shapes follow the size
+  // of the launch (4 steps, us, group kernels / the plan's: 4 x 32^2 311 / 189,
+  // 256 x 32^2 378 / 244, 1 x 512^2 551 / 315, 32 x 512^2 2371 / 2098).  Same bits.
+  if (convs.size() == 1)
+    return ns_run(convs[0].plan, convs[0].state, convs[0].state, g->d_slots, convs[0].count, nsteps, s,
+                  g->graphs.enabled);
   // external states -> the plans' internal layout, the steps, and back
   for (const Conv& c : convs)
     if ((rc = ns_launch_state_convert(c.n, true, c.state, c.plan->ws, g->d_slots + c.slot_off, c.count, s)))

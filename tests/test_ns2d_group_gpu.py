@@ -151,3 +151,41 @@ def test_group_rejects_bad_members():
   other = _plan(dataclasses.replace(fam.spec, tableau=rk3), 1)
   with pytest.raises(NotImplementedError):
     group.step([(plan, w, [0]), (other, w[:1].clone(), [0])], 1)  # stage counts differ
+
+
+@pytest.mark.parametrize("n,batch", [(32, 4), (512, 1), (1024, 9)])
+def test_single_member_group(n, batch):
+  """A group of one plan steps as the plan does, in its time: bit for bit over
+  direct and replayed steps, and not by the group kernels' fixed shapes."""
+  spec = _family(n).spec
+  plan, one = _plan(spec, batch + 1), _plan(spec, 1)
+  gen = torch.Generator(device=_dev()).manual_seed(n)
+  w0 = 0.01 * plan.rfft2(torch.randn((batch + 1, n, n), device=_dev(), generator=gen))
+  slots = list(range(batch, 0, -1))
+  for graphs in (True, False):
+    group, w = _group(), w0.clone()
+    group.set_graphs(graphs)
+    group.step([(plan, w, slots)], 35)
+    for s in (1, batch):
+      assert torch.equal(w[s], one.step(w0[s].clone(), 35)), (graphs, s)
+    assert torch.equal(w[0], w0[0])
+  group.step([(plan, w, slots)], 1)
+  assert set(group.time_kernels(2)) == set(plan.KERNELS)
+
+  dev_slots = torch.tensor(slots, dtype=torch.int32, device=_dev())
+
+  def best(f):
+    times = []
+    for _ in range(5):
+      start, end = torch.cuda.Event(True), torch.cuda.Event(True)
+      start.record()
+      for _ in range(5):
+        f()
+      end.record()
+      end.synchronize()
+      times.append(start.elapsed_time(end))
+    return min(times)
+
+  w = w0.clone()
+  alone = best(lambda: plan.step_slots(w, dev_slots, 8))
+  assert best(lambda: group.step([(plan, w, slots)], 8)) <= 1.25 * alone
