@@ -412,7 +412,8 @@ int jcfd_ns2d_plan_set_graphs(jcfd_ns2d_plan* plan, int32_t enabled);
 
 /* Tile shapes and FFT radix schedule of the step kernels (see
  * jcfd_fvm_tiles; no counterpart in the reference).  Tile shapes never
- * change results; radix 4 changes the FFT rounding. */
+ * change results; radix 4 changes the FFT rounding.  Batches above 2^23 cells
+ * step in parts; get_tiles then reports a part's shapes. */
 typedef struct {
   int32_t cols;  /* packed spectrum columns per workgroup of the column kernels: 1..16 */
   int32_t rows;  /* rows per workgroup of the row (nonlinear product) kernel: 1, 2, 4, 8, 16 */

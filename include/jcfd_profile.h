@@ -51,6 +51,8 @@ int jcfd_li_kernel_flops(const jcfd_li_plan* plan, double* flops_per_launch);
 #define JCFD_NS2D_KERNEL_COLS_UPDATE 3        /* forward cols + final update */
 #define JCFD_NS2D_KERNEL_COUNT 4
 
+/* A batch that steps in parts is timed part by part; the times of all parts
+ * together are reported, for the bytes of the whole batch. */
 int jcfd_ns2d_time_kernels(jcfd_ns2d_plan* plan, const jcfd_tensor* w_hat, int32_t reps,
                            double* ms_per_launch, void* stream);
 int jcfd_ns2d_kernel_bytes(const jcfd_ns2d_plan* plan, int64_t* bytes_per_launch);

@@ -1975,7 +1975,43 @@ int jcfd_fvm_group_launch_shape(const jcfd_fvm_group* g, int32_t* grid, int32_t*
 
 // ------------------------------------------------------------ spectral path
 namespace {
-constexpr size_t kNsPartCells = size_t(8) << 20;  // cells stepped together, see ns_run
+// A step streams 28 bytes per cell through its kernels.  Batches whose
+// share exceeds the 256 MB last-level cache run in parts that fit, each
+// part all its steps: the spectra one kernel writes are then still cached
+// when the next reads them (512^2: 17.1 us per instance and step at 32
+// instances, 18.5 at 16, 19.1 at 64).
+constexpr size_t kNsPartCells = size_t(8) << 20;
+int ns_parts(int n, int count) {
+  const int most = static_cast<int>(std::max<size_t>(1, kNsPartCells / (static_cast<size_t>(n) * n)));
+  return (count + most - 1) / most;
+}
+
+// Part k of `parts` of count instances: its instances (reached through the slot
+// list, or by offset), their shapes and buffers.
+struct NsPart {
+  int m = 0;                  // instances
+  const int* slots = nullptr;
+  size_t offset = 0;          // words of the external layout before the first
+  NsParams stages[JCFD_MAX_RK_STAGES];
+  NsBuffers b{};
+  NsPart(const jcfd_ns2d_plan* p, const int* all_slots, int count, int k, int parts) {
+    const size_t n = static_cast<size_t>(p->n), half = n * (n / 2), ext = n * (n / 2 + 1);
+    const int first = static_cast<int>(static_cast<int64_t>(count) * k / parts);
+    m = static_cast<int>(static_cast<int64_t>(count) * (k + 1) / parts) - first;
+    slots = all_slots ? all_slots + first : nullptr;
+    const size_t o = all_slots ? 0 : static_cast<size_t>(first);
+    offset = o * ext;
+    for (int i = 0; i < p->n_stages; ++i) {
+      stages[i] = p->stages[i];
+      stages[i].slots = slots;
+      if (!p->tiles_set) (void)ns_default_tiles(&stages[i], p->n, m);
+    }
+    b.u_in = b.u_out = p->ws + offset;
+    b.h = p->h + offset;
+    b.g = p->g + o * 4 * half;
+    b.pbuf = p->pbuf + o * half;
+  }
+};
 
 // nsteps CN-RK4 steps of `count` instances (slots, or 0..count-1) from
 // w_in to w_out (external layout; may alias or overlap): the state is moved into the
@@ -1983,16 +2019,8 @@ constexpr size_t kNsPartCells = size_t(8) << 20;  // cells stepped together, see
 // enabled) and moved back.
 int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slots, int count,
            int64_t nsteps, hipStream_t s, bool use_graphs = true) {
-  const size_t n = static_cast<size_t>(p->n);
-  const size_t ext = n * (n / 2 + 1), half = n * (n / 2);
-  const int ns = p->n_stages;
-  // A step streams 28 bytes per cell through its kernels.  Batches whose
-  // share exceeds the 256 MB last-level cache run in parts that fit, each
-  // part all its steps: the spectra one kernel writes are then still cached
-  // when the next reads them (512^2: 17.1 us per instance and step at 32
-  // instances, 18.5 at 16, 19.1 at 64).
-  const int most = static_cast<int>(std::max<size_t>(1, kNsPartCells / (n * n)));
-  const int parts = (count + most - 1) / most;
+  const size_t ext = static_cast<size_t>(p->n) * (p->n / 2 + 1);
+  const int parts = ns_parts(p->n, count);
   // Graph replay saves 2 to 4 % of a part's steps (65 steps of 64 x 512^2, two
   // parts: 67.1 against 68.7 ms).  Every part has graphs of its own; more parts
   // than half the cache holds would replace each other's on every call.
@@ -2005,28 +2033,13 @@ int ns_run(jcfd_ns2d_plan* p, const float2* w_in, float2* w_out, const int* slot
   int rc;
   if (read_first && (rc = ns_launch_state_convert(p->n, true, w_in, p->ws, slots, count, s))) return rc;
   for (int k = 0; k < parts; ++k) {
-    const int first = static_cast<int>(static_cast<int64_t>(count) * k / parts);
-    const int m = static_cast<int>(static_cast<int64_t>(count) * (k + 1) / parts) - first;
-    // instances are reached through the slot list, or by offset
-    const int* sl = slots ? slots + first : nullptr;
-    const size_t o = slots ? 0 : static_cast<size_t>(first);
-    NsParams stages[JCFD_MAX_RK_STAGES];
-    for (int i = 0; i < ns; ++i) {
-      stages[i] = p->stages[i];
-      stages[i].slots = sl;
-      if (!p->tiles_set) (void)ns_default_tiles(&stages[i], p->n, m);
-    }
-    NsBuffers b{};
-    b.u_in = p->ws + o * ext;
-    b.u_out = p->ws + o * ext;
-    b.h = p->h + o * ext;
-    b.g = p->g + o * 4 * half;
-    b.pbuf = p->pbuf + o * half;
-    auto step = [&](hipStream_t gs) { return ns_launch_step(p->n, stages, ns, b, m, gs); };
-    if (!read_first && (rc = ns_launch_state_convert(p->n, true, w_in + o * ext, p->ws + o * ext, sl, m, s))) return rc;
+    const NsPart t(p, slots, count, k, parts);
+    const size_t o = t.offset;
+    auto step = [&](hipStream_t gs) { return ns_launch_step(p->n, t.stages, p->n_stages, t.b, t.m, gs); };
+    if (!read_first && (rc = ns_launch_state_convert(p->n, true, w_in + o, p->ws + o, t.slots, t.m, s))) return rc;
     if ((rc = step(s))) return rc;
-    if ((rc = run_steps(p->graphs, b.u_out, nullptr, sl, m, nsteps - 1, s, step, graphs))) return rc;
-    if ((rc = ns_launch_state_convert(p->n, false, p->ws + o * ext, w_out + o * ext, sl, m, s))) return rc;
+    if ((rc = run_steps(p->graphs, t.b.u_out, nullptr, t.slots, t.m, nsteps - 1, s, step, graphs))) return rc;
+    if ((rc = ns_launch_state_convert(p->n, false, p->ws + o, w_out + o, t.slots, t.m, s))) return rc;
   }
   return JCFD_OK;
 }
@@ -2158,7 +2171,7 @@ int jcfd_ns2d_plan_create(const jcfd_ns2d_config* config, jcfd_ns2d_plan** plan)
     q.mu = static_cast<float>(0.5 * c.dt * (alpha[k + 1] - alpha[k]));
     q.read_h = k > 0 ? 1 : 0;
     q.slots = nullptr;
-    (void)ns_default_tiles(&q, n, c.batch);
+    (void)ns_default_tiles(&q, n, (c.batch + ns_parts(n, c.batch) - 1) / ns_parts(n, c.batch));
   }
   *plan = p;
   return JCFD_OK;
@@ -2254,25 +2267,27 @@ int jcfd_ns2d_time_kernels(jcfd_ns2d_plan* p, const jcfd_tensor* w_hat, int32_t 
   float2* tmp = nullptr;
   int64_t unused = 0;
   if ((rc = device_alloc(&tmp, count, &unused))) return rc;
-  NsBuffers b{};
-  b.u_in = p->ws;
-  b.u_out = tmp;
-  b.h = p->h;
-  b.g = p->g;
-  b.pbuf = p->pbuf;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   rc = ns_launch_state_convert(p->n, true, static_cast<const float2*>(pin), p->ws, nullptr, p->batch, s);
   if (!rc) rc = check_hip(hipEventCreate(&e0), "event");
   if (!rc) rc = check_hip(hipEventCreate(&e1), "event");
-  if (!rc) rc = ns_launch_step(p->n, p->stages, p->n_stages, b, p->batch, s);  // fills every scratch buffer
-  for (int k = 0; k < JCFD_NS2D_KERNEL_COUNT && rc == JCFD_OK; ++k) {
-    rc = check_hip(hipEventRecord(e0, s), "event record");
-    for (int r = 0; r < reps && rc == JCFD_OK; ++r) rc = ns_launch_kernel(p->n, k, p->stages, p->n_stages, b, p->batch, s);
-    if (!rc) rc = check_hip(hipEventRecord(e1, s), "event record");
-    if (!rc) rc = check_hip(hipEventSynchronize(e1), "event sync");
-    float ms = 0.f;
-    if (!rc) rc = check_hip(hipEventElapsedTime(&ms, e0, e1), "elapsed");
-    ms_per_launch[k] = static_cast<double>(ms) / reps;
+  for (int k = 0; k < JCFD_NS2D_KERNEL_COUNT; ++k) ms_per_launch[k] = 0.0;
+  // part by part, as a step runs them
+  const int parts = ns_parts(p->n, p->batch);
+  for (int i = 0; i < parts && rc == JCFD_OK; ++i) {
+    NsPart t(p, nullptr, p->batch, i, parts);
+    t.b.u_out = tmp + t.offset;
+    rc = ns_launch_step(p->n, t.stages, p->n_stages, t.b, t.m, s);  // fills every scratch buffer
+    for (int k = 0; k < JCFD_NS2D_KERNEL_COUNT && rc == JCFD_OK; ++k) {
+      rc = check_hip(hipEventRecord(e0, s), "event record");
+      for (int r = 0; r < reps && rc == JCFD_OK; ++r)
+        rc = ns_launch_kernel(p->n, k, t.stages, p->n_stages, t.b, t.m, s);
+      if (!rc) rc = check_hip(hipEventRecord(e1, s), "event record");
+      if (!rc) rc = check_hip(hipEventSynchronize(e1), "event sync");
+      float ms = 0.f;
+      if (!rc) rc = check_hip(hipEventElapsedTime(&ms, e0, e1), "elapsed");
+      ms_per_launch[k] += static_cast<double>(ms) / reps;
+    }
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);

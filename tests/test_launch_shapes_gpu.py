@@ -181,3 +181,27 @@ def test_fvm_marching_rows_of_1024(convect, batch):
     plan.set_tiles(rows, 1, 1, 8)
     got = plan.step(u, v, 2)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), rows
+
+
+# kernel times are those of the launches a step makes: with parts, their sum
+# over a step is the step's own time but for launch gaps (one launch over all of
+# 64 x 512^2, beyond the cache, adds up to 1.2 steps)
+@pytest.mark.parametrize("n,batch", [(512, 64), (256, 256)])
+def test_spectral_kernel_times_add_up(n, batch):
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  plan = _ns2d.Ns2dPlan(serving.SpectralFamily(n, _dev()).spec, batch, _dev())
+  w = 0.01 * plan.rfft2(torch.randn((batch, n, n), device=_dev(),
+                                    generator=torch.Generator(device=_dev()).manual_seed(n)))
+  times = []
+  for _ in range(5):
+    start, end = torch.cuda.Event(True), torch.cuda.Event(True)
+    start.record()
+    plan.step(w, 33, out=w)
+    end.record()
+    end.synchronize()
+    times.append(start.elapsed_time(end) / 33)
+  ms = plan.time_kernels(w, 20)
+  total = sum(ms[k] * plan.LAUNCHES_PER_STEP[k] for k in ms)
+  print(f"{batch} x {n}^2: step {min(times):.3f} ms, kernels {total:.3f} ms", flush=True)
+  assert 0.8 * min(times) <= total <= 1.1 * min(times)
