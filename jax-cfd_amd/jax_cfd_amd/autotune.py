@@ -96,10 +96,18 @@ def _device_name(device) -> str:
     return 'unknown'
 
 
+# Part of every cache key, to be raised when the kernels behind the menu change:
+# shapes measured on others are measured again (spectral 64 x 512^2: the shapes
+# that were fastest on the staged kernels, cols 2 rows 2, take 2.55 ms per two
+# steps on the register ones, where the staged kernels took 2.41 and untuned
+# plans take 2.1).
+_KERNELS = 2
+
+
 def _key(plan, t: Tunables, radices: Sequence[int]) -> str:
   s = plan.spec
   extra = f'|convect={s.convect}' if t.solver == 'fvm' else ''
-  return (f'{_device_name(plan.device)}|{t.solver}|n={s.n}|batch={plan.batch}{extra}|'
+  return (f'{_device_name(plan.device)}|{t.solver}|kernels={_KERNELS}|n={s.n}|batch={plan.batch}{extra}|'
           f'radices={",".join(map(str, radices))}')
 
 

@@ -124,3 +124,16 @@ def test_spectral_choice_weights_kernels_by_launches(tmp_path, monkeypatch):
   res = autotune.tune_ns2d(plan, w=object(), reps=1)
   assert plan.tiles == dict(cols=8, rows=1, radix=8)
   assert res['timings']['8']['rows'].keys() == {'1', '2', '4'}
+
+
+def test_choices_of_other_kernels_are_measured_again(tmp_path, monkeypatch):
+  cache = tmp_path / 'tiles.json'
+  monkeypatch.setenv('JCFD_TUNE_CACHE', str(cache))
+  stale = dict(cols=1, rows=4, radix=8, ms_per_step=0.0)
+  # as stored before keys named the kernels, and by another generation of them
+  keys = {f'unknown|spectral|{g}n=128|batch=2|radices=8': stale for g in ('', 'kernels=1|')}
+  cache.write_text(json.dumps(keys))
+  plan = FakeNsPlan()
+  res = autotune.tune_ns2d(plan, w=object(), reps=1)
+  assert not res['cached'] and plan.tiles == dict(cols=8, rows=1, radix=8)
+  assert len(json.loads(cache.read_text())) == 3  # the others' entries stay
