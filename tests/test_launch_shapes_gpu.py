@@ -1,7 +1,8 @@
-"""Launch shapes picked from a launch's size, on both sides of every line of
-the rules: each must step bit-identically to the same plan with one-row,
-one-column tiles set by hand (tile shapes never change results), for whole
-batches and for short slot lists of a large batch."""
+"""Launch shapes picked from a launch's size: each must step bit-identically to
+the same plan with one-row, one-column tiles set by hand (tile shapes never
+change results), on both sides of every line of the rules (where the shapes have
+to differ, so a line that moves is noticed), for whole batches and for short slot
+lists of a large batch."""
 import pytest
 import torch
 
@@ -23,7 +24,6 @@ def _fvm(n, batch, **kw):
   return _fvm.FvmPlan(spec, _dev(), batch=batch), u, v
 
 
-# rows or columns over all instances at the rules' lines, and one below
 @pytest.mark.parametrize("n,batch", [(32, 7), (32, 32), (32, 512), (64, 7), (64, 8), (64, 15), (64, 64),
                                      (64, 256), (128, 7), (128, 8), (128, 31), (128, 128),
                                      (256, 2), (256, 3), (256, 4), (256, 16), (256, 47), (256, 48),
@@ -193,6 +193,7 @@ def test_spectral_kernel_times_add_up(n, batch):
   plan = _ns2d.Ns2dPlan(serving.SpectralFamily(n, _dev()).spec, batch, _dev())
   w = 0.01 * plan.rfft2(torch.randn((batch, n, n), device=_dev(),
                                     generator=torch.Generator(device=_dev()).manual_seed(n)))
+  plan.set_graphs(False)  # direct launches, as the kernel times are
   times = []
   for _ in range(5):
     start, end = torch.cuda.Event(True), torch.cuda.Event(True)
@@ -205,3 +206,74 @@ def test_spectral_kernel_times_add_up(n, batch):
   total = sum(ms[k] * plan.LAUNCHES_PER_STEP[k] for k in ms)
   print(f"{batch} x {n}^2: step {min(times):.3f} ms, kernels {total:.3f} ms", flush=True)
   assert 0.8 * min(times) <= total <= 1.1 * min(times)
+
+
+# (n, rows over all instances from which a rule picks another shape)
+FVM_LINES = [(n, rows) for n, lines in {
+    32: (1024, 2048, 4096, 16384), 64: (1024, 2048, 4096, 16384), 128: (1024, 2048, 4096, 16384, 32768),
+    256: (1024, 2048, 4096, 8192), 512: (1024, 2048, 4096), 1024: (2048, 4096, 16384)}.items() for rows in lines]
+SPECTRAL_LINES = [(n, rows) for n, lines in {
+    32: (2048, 8192), 64: (2048, 16384), 128: (1024, 2048, 4096, 8192, 16384), 256: (512, 1024, 4096, 8192),
+    512: (4096,), 1024: (2048, 4096)}.items() for rows in lines]
+
+
+@pytest.mark.parametrize("n,rows", FVM_LINES)
+def test_fvm_rules_on_both_sides(n, rows):
+  below, above = _fvm(n, rows // n - 1), _fvm(n, rows // n)
+  assert below[0].tiles != above[0].tiles
+  for plan, u, v in (below, above):
+    u, v = u.reshape(plan.shape), v.reshape(plan.shape)
+    got = plan.step(u, v, 2)
+    plan.set_tiles(1, 1, 1, 8)
+    want = plan.step(u, v, 2)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n,rows", SPECTRAL_LINES)
+def test_spectral_rules_on_both_sides(n, rows):
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  spec = serving.SpectralFamily(n, _dev()).spec
+  plans = [_ns2d.Ns2dPlan(spec, rows // n - k, _dev()) for k in (1, 0)]
+  assert plans[0].tiles != plans[1].tiles
+  for plan in plans:
+    gen = torch.Generator(device=_dev()).manual_seed(n + plan.batch)
+    w = plan.rfft2(torch.randn(plan.real_shape, device=_dev(), generator=gen))
+    got = plan.step(w, 2)
+    plan.set_tiles(1, 1, 8)
+    assert torch.equal(got, plan.step(w, 2))
+
+
+# the marching stencil at its other sizes, and a group's, whose workgroups hold
+# two cells of a 512 row per thread: every scheme against one-row tiles
+@pytest.mark.parametrize("convect", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [256, 512])
+def test_fvm_marching_rows_of_every_scheme(n, convect):
+  from jax_cfd_amd.base import _fvm as fvm
+  plan, u, v = _fvm(n, 2, convect=convect)
+  plan.set_tiles(1, 1, 1, 8)
+  want = plan.step(u, v, 2)
+  for rows in (16, 32):
+    plan.set_tiles(rows, 1, 1, 8)
+    got = plan.step(u, v, 2)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), rows
+  gu, gv = u.clone(), v.clone()
+  fvm.FvmGroup(_dev()).step([(plan, gu, gv, [0, 1])], 2)
+  assert torch.equal(gu, want[0]) and torch.equal(gv, want[1])
+
+
+# wavenumbers of other boxes: the register kernels form them from the box's
+# length, the staged ones read the table
+@pytest.mark.parametrize("n,batch", [(32, 256), (64, 256), (128, 128), (256, 64), (512, 16), (1024, 4)])
+@pytest.mark.parametrize("box", [(1.0, 3.0), (10.7, 0.3), (3.141592653589793, 100.0)])
+def test_spectral_boxes_step_as_one_column_tiles(n, batch, box):
+  import dataclasses
+  from jax_cfd_amd import serving
+  from jax_cfd_amd.spectral import _ns2d
+  spec = dataclasses.replace(serving.SpectralFamily(n, _dev()).spec, dx=box[0] / n, dy=box[1] / n, dt=1e-5)
+  plan = _ns2d.Ns2dPlan(spec, batch, _dev())
+  gen = torch.Generator(device=_dev()).manual_seed(n)
+  w = 0.01 * plan.rfft2(torch.randn((batch, n, n), device=_dev(), generator=gen))
+  got = plan.step(w, 2)
+  plan.set_tiles(1, 1, 8)
+  assert torch.isfinite(torch.view_as_real(got)).all() and torch.equal(got, plan.step(w, 2))
