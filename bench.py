@@ -545,10 +545,13 @@ def _served(dev, requests, kernel_reps, group=(), runs=3, warmup_passes=1):
   tiles = plan.tiles
   key = (_ns2d_kernel_key(kname, n, plan.batch, tiles) if solver == "spectral"
          else _fvm_plan_kernel_key(kname, n, plan.batch, tiles))
+  # the times and bytes are those of the whole pool: of all its parts' launches
+  parts = _ns2d_parts(n, plan.batch) if solver == "spectral" else 1
+  traffic = _traffic(key)
   roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
               "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-              "traffic": _traffic(key), "kernel": kname, "launch": key,
-              "pool": f"{solver} {n}^2 x {plan.batch} slots",
+              "traffic": None if traffic is None else traffic * parts, "kernel": kname, "launch": key,
+              "launches": parts, "pool": f"{solver} {n}^2 x {plan.batch} slots",
               "bytes_per_launch": nbytes, "ms_per_launch": round(ms, 5)}
   copy_gbps = _copy_rate(dev, nbytes)
   roofline["copy_GBps"] = round(copy_gbps, 1)
@@ -596,8 +599,16 @@ def _served(dev, requests, kernel_reps, group=(), runs=3, warmup_passes=1):
   return summ, roofline
 
 
+def _ns2d_parts(n, batch):
+  """Launches of each step kernel a spectral batch makes per stage: batches
+  above 2^23 cells step in parts."""
+  return -(-batch // max(1, (1 << 23) // (n * n)))
+
+
 def _ns2d_kernel_key(kname, n, batch, tiles):
-  """_kernel_key of a spectral plan's step kernel for its tiles."""
+  """_kernel_key of a spectral plan's step kernel for its tiles (of a batch in
+  parts: one part's launch)."""
+  batch = -(-batch // _ns2d_parts(n, batch))
   w, rb, radix = tiles["cols"], tiles["rows"], tiles["radix"]
   if kname == "ns_rows":
     rs = 1024 // n  # rows per wavefront

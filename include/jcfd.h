@@ -158,8 +158,8 @@ int jcfd_fvm_cg_solves(const jcfd_fvm_plan* plan, int64_t* counts);
  * round-off of each other). */
 typedef struct {
   int32_t rows_forward; /* rows per workgroup of the stencil kernel: 1, 2, 4, 8, 16, 32; 16 and 32
-                           (n 256, 512) and 4 to 32 (n 1024) march over the rows with a
-                           ring of staged rows */
+                           (n 256, 512) and 4 to 32 (n 1024) march over the rows, the cells
+                           around each thread's own in registers */
   int32_t poisson_cols; /* spectrum columns per workgroup: 1, 2, 4, 8, 16 */
   int32_t rows_project; /* rows per workgroup of the projection kernel: 1, 2, 4, 8 */
   int32_t radix;        /* largest FFT radix: 8 or 4 */

@@ -76,7 +76,7 @@ __device__ __forceinline__ float mean2(float a, float b) { return __builtin_fmaf
 // Van Leer flux correction (advection.py:284-334 for one face):
 // pre = 0.5 (1 - (dt/h)|U|)|U|;  phi = num (sgn den + sgn num) den / D,
 // D = |den| + |num| if |den| > 0 else 1.  The marching stencil is bound by
-// these instructions (some 300 per cell, four cycles each), so:
+// these instructions (some 250 per cell, four cycles each), so:
 //   - the quotient is ratio's for D in its range [2^-126, 2^126]; a wavefront
 //     that meets another D (differences of 8e37 and more, their infinite sum,
 //     subnormal ones; D = 0 with its den = 0 gives 0 either way) divides there

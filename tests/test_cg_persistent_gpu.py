@@ -1,4 +1,4 @@
-"""CG solves as one cooperative launch (grid barriers between the iteration
+"""CG solves as one cooperative launch (messages between the iteration
 steps) against the two-launches-per-iteration form: the same iterates, so
 the same results bit for bit and the same iteration counts, for the pressure
 solve (pressure.py:67-112) and the implicit diffusion solve
