@@ -1261,8 +1261,12 @@ __device__ __forceinline__ void group_tile(const FvmGroupDesc& d, int tile, int 
 // One workgroup per item (the host launches exactly the phase's item
 // count): the hardware's workgroup dispatch keeps the CUs full, as for the
 // per-size kernels, with no loop state held in registers (a persistent
-// fixed-stride walk over the list measured 7-15 % slower).
-template <int PHASE>
+// fixed-stride walk over the list measured 7-15 % slower).  Groups without
+// sizes that march have a stencil build of their own (MARCH = false): the
+// marching bodies' window costs every other size registers (36 against 114; 4
+// steps of 128 x 128^2 223 us with the one build, 193 so, of 256 x 64^2 168 and
+// 145).
+template <int PHASE, bool MARCH>
 __global__ __launch_bounds__(kThreads) void fvm_group_phase(FvmGroupQueue q) {
   extern __shared__ float4 fvm_group_smem[];
   char* smem = reinterpret_cast<char*>(fvm_group_smem);
@@ -1291,8 +1295,12 @@ __global__ __launch_bounds__(kThreads) void fvm_group_phase(FvmGroupQueue q) {
     case 32: group_tile<32, PHASE>(d, w.tile, t, smem); break;
     case 64: group_tile<64, PHASE>(d, w.tile, t, smem); break;
     case 128: group_tile<128, PHASE>(d, w.tile, t, smem); break;
-    case 256: group_tile<256, PHASE>(d, w.tile, t, smem); break;
-    case 512: group_tile<512, PHASE>(d, w.tile, t, smem); break;
+    case 256:
+      if constexpr (MARCH) group_tile<256, PHASE>(d, w.tile, t, smem);
+      break;
+    case 512:
+      if constexpr (MARCH) group_tile<512, PHASE>(d, w.tile, t, smem);
+      break;
     default: break;  // rejected on the host
   }
 }
@@ -1367,9 +1375,14 @@ int fvm_group_launch(int phase, int max_n, const FvmGroupQueue& q, int grid, hip
     return fail(JCFD_ERR_UNSUPPORTED, "group grid size not supported: " + std::to_string(max_n));
   const size_t lds = static_cast<size_t>(group_lds(phase, max_n));
   switch (phase) {
-    case 0: hipLaunchKernelGGL(fvm_group_phase<0>, dim3(grid), dim3(kThreads), lds, s, q); break;
-    case 1: hipLaunchKernelGGL(fvm_group_phase<1>, dim3(grid), dim3(kThreads), lds, s, q); break;
-    default: hipLaunchKernelGGL(fvm_group_phase<2>, dim3(grid), dim3(kThreads), lds, s, q);
+    case 0:
+      if (max_n >= 256)
+        hipLaunchKernelGGL((fvm_group_phase<0, true>), dim3(grid), dim3(kThreads), lds, s, q);
+      else
+        hipLaunchKernelGGL((fvm_group_phase<0, false>), dim3(grid), dim3(kThreads), lds, s, q);
+      break;
+    case 1: hipLaunchKernelGGL((fvm_group_phase<1, true>), dim3(grid), dim3(kThreads), lds, s, q); break;
+    default: hipLaunchKernelGGL((fvm_group_phase<2, true>), dim3(grid), dim3(kThreads), lds, s, q);
   }
   return check_hip(hipGetLastError(), "fvm group launch");
 }
